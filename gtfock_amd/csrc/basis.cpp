@@ -404,6 +404,8 @@ void gtf_boys_taylor_tables(double* t8)
                 t8[at] = c;
             }
         }
+    double* e = t8 + (size_t)BOYS8_NM * BOYS8_SLAB;
+    for (int i = 0; i < BOYS8_EXP; i++) e[i] = (double)expl(-(long double)i * BOYS8_DELTA);
 }
 
 void gtf_boys_table(double* tab, int ngrid, int ncol, double delta)

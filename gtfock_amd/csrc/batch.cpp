@@ -165,7 +165,6 @@ __global__ void binv_sqrt_kernel(const double* W, const double* lam, int n, int 
 
 int GtfBatch::enqueue_fock()
 {
-    if (gtf_fill(stream, d_J, total, 0.0) || gtf_fill(stream, d_K, total, 0.0)) return -1;
     if (sys.jk(d_D, d_J, d_K)) return -1;
     if (sys.symmetrize(d_J) || sys.symmetrize(d_K)) return -1;
     return gtf_add(stream, d_J, d_K, d_G, total);
@@ -1076,20 +1075,34 @@ double gtf_batch_job_bytes(BasisSet_t basis)
 {
     if (!basis) return -1.0;
     const BasisSet* b = basis;
-    double pairs = 0.0;
+    double pairs = 0.0, blocks = 0.0;
+    int most[GTF_NPAIRTYPES] = {0};  // primitive pairs of a shell pair, by type
+    double record[GTF_NPAIRTYPES] = {0.0};
     for (int s = 0; s < b->nshells; s++)
         for (int t = 0; t <= s; t++) {
             int la = b->L[s], lb = b->L[t];
             if (lb > la) std::swap(la, lb);
-            const double np = (double)b->nprim[s] * b->nprim[t];
+            const int np = b->nprim[s] * b->nprim[t], type = pair_type(la, lb);
+            const int full = nsph(la) * nsph(lb) * nherm(la + lb), nnz = herm_nnz_lookup(la, lb);
+            most[type] = std::max(most[type], np);
+            // ket record of a primitive pair (KetView)
+            record[type] = 16.0 * KetView::rec(nnz) + 8.0 * ((KetView::full(type) ? full : 0) + 1);
             // per primitive pair: (p, P), its Schwarz bound, full and compact E
-            pairs += np * (40.0 + 8.0 * (nsph(la) * nsph(lb) * nherm(la + lb) + herm_nnz_lookup(la, lb))) + 96.0;
+            // in both precisions, the ket record with the padding of its block
+            pairs += np * (40.0 + 12.0 * (full + nnz) + 1.25 * record[type]) + 128.0;
+        }
+    // a type's kets are padded to 64 in every primitive-count bucket
+    for (int t = 0; t < GTF_NPAIRTYPES; t++)
+        for (int k = 0; k < GtfSystem::NBUCKET; k++) {
+            static const int top[GtfSystem::NBUCKET] = {1, 4, 12, 32, INT32_MAX};
+            if (most[t] > (k > 0 ? top[k - 1] : 0)) blocks += 64.0 * std::min(top[k], most[t]) * record[t];
         }
     const double n = b->nbf, pl = ((b->nbf + 63) / 64) * 64;
     // + the split purification's BF16 slices of both operands at the most
     // slices (and their exponents and row maxima)
     const double split = 2.0 * 2.0 * OZ_SLICES_MAX * pl * pl + 4.0 * 8.0 * pl * pl / 64.0;
-    return pairs * 1.6 + 8.0 * (9.0 * n * n + (8.0 + 2.0 * B_MAX_DIIS) * pl * pl) + split + (1 << 20);
+    // + the list-ordered density and J_PQ copies (an n x n matrix)
+    return pairs * 1.6 + blocks + 8.0 * (10.5 * n * n + (8.0 + 2.0 * B_MAX_DIIS) * pl * pl) + split + (1 << 20);
 }
 
 int gtf_batch_get_density(gtf_batch_t b, int m, double* D)

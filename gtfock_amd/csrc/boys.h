@@ -19,19 +19,25 @@
 //   F_M(T) = sum_k c_k (T0 - T)^k,  |T0 - T| <= BOYS8_DELTA / 2
 // (truncation below 1e-15 relative).  FP64 in every kernel, the FP32 tiles
 // included.  A class touches one slab (23 KB), small enough to stay in the
-// vector L1 cache or in LDS.
-template <int M>
+// vector L1 cache or in LDS.  COLS: the slab is an LDS copy stored as four
+// columns of BOYS8_NGRID double2 -- rows of 64 bytes would put the same part
+// of every row on 4 of the 16 bank groups of a 16-byte read.
+//
+// The recursions' exp(-T): below BOYS_TMAX exp(-T0), tabulated after the
+// slabs, times the exponential series of T0 - T (8 terms beyond 1: the next is
+// below 1e-17); above it exp(-T) only corrects F_m by 1e-8 of itself or less,
+// and 2^n times the hardware's 2^f in FP32 (1e-7 of it) is enough.  The
+// library's exp costs 30 instructions and a dozen constants in registers, a
+// third of a low-L primitive quartet.
+template <int M, bool COLS = false>
 __device__ __forceinline__ void boys_eval8(double T, double* F, const double* __restrict__ slab)
 {
-    // exp(-T) serves both regimes; computed once before the branch, so a
-    // wavefront with lanes on both sides does not run it twice
-    double e = 0.0;
-    if constexpr (M > 0) e = exp(-T);
     if (T < BOYS_TMAX) {
         const int i = (int)(T * BOYS8_INV_DELTA + 0.5);
-        const double dt = i * BOYS8_DELTA - T;
-        const double2* r = reinterpret_cast<const double2*>(slab + i * BOYS8_NTERM);
-        const double2 c01 = r[0], c23 = r[1], c45 = r[2], c67 = r[3];
+        const double dt = fma((double)i, BOYS8_DELTA, -T);
+        const double2* r = reinterpret_cast<const double2*>(slab) + i * (COLS ? 1 : BOYS8_NTERM / 2);
+        constexpr int S = COLS ? BOYS8_NGRID : 1;
+        const double2 c01 = r[0], c23 = r[S], c45 = r[2 * S], c67 = r[3 * S];
         double f = fma(c67.y, dt, c67.x);
         f = fma(f, dt, c45.y);
         f = fma(f, dt, c45.x);
@@ -41,6 +47,15 @@ __device__ __forceinline__ void boys_eval8(double T, double* F, const double* __
         f = fma(f, dt, c01.x);
         F[M] = f;
         if constexpr (M > 0) {
+            const double e0 = slab[(COLS ? 1 : BOYS8_NM - M) * BOYS8_SLAB + i];
+            double x = fma(dt, 1.0 / 40320.0, 1.0 / 5040.0);
+            x = fma(x, dt, 1.0 / 720.0);
+            x = fma(x, dt, 1.0 / 120.0);
+            x = fma(x, dt, 1.0 / 24.0);
+            x = fma(x, dt, 1.0 / 6.0);
+            x = fma(x, dt, 0.5);
+            x = fma(x, dt, 1.0);
+            const double e = fma(e0 * x, dt, e0);
             const double t2 = T + T;
             static_for<0, M>([&](auto k) {
                 constexpr int m = M - 1 - decltype(k)::value;
@@ -51,6 +66,9 @@ __device__ __forceinline__ void boys_eval8(double T, double* F, const double* __
         const double rt = rsqrt_nr(T);
         F[0] = 0.88622692545275801365 * rt;  // sqrt(pi)/2
         if constexpr (M > 0) {
+            const double y = T * -1.4426950408889634074;  // -log2(e)
+            const double n = rint(y);
+            const double e = ldexp((double)__builtin_amdgcn_exp2f((float)(y - n)), (int)n);
             const double h = 0.5 * rt * rt;
             static_for<1, M + 1>([&](auto k) {
                 constexpr int m = decltype(k)::value;

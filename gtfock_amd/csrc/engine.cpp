@@ -95,6 +95,7 @@ int GtfSystem::init(const std::vector<const BasisSet*>& mols, hipStream_t st)
         mat_total += (long)b->nbf * b->nbf;
     }
     fstart.push_back(mols[nmol - 1]->nbf);
+    h_fstart = fstart;
     std::vector<int> moln(mol_nbf);
     d_L = dalloc<int>(nshells);
     d_nprim = dalloc<int>(nshells);
@@ -127,7 +128,7 @@ int GtfSystem::init(const std::vector<const BasisSet*>& mols, hipStream_t st)
     std::vector<double> boys((size_t)BOYS_NGRID * BOYS_NCOL);
     gtf_boys_table(boys.data(), BOYS_NGRID, BOYS_NCOL, BOYS_DELTA);
     if (upload(d_boys, boys, st)) return -1;
-    std::vector<double> b8((size_t)BOYS8_NM * BOYS8_SLAB);
+    std::vector<double> b8((size_t)BOYS8_TOTAL);
     gtf_boys_taylor_tables(b8.data());
     d_boys8 = dalloc<double>(b8.size());
     if (!d_boys8) return -2;
@@ -144,8 +145,11 @@ int GtfSystem::init(const std::vector<const BasisSet*>& mols, hipStream_t st)
     h_type.resize(npairs);
     h_pnprim.resize(npairs);
     h_pair_mol.resize(npairs);
-    std::vector<int> ppoff(npairs);
-    std::vector<long> peoff(npairs), pzoff(npairs);
+    h_ppoff.resize(npairs);
+    h_peoff.resize(npairs);
+    h_pzoff.resize(npairs);
+    std::vector<int>& ppoff = h_ppoff;
+    std::vector<long>&peoff = h_peoff, &pzoff = h_pzoff;
     long np = 0, ne = 0, nz = 0;
     for (int m = 0; m < nmol; m++) {
         const int s0 = mol_shell_off[m];
@@ -176,6 +180,7 @@ int GtfSystem::init(const std::vector<const BasisSet*>& mols, hipStream_t st)
         }
     nprimpairs = np;
     nE = ne;
+    nEz = nz;
     d_s1 = dalloc<int>(npairs);
     d_s2 = dalloc<int>(npairs);
     d_pnprim = dalloc<int>(npairs);
@@ -226,13 +231,13 @@ void GtfSystem::dfree(void* p)
 
 PairView GtfSystem::pair_view() const
 {
-    return PairView{d_s1, d_s2, d_pnprim, d_ppoff, d_peoff, d_prim, d_E, d_pzoff, d_Ez, d_pq, 0.0};
+    return PairView{d_s1, d_s2, d_pnprim, d_ppoff, d_peoff, d_prim, d_E, d_pzoff, d_Ez, d_pq, d_Ef, d_Ezf, 0.0};
 }
 
-static int launch(eri_kernel_t fn, EriArgs& a, int blocks, hipStream_t st, size_t lds = 0)
+static int launch(eri_kernel_t fn, EriArgs& a, int blocks, hipStream_t st, size_t lds = 0, int threads = 256)
 {
     void* args[] = {&a};
-    SYS_CHECK(hipLaunchKernel((const void*)fn, dim3(blocks), dim3(256), args, lds, st));
+    SYS_CHECK(hipLaunchKernel((const void*)fn, dim3(blocks), dim3(threads), args, lds, st));
     return 0;
 }
 
@@ -247,7 +252,18 @@ int GtfSystem::screen(double tolscr)
         int dev = 0, lds = 0;
         if (hipGetDevice(&dev) == hipSuccess &&
             hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && lds > 0)
-            max_lds = (size_t)lds;
+            max_lds = (size_t)lds - 64;  // the kernels' static LDS
+        if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1) ncu = 256;
+        for (int c = 0; c < GTF_NCLASSES; c++) {
+            const EriClassInfo* ci = gtf_eri_class(c);
+            for (int ex = 0; ex < 2; ex++) {
+                hipFuncAttributes fa{};
+                const eri_kernel_t fn = ex ? ci->jk_tile_t[1] : ci->jk_tile[1];
+                tile_regs[2 * c + ex] = 256;
+                if (fn && hipFuncGetAttributes(&fa, (const void*)fn) == hipSuccess && fa.numRegs > 0)
+                    tile_regs[2 * c + ex] = (fa.numRegs + 7) / 8 * 8;
+            }
+        }
     }
     tol = tolscr;
     tol2 = tolscr * tolscr;
@@ -384,6 +400,8 @@ int GtfSystem::screen(double tolscr)
                            o.s_id, o.sortnprim, o.sigmol};
         for (void* q : scratch) dfree(q);
     }
+    if (const int rc = pack_kets()) return rc;
+    if (const int rc = reserve_jk(1)) return rc;
     dfree(d_vbits);
     dfree(d_eta);
     dfree(d_ptype);
@@ -464,6 +482,71 @@ int GtfSystem::screen(double tolscr)
     return 0;
 }
 
+// The ket records of every list: a segment's kets in blocks of 64, a block's
+// rows as many as its largest primitive count.  One allocation and one upload
+// for all lists: a list each cost PFock_create of C24H12 a tenth of its time.
+int GtfSystem::pack_kets()
+{
+    static const int la[GTF_NPAIRTYPES] = {0, 1, 1, 2, 2, 2}, lb[GTF_NPAIRTYPES] = {0, 0, 1, 0, 1, 2};
+    long n = 0, rows[GTF_NPAIRTYPES], bytes = 0;
+    for (int t = 0; t < GTF_NPAIRTYPES; t++) n += nsig[t];
+    std::vector<int> base(n);
+    KetPack k[GTF_NPAIRTYPES] = {};
+    int* at = base.data();
+    for (int t = 0; t < GTF_NPAIRTYPES; at += nsig[t++]) {
+        rows[t] = 0;
+        for (int g = 0; g < nseg; g++)
+            for (int j0 = 0; j0 < seg_len[t][g]; j0 += GTF_KET_BLOCK) {
+                const int s0 = seg_start[t][g] + j0, m = std::min(GTF_KET_BLOCK, seg_len[t][g] - j0);
+                int mx = 0;
+                for (int l = 0; l < m; l++) {
+                    at[s0 + l] = (int)(rows[t] * GTF_KET_BLOCK + l);
+                    mx = std::max(mx, h_pnprim[h_sig[t][s0 + l]]);
+                }
+                rows[t] += mx;
+            }
+        if (rows[t] * GTF_KET_BLOCK > INT32_MAX) return -2;
+        k[t].n = nsig[t];
+        k[t].sig = d_sig[t];
+        k[t].nnz = herm_nnz_lookup(la[t], lb[t]);
+        k[t].nfull = KetView::full(t) ? nsph(la[t]) * nsph(lb[t]) * nherm(la[t] + lb[t]) : 0;
+    }
+    // records, bounds, full coefficients, then info and the int arrays; every
+    // part is a multiple of 16 bytes or comes last
+    auto part = [&](long size) {
+        const long o = bytes;
+        bytes += (size + 15) / 16 * 16;
+        return o;
+    };
+    long od[GTF_NPAIRTYPES], of[GTF_NPAIRTYPES], oq[GTF_NPAIRTYPES], oi[GTF_NPAIRTYPES], on[GTF_NPAIRTYPES];
+    for (int t = 0; t < GTF_NPAIRTYPES; t++) {
+        const long slots = rows[t] * GTF_KET_BLOCK;
+        od[t] = part(slots * KetView::rec(k[t].nnz) * (long)sizeof(double2));
+        of[t] = part(slots * k[t].nfull * (long)sizeof(double));
+        oq[t] = part(slots * (long)sizeof(double));
+        oi[t] = part(nsig[t] * (long)sizeof(int4));
+        on[t] = part(nsig[t] * (long)sizeof(int));
+    }
+    const long ob = part(n * (long)sizeof(int));
+    char* mem = dalloc<char>(bytes);
+    if (!mem) return -2;
+    int* d_base = (int*)(mem + ob);
+    if (upload(d_base, base, stream)) return -1;
+    for (int t = 0; t < GTF_NPAIRTYPES; d_base += nsig[t++]) {
+        k[t].base = d_base;
+        k[t].d = (double2*)(mem + od[t]);
+        k[t].f = (double*)(mem + of[t]);
+        k[t].q = (double*)(mem + oq[t]);
+        k[t].info = (int4*)(mem + oi[t]);
+        k[t].nprim = (int*)(mem + on[t]);
+        if (gtf_pack_kets(stream, pair_view(), d_fstart, k[t])) return -1;
+        kv[t] = KetView{k[t].base, k[t].d, k[t].f, k[t].q, k[t].info, k[t].nprim};
+    }
+    // the upload reads base
+    SYS_CHECK(hipStreamSynchronize(stream));
+    return 0;
+}
+
 // prefix sums of primitive-pair counts over a type list in value order
 // (segment by segment): kp[s0 + k] - kp[s0] = sum over the k largest of a segment
 std::vector<double> GtfSystem::ket_prim_prefix(int B) const
@@ -530,8 +613,10 @@ int GtfSystem::prim_census(double* hi, double* lo)
     SYS_CHECK(hipMemsetAsync(d_out, 0, sizeof(unsigned long long) * 2 * GTF_NCLASSES, stream));
     PairView pv = pair_view();
     pv.peps = prim_tol;
-    std::vector<std::vector<int4>> rows;  // tile lists of the classes that run without tiles
-    std::vector<int4*> tmp;
+    // run lists of the classes that run without tiles
+    std::vector<std::vector<int4>> rows;
+    std::vector<std::vector<int>> bras;
+    std::vector<void*> tmp;
     int rc = 0;
     for (int cls = 0; cls < GTF_NCLASSES && rc == 0; cls++) {
         if (nq[cls] == 0) continue;
@@ -552,15 +637,17 @@ int GtfSystem::prim_census(double* hi, double* lo)
         if (ntiles[cls] > 0 || ntiles_lo[cls] > 0) {
             c.tau2 = class_tau2(cls);
             if (ntiles[cls] > 0) {
-                c.tiles = d_tiles[cls];
-                c.ntiles = ntiles[cls];
+                c.runs = d_runs[cls];
+                c.run_row = d_run_row[cls];
+                c.nruns = nruns[cls];
                 c.low = 0;
                 c.out = d_out + cls;
                 if (gtf_prim_census(stream, c)) rc = -1;
             }
             if (ntiles_lo[cls] > 0 && rc == 0) {
-                c.tiles = d_tiles_lo[cls];
-                c.ntiles = ntiles_lo[cls];
+                c.runs = d_runs_lo[cls];
+                c.run_row = d_run_row_lo[cls];
+                c.nruns = nruns_lo[cls];
                 c.low = 1;
                 c.pv.peps = prim_tol_fp32();
                 c.out = d_out + GTF_NCLASSES + cls;
@@ -569,21 +656,26 @@ int GtfSystem::prim_census(double* hi, double* lo)
         } else {
             // the global-atomic path evaluates each row's exact ket prefix in FP64
             rows.emplace_back();
-            std::vector<int4>& v = rows.back();
+            bras.emplace_back();
             for (int k = 0; k < nrows[cls]; k++)
-                if (h_exact[cls][k] > 0) {
-                    const int s0 = seg_start[B][h_row_seg[cls][k]];
-                    v.push_back(make_int4(h_row_bra[cls][k], s0, s0 + (int)h_exact[cls][k], 1));
+                for (long b = 0; b < h_exact[cls][k]; b += GTF_RUN_MAX_KETS) {
+                    const int n = (int)std::min<long>(GTF_RUN_MAX_KETS, h_exact[cls][k] - b);
+                    rows.back().push_back(make_int4(seg_start[B][h_row_seg[cls][k]] + (int)b, GTF_RUN_SPAN(n, 0, 1),
+                                                    GTF_RUN_CHUNKS(0, 0, 0, 1), 0));
+                    bras.back().push_back(h_row_bra[cls][k]);
                 }
-            if (v.empty()) continue;
-            int4* d = dalloc<int4>(v.size());
-            if (!d || upload(d, v, stream)) {
+            if (rows.back().empty()) continue;
+            int4* d = dalloc<int4>(rows.back().size());
+            if (d) tmp.push_back(d);
+            int* dr = dalloc<int>(bras.back().size());
+            if (dr) tmp.push_back(dr);
+            if (!d || !dr || upload(d, rows.back(), stream) || upload(dr, bras.back(), stream)) {
                 rc = -1;
                 break;
             }
-            tmp.push_back(d);
-            c.tiles = d;
-            c.ntiles = (int)v.size();
+            c.runs = d;
+            c.run_row = dr;
+            c.nruns = (int)rows.back().size();
             c.tau2 = 0.0;
             c.low = 0;
             c.out = d_out + cls;
@@ -595,7 +687,7 @@ int GtfSystem::prim_census(double* hi, double* lo)
                     hipStreamSynchronize(stream) != hipSuccess))
         rc = -1;
     (void)hipStreamSynchronize(stream);  // the row lists are read by the uploads
-    for (int4* d : tmp) dfree(d);
+    for (void* d : tmp) dfree(d);
     dfree(d_out);
     if (rc) return rc;
     for (int cls = 0; cls < GTF_NCLASSES; cls++) {
@@ -633,13 +725,19 @@ int GtfSystem::build_tiles()
     const double t0 = sys_wtime();
     // the previous tiles may still be read by a launch in flight
     SYS_CHECK(hipStreamSynchronize(stream));
+    if (tau > 0.0 && !d_Ezf) {
+        // the FP32 tiles read the bra coefficients as scalars, already rounded
+        d_Ef = dalloc<float>(nE);
+        d_Ezf = dalloc<float>(nEz);
+        if (!d_Ef || !d_Ezf || gtf_round_f32(stream, d_E, nE, d_Ef) || gtf_round_f32(stream, d_Ez, nEz, d_Ezf)) return -1;
+    }
     // fill the shared prefix and segment-maximum caches first: the classes
     // are then cut on host threads that only read shared state
     for (int t = 0; t < GTF_NPAIRTYPES; t++) {
         list_prim_prefix(t);
         seg_nprim_max(t, 0);
     }
-    std::vector<int4> hv[GTF_NCLASSES], lv[GTF_NCLASSES];
+    TileList hv[GTF_NCLASSES], lv[GTF_NCLASSES];
     {
         const int nth = std::max(1, std::min<int>(16, (int)std::thread::hardware_concurrency()));
         std::atomic<int> next{0};
@@ -651,10 +749,7 @@ int GtfSystem::build_tiles()
         work();
         for (std::thread& t : pool) t.join();
     }
-    for (int cls = 0; cls < GTF_NCLASSES; cls++)
-        if (upload_class_tiles(cls, hv[cls], lv[cls])) return -1;
-    // the uploads read hv / lv
-    SYS_CHECK(hipStreamSynchronize(stream));
+    if (upload_tiles(hv, lv, 0, GTF_NCLASSES)) return -1;
     setup_s[5] = sys_wtime() - t0;
     return 0;
 }
@@ -666,146 +761,295 @@ int GtfSystem::build_class_tiles(int cls)
     SYS_CHECK(hipStreamSynchronize(stream));
     list_prim_prefix(B);
     seg_nprim_max(B, 0);
-    std::vector<int4> hv, lv;
-    cut_class_tiles(cls, hv, lv);
-    if (upload_class_tiles(cls, hv, lv)) return -1;
+    TileList hv[GTF_NCLASSES], lv[GTF_NCLASSES];
+    cut_class_tiles(cls, hv[cls], lv[cls]);
+    return upload_tiles(hv, lv, cls, cls + 1);
+}
+
+// Replaces the device tiles of the classes [c0, c1) by hv (FP64) and lv
+// (FP32), in one allocation and one copy; the stream must have no launch in
+// flight that reads the old ones.  An allocation that several classes share is
+// freed with the last of them.
+int GtfSystem::upload_tiles(const TileList* hv, const TileList* lv, int c0, int c1)
+{
+    for (int c = c0; c < c1; c++) {
+        void* old = tile_mem[c];
+        tile_mem[c] = nullptr;
+        if (old && std::find(tile_mem, tile_mem + GTF_NCLASSES, old) == tile_mem + GTF_NCLASSES) dfree(old);
+    }
+    std::vector<char> host;
+    size_t size = 0;
+    for (int c = c0; c < c1; c++)
+        for (const TileList* v : {&hv[c], &lv[c]})
+            size += v->tiles.size() * sizeof(TileHead) + v->runs.size() * (sizeof(int4) + sizeof(int)) + 256;
+    host.reserve(size);
+    auto put = [&](const void* p, size_t bytes) {
+        const size_t o = host.size();
+        host.insert(host.end(), (const char*)p, (const char*)p + bytes);
+        host.resize(o + (bytes + 63) / 64 * 64);
+        return o;
+    };
+    size_t at[GTF_NCLASSES][2][3];
+    for (int c = c0; c < c1; c++)
+        for (int low = 0; low < 2; low++) {
+            const TileList& v = low ? lv[c] : hv[c];
+            at[c][low][0] = put(v.tiles.data(), v.tiles.size() * sizeof(TileHead));
+            at[c][low][1] = put(v.runs.data(), v.runs.size() * sizeof(int4));
+            at[c][low][2] = put(v.run_row.data(), v.run_row.size() * sizeof(int));
+        }
+    char* mem = dalloc<char>(host.size());
+    if (!mem) return -1;
+    if (upload(mem, host, stream)) return -1;
+    for (int c = c0; c < c1; c++) {
+        tile_mem[c] = mem;
+        d_tiles[c] = (TileHead*)(mem + at[c][0][0]);
+        d_runs[c] = (int4*)(mem + at[c][0][1]);
+        d_run_row[c] = (int*)(mem + at[c][0][2]);
+        nruns[c] = (int)hv[c].runs.size();
+        d_tiles_lo[c] = (TileHead*)(mem + at[c][1][0]);
+        d_runs_lo[c] = (int4*)(mem + at[c][1][1]);
+        d_run_row_lo[c] = (int*)(mem + at[c][1][2]);
+        nruns_lo[c] = (int)lv[c].runs.size();
+    }
+    // the upload reads host
     SYS_CHECK(hipStreamSynchronize(stream));
     return 0;
 }
 
-// replaces the device tiles of a class by hv (FP64) and lv (FP32); the
-// stream must have no launch in flight that reads the old ones
-int GtfSystem::upload_class_tiles(int cls, const std::vector<int4>& hv, const std::vector<int4>& lv)
-{
-    dfree(d_tiles[cls]);
-    dfree(d_tiles_lo[cls]);
-    d_tiles[cls] = d_tiles_lo[cls] = nullptr;
-    if (!hv.empty()) {
-        d_tiles[cls] = dalloc<int4>(hv.size());
-        if (!d_tiles[cls] || upload(d_tiles[cls], hv, stream)) return -1;
-    }
-    if (!lv.empty()) {
-        d_tiles_lo[cls] = dalloc<int4>(lv.size());
-        if (!d_tiles_lo[cls] || upload(d_tiles_lo[cls], lv, stream)) return -1;
-    }
-    return 0;
-}
-
-// Tiles of one class: up to shape.units work units of one bra row; (bra row,
-// first ket, end ket) with ket positions absolute in the ket type list.  With
-// tau > 0 each row splits at the first ket whose Schwarz bound
-// sqrt(v_bra v_ket) < tau: FP64 tiles cover the block-padded prefix, FP32
-// tiles start at the block holding the split; the kernels re-test the exact
-// predicates per quartet.  Host work only; reads the class's own fields and
-// shared state that list_prim_prefix / seg_nprim_max have cached already.
-void GtfSystem::cut_class_tiles(int cls, std::vector<int4>& hv, std::vector<int4>& lv)
+// Tiles of one class: runs of kets of one bra row, ket positions absolute in
+// the ket type list.  With tau > 0 each row splits at the first ket whose
+// Schwarz bound sqrt(v_bra v_ket) < tau: FP64 runs cover the block-padded
+// prefix, FP32 runs start at the block holding the split; the kernels re-test
+// the exact predicates per quartet.  Host work only; reads the class's own
+// fields and shared state that list_prim_prefix / seg_nprim_max have cached
+// already.
+//
+// A row holds the kets of one primitive-count bucket, often fewer than a
+// hundred, so a tile takes the runs of all of its bra's rows until it has
+// about tile_pq primitive quartets; a row beyond that is cut at multiples of
+// 64 kets, then by bra-primitive chunks, then by component chunks.
+void GtfSystem::cut_class_tiles(int cls, TileList& hv, TileList& lv)
 {
     const double tau2 = class_tau2(cls);
-    {
-        int A, B;
-        gtf_class_types(cls, A, B);
-        const EriClassInfo* ci = gtf_eri_class(cls);
-        const int NA = 2 * ci->la + 1, NB = 2 * ci->lb + 1;
-        const int NCD = (2 * ci->lc + 1) * (2 * ci->ld + 1);
-        const TileShape sh = shape[cls];
-        // threads per quartet of the kernel that runs the class, and the most
-        // kets a tile can hold (its J_PQ rows live in LDS)
-        const int ns = exchanged(cls) ? ci->nsplit_t : ci->nsplit;
-        const int kmax = std::max(1, sh.units / ns);
-        // LDS of a launch: the Boys slab (if staged) plus one work area
-        // (strips, J_MN, J_PQ rows) per density digested
-        tile_lds_work[cls] = sizeof(double) * ((size_t)(NA + NB) * nbf + NA * NB + (size_t)kmax * NCD);
-        tile_lds[cls] = sizeof(double) * (sh.boys_lds ? GTF_BOYS_LDS : 0) + tile_lds_work[cls];
-        ntiles[cls] = ntiles_lo[cls] = 0;
-        nq_lo[cls] = 0;
-        nprimq_lo[cls] = 0.0;
-        hv.clear();
-        lv.clear();
-        if (nq[cls] == 0 || !use_tiles || tile_lds[cls] > max_lds) return;
-        const std::vector<double>& vs = h_sorted[B];
-        const std::vector<double> kp = ket_prim_prefix(B);
-        // Tiles of the kets [b, e) of one row of segment sg, cut by work units
-        // and by primitive quartets.  nic (bra-primitive chunks per quartet)
-        // follows the largest ket primitive count of the segment (kets of a
-        // segment share a primitive-count bucket); with it fixed, a tile's unit
-        // count grows by a constant per ket, and its primitive-quartet cost is
-        // read off the prefix sums of the list, so each tile end is one binary
-        // search.
-        const std::vector<double>& lp = h_listprim[B];
-        const bool exch = exchanged(cls);
-        std::vector<std::pair<double, int4>> hi, lo;
-        auto cut = [&](std::vector<std::pair<double, int4>>& out, int r, int nb, int nkmax, long b, long e) {
-            // bra-primitive chunks per quartet: about unit_pq primitive
-            // quartets per unit; a power of two not above nb when one thread
-            // owns the whole bra (its lanes then reduce with shuffles); none
-            // for the exchanged kernels
-            const int ich = std::max(1, std::min(nb, (sh.unit_pq + nkmax - 1) / nkmax));
-            int nic = exch ? 1 : (nb + ich - 1) / ich;
-            if (ns == 1) {
-                int p2 = 1;
-                while (2 * p2 <= nic && 2 * p2 <= 64) p2 *= 2;  // a group stays in one wavefront
-                nic = p2;
-            }
-            // keep one ket's units within a tile
-            while (nic * ns > sh.units && nic > 1) nic = ns == 1 ? nic / 2 : nic - 1;
-            const long per_ket = (long)nic * ns;
-            const long max_kets = std::max(1L, std::min<long>(sh.units / per_ket, kmax));
-            long j = b;
-            while (j < e) {
-                // the most kets whose primitive quartets stay within tile_pq
-                const double limit = lp[j] + (double)sh.tile_pq / nb;
-                long je = std::upper_bound(lp.begin() + j + 1, lp.begin() + e + 1, limit) - lp.begin() - 1;
-                je = std::max(j + 1, std::min(je, std::min(e, j + max_kets)));
-                out.push_back({(double)nb * (lp[je] - lp[j]), make_int4(r, (int)j, (int)je, nic)});
-                j = je;
-            }
+    int A, B;
+    gtf_class_types(cls, A, B);
+    const EriClassInfo* ci = gtf_eri_class(cls);
+    const TileShape sh = shape[cls];
+    // component chunks of the kernel that runs the class, and the most kets of
+    // a run
+    const int ns = exchanged(cls) ? ci->nsplit_t : ci->nsplit_tile;
+    const int kmax = std::min(GTF_RUN_MAX_KETS, std::max(1, sh.units / ns));
+    ntiles[cls] = ntiles_lo[cls] = 0;
+    nq_lo[cls] = 0;
+    nprimq_lo[cls] = 0.0;
+    hv = TileList();
+    lv = TileList();
+    if (nq[cls] == 0 || !use_tiles || tile_launch(cls, 1, 1).grid == 0) return;
+    const std::vector<double>& vs = h_sorted[B];
+    const std::vector<double> kp = ket_prim_prefix(B);
+    auto log2_floor = [](long x) {
+        int l = 0;
+        while ((2L << l) <= x) l++;
+        return l;
+    };
+    // How the kets of a row are chunked: a unit (64 lanes) has about unit_pq
+    // primitive quartets per lane; a remainder of at most 32 kets lets several
+    // lanes share a ket.
+    struct Chunking {
+        int lic, ljc;
+        double unit;  // cost of a unit, primitive quartets of a full wavefront
+    };
+    // a unit's loads, digestion and bookkeeping cost about as much as this many
+    // primitive quartets per lane
+    const double unit_fixed = 12.0;
+    auto chunking = [&](int nb, int nkmax, long kets) {
+        Chunking c{0, 0, 0.0};
+        if (kets <= GTF_KET_BLOCK / 2) c.ljc = std::min(log2_floor(GTF_KET_BLOCK / kets), log2_floor(nkmax));
+        const long upq = std::max(1L, (long)nb * nkmax >> c.ljc);
+        c.lic = std::min({log2_floor(std::max(1, nkmax >> c.ljc)), log2_floor((upq + sh.unit_pq - 1) / sh.unit_pq),
+                          GTF_MAX_LIC});
+        c.unit = GTF_KET_BLOCK * ((double)upq / (1L << c.lic) + unit_fixed);
+        return c;
+    };
+    auto blocks = [](long kets, int ljc) { return ((kets << ljc) + GTF_KET_BLOCK - 1) / GTF_KET_BLOCK; };
+    // the part of each row in FP64 and in FP32 runs
+    struct Part {
+        int r, nb, nkmax;
+        long b, e;
+    };
+    std::vector<Part> hi, lo;
+    for (int row = 0; row < nrows[cls]; row++) {
+        const long c = h_exact[cls][row];
+        if (c == 0) continue;
+        const int r = h_row_bra[cls][row], sg = h_row_seg[cls][row];
+        const int s0 = seg_start[B][sg], nket = seg_len[B][sg];
+        const int nb = h_pnprim[h_sig[A][r]];
+        long c64 = c;
+        if (tau2 > 0.0) {
+            const double vk = h_sigv[A][r];
+            c64 = std::upper_bound(vs.begin() + s0, vs.begin() + s0 + c, vk, [&](double v, double x) {
+                      return !(v * x >= tau2);
+                  }) - (vs.begin() + s0);
+        }
+        const long pad = std::min<long>(nket, ((c + GTF_KET_BLOCK - 1) / GTF_KET_BLOCK) * GTF_KET_BLOCK);
+        const long pad64 = std::min<long>(nket, ((c64 + GTF_KET_BLOCK - 1) / GTF_KET_BLOCK) * GTF_KET_BLOCK);
+        const int nkmax = h_segmax[B][sg];
+        if (pad64 > 0) hi.push_back({r, nb, nkmax, s0, s0 + pad64});
+        if (c > c64) {
+            const long b0 = (c64 / GTF_KET_BLOCK) * GTF_KET_BLOCK;
+            lo.push_back({r, nb, nkmax, s0 + b0, s0 + pad});
+            nq_lo[cls] += c - c64;
+            nprimq_lo[cls] += (double)nb * (kp[s0 + c] - kp[s0 + c64]);
+        }
+    }
+    const bool full_E = !exchanged(cls) && ci->full_E;
+    auto head = [&](int r, int run0, int nrun) {
+        TileHead h{};
+        const int id = h_sig[A][r], m = h_sigmol[A][r];
+        h.row = r;
+        h.run0 = run0;
+        h.nrun = nrun;
+        h.bra = id;
+        h.prim = h_ppoff[id];
+        h.nprim = h_pnprim[id];
+        h.oM = h_fstart[h_s1[id]];
+        h.oN = h_fstart[h_s2[id]];
+        h.two = h_s1[id] != h_s2[id];
+        h.nbf = mol_nbf[m];
+        h.mol = m;
+        h.rank = h_rank[A][r];
+        h.mat = mol_mat_off[m];
+        h.E = full_E ? h_peoff[id] : h_pzoff[id];
+        return h;
+    };
+    const int resident = std::max(1, tile_launch(cls, INT32_MAX, 1).grid);
+    auto cut = [&](const std::vector<Part>& parts, TileList& out) {
+        double total = 0.0, units = 1.0;
+        for (const Part& p : parts) {
+            const Chunking c = chunking(p.nb, p.nkmax, p.e - p.b);
+            const double n = (double)blocks(p.e - p.b, c.ljc) * (1L << c.lic) * ns;
+            total += c.unit * n;
+            units += n;
+        }
+        // a class with little work is cut finer, so that it spreads over the
+        // chip, down to a unit for each wavefront
+        const double target = std::min<double>(
+            sh.tile_pq, std::max(total / (GTF_TILES_PER_WG * resident), GTF_MIN_TILE_UNITS * total / units));
+        // a wavefront takes all chunks of 64 kets: at most an eighth of a tile
+        const double most = target / 8;
+        struct Tile {
+            double cost;
+            int row, run0, nrun;
         };
-        for (int row = 0; row < nrows[cls]; row++) {
-            const long c = h_exact[cls][row];
-            if (c == 0) continue;
-            const int r = h_row_bra[cls][row], sg = h_row_seg[cls][row];
-            const int s0 = seg_start[B][sg], nket = seg_len[B][sg];
-            const int nb = h_pnprim[h_sig[A][r]];
-            long c64 = c;
-            if (tau2 > 0.0) {
-                const double vk = h_sigv[A][r];
-                c64 = std::upper_bound(vs.begin() + s0, vs.begin() + s0 + c, vk, [&](double v, double x) {
-                          return !(v * x >= tau2);
-                      }) - (vs.begin() + s0);
+        std::vector<Tile> tiles;
+        double cost = 0.0;
+        int first = 0;
+        auto close = [&](int r) {
+            if ((int)out.runs.size() > first)
+                tiles.push_back({cost, r, first, (int)out.runs.size() - first});
+            first = (int)out.runs.size();
+            cost = 0.0;
+        };
+        for (size_t k = 0; k < parts.size(); k++) {
+            const Part& p = parts[k];
+            for (long j = p.b; j < p.e;) {
+                const Chunking c = chunking(p.nb, p.nkmax, p.e - j);
+                const long nic = 1L << c.lic;
+                long icn = nic, spn = ns;
+                while (icn > 1 && c.unit * spn * icn > most) icn >>= 1;
+                while (spn > 1 && c.unit * spn * icn > most) spn = (spn + 1) / 2;
+                // kets of this run: what the target leaves, in blocks of 64
+                long n = std::min<long>(kmax, p.e - j);
+                if (n > GTF_KET_BLOCK) {
+                    const long fit = (long)((target - cost) / (c.unit * icn * spn));
+                    n = std::min(n, std::max(1L, fit) * GTF_KET_BLOCK);
+                    if (n < p.e - j && n > GTF_KET_BLOCK) n -= n % GTF_KET_BLOCK;
+                }
+                const long nblk = blocks(n, c.ljc);
+                for (long ic = 0; ic < nic; ic += icn)
+                    for (long sp = 0; sp < ns; sp += spn) {
+                        const long m = std::min(spn, ns - sp);
+                        out.runs.push_back(make_int4((int)j, GTF_RUN_SPAN((int)n, (int)sp, (int)m),
+                                                     GTF_RUN_CHUNKS(c.lic, c.ljc, (int)ic, (int)icn), 0));
+                        out.run_row.push_back(p.r);
+                        cost += c.unit * nblk * m * icn;
+                        if (cost >= target) close(p.r);
+                    }
+                j += n;
             }
-            const long pad = std::min<long>(nket, ((c + GTF_KET_BLOCK - 1) / GTF_KET_BLOCK) * GTF_KET_BLOCK);
-            const long pad64 = std::min<long>(nket, ((c64 + GTF_KET_BLOCK - 1) / GTF_KET_BLOCK) * GTF_KET_BLOCK);
-            const int nkmax = h_segmax[B][sg];
-            cut(hi, r, nb, nkmax, s0, s0 + pad64);
-            if (c > c64) {
-                const long b0 = (c64 / GTF_KET_BLOCK) * GTF_KET_BLOCK;
-                cut(lo, r, nb, nkmax, s0 + b0, s0 + pad);
-                nq_lo[cls] += c - c64;
-                nprimq_lo[cls] += (double)nb * (kp[s0 + c] - kp[s0 + c64]);
-            }
+            if (k + 1 == parts.size() || parts[k + 1].r != p.r) close(p.r);
         }
         // heaviest tiles first, so the light ones fill the tail
-        auto heavy_first = [](const std::pair<double, int4>& x, const std::pair<double, int4>& y) {
-            return x.first > y.first;
-        };
-        std::stable_sort(hi.begin(), hi.end(), heavy_first);
-        std::stable_sort(lo.begin(), lo.end(), heavy_first);
-        hv.reserve(hi.size());
-        lv.reserve(lo.size());
-        for (auto& x : hi) hv.push_back(x.second);
-        for (auto& x : lo) lv.push_back(x.second);
-        ntiles[cls] = (int)hv.size();
-        ntiles_lo[cls] = (int)lv.size();
-    }
+        std::stable_sort(tiles.begin(), tiles.end(), [](const Tile& x, const Tile& y) { return x.cost > y.cost; });
+        out.tiles.reserve(tiles.size());
+        for (const Tile& t : tiles) out.tiles.push_back(head(t.row, t.run0, t.nrun));
+    };
+    cut(hi, hv);
+    cut(lo, lv);
+    ntiles[cls] = (int)hv.tiles.size();
+    ntiles_lo[cls] = (int)lv.tiles.size();
 }
-
 
 bool GtfSystem::fits_densities(int nd) const
 {
     for (int cls = 0; cls < GTF_NCLASSES; cls++)
-        if (ntiles[cls] + ntiles_lo[cls] > 0 && tile_lds[cls] + (size_t)(nd - 1) * tile_lds_work[cls] > max_lds)
-            return false;
+        if (ntiles[cls] + ntiles_lo[cls] > 0 && tile_launch(cls, 1, nd).grid == 0) return false;
     return true;
+}
+
+// Workgroup size: the one that puts more wavefronts on a CU under the LDS and
+// register limits, 256 threads on a tie (shorter waits at a tile's end).  The
+// grid is what the chip holds at once, at most the shape's: more workgroups
+// would only start later and set up their LDS again.
+GtfSystem::TileLaunch GtfSystem::tile_launch(int cls, int n, int nd) const
+{
+    TileLaunch t{};
+    const EriClassInfo* ci = gtf_eri_class(cls);
+    const int NA = 2 * ci->la + 1, NB = 2 * ci->lb + 1, NCD = (2 * ci->lc + 1) * (2 * ci->ld + 1);
+    const int simd_waves = std::max(1, 512 / std::max(1, tile_regs[2 * cls + (exchanged(cls) ? 1 : 0)]));
+    const size_t rows = (size_t)(NA + NB) * nbf;
+    int best = 0;
+    for (int threads = 256; threads <= ci->tile_threads; threads *= 2) {
+        const int w = threads / 64;
+        const size_t plain = sizeof(double) * (size_t)nd * tile_work(NA + NB, nbf, NA * NB, NCD, nd == 1 ? w : 0);
+        const size_t with = plain + sizeof(double) * ((size_t)nd * rows + GTF_BOYS_LDS);
+        const bool staged = shape[cls].boys_lds && with <= max_lds;
+        const size_t lds = staged ? with : plain;
+        const int wgs = (int)std::min<size_t>(max_lds / lds, std::max(1, 4 * simd_waves / w));
+        if (wgs * w > best) {
+            best = wgs * w;
+            t.staged = staged;
+            t.lds = lds;
+            t.threads = threads;
+            t.grid = std::min({n, shape[cls].grid, wgs * ncu});
+        }
+    }
+    return t;
+}
+
+// J_PQ and density copies for nd densities
+int GtfSystem::reserve_jk(int nd)
+{
+    if (nd <= jk_nd) return 0;
+    SYS_CHECK(hipStreamSynchronize(stream));
+    static const int nc[GTF_NPAIRTYPES] = {1, 3, 3, 5, 5, 5}, nf[GTF_NPAIRTYPES] = {1, 1, 3, 1, 3, 5};
+    dfree(d_jkl);
+    size_t n = 0;
+    for (int t = 0; t < GTF_NPAIRTYPES; t++) n += (size_t)nd * nc[t] * nf[t] * nsig[t];
+    d_jkl = dalloc<double>(2 * n);
+    jk_nd = 0;
+    if (!d_jkl) return -2;
+    double* p = d_jkl;
+    for (int t = 0; t < GTF_NPAIRTYPES; t++) {
+        const size_t m = (size_t)nd * nc[t] * nf[t] * nsig[t];
+        jkl.t[t] = JkList{nsig[t], nc[t], nf[t], kv[t].info, p, p + n};
+        p += m;
+    }
+    jkl.s1 = d_s1;
+    jkl.mbase = d_mbase;
+    jkl.mld = d_mld;
+    jk_nd = nd;
+    return 0;
 }
 
 int GtfSystem::jk(const double* D, double* J, double* K, int nd, long dstride)
@@ -817,7 +1061,7 @@ int GtfSystem::jk(const double* D, double* J, double* K, int nd, long dstride)
             for (int lo = 0; lo < 2; lo++) {
                 const int n = nq[cls] == 0 ? 0 : lo ? ntiles_lo[cls] : ntiles[cls];
                 wg_off[2 * cls + lo] = tot;
-                wg_n[2 * cls + lo] = std::min(n, shape[cls].grid);
+                wg_n[2 * cls + lo] = n > 0 ? tile_launch(cls, n, nd).grid : 0;
                 tot += wg_n[2 * cls + lo];
             }
         if (tot > wgstat_cap) {
@@ -828,7 +1072,8 @@ int GtfSystem::jk(const double* D, double* J, double* K, int nd, long dstride)
             wgstat_cap = tot;
         }
     }
-    if (gtf_fill_int(stream, d_counters, 2 * GTF_NCLASSES, 0)) return -1;
+    if (reserve_jk(nd)) return -1;
+    if (gtf_jk_begin(stream, jkl, D, J, K, mat_total, nd, dstride, d_counters, 2 * GTF_NCLASSES)) return -1;
     if (!cstream[0]) {
         for (int s = 0; s < NSTREAMS; s++) {
             SYS_CHECK(hipStreamCreate(&cstream[s]));
@@ -855,7 +1100,7 @@ int GtfSystem::jk(const double* D, double* J, double* K, int nd, long dstride)
         SYS_CHECK(hipEventRecord(join_ev[s], cstream[s]));
         SYS_CHECK(hipStreamWaitEvent(stream, join_ev[s], 0));
     }
-    return 0;
+    return gtf_jk_end(stream, jkl, J, nd, dstride);
 }
 
 int GtfSystem::launch_class(int cls, hipStream_t cs, const double* D, double* J, double* K, int nd, long dstride)
@@ -892,30 +1137,28 @@ int GtfSystem::launch_class(int cls, hipStream_t cs, const double* D, double* J,
     a.mol_active = d_mol_active;
     a.row_bra = d_row_bra[cls];
     a.row_kstart = d_row_kstart[cls];
+    a.kv = kv[B];
+    a.dk = jkl.t[B].dk;
+    a.jk = jkl.t[B].jk;
+    a.nket = nsig[B];
     a.pv.peps = prim_tol;
     if (ntiles[cls] > 0 || ntiles_lo[cls] > 0) {
         a.nbf = nbf;
         a.tau2 = class_tau2(cls);
         const bool exch = exchanged(cls);
-        const int grid = shape[cls].grid;
-        const int bl = shape[cls].boys_lds ? 1 : 0;
-        const size_t lds = tile_lds[cls] + (size_t)(nd - 1) * tile_lds_work[cls];
-        if (ntiles[cls] > 0) {
-            a.tiles = d_tiles[cls];
-            a.ntiles = ntiles[cls];
-            a.counter = d_counters + cls;
-            a.wg_stat = wg_record(2 * cls, std::min(a.ntiles, grid));
-            if (launch(exch ? ci->jk_tile_t[bl] : ci->jk_tile[bl], a, std::min(a.ntiles, grid), cs, lds))
-                return -1;
-        }
-        if (ntiles_lo[cls] > 0) {
-            a.tiles = d_tiles_lo[cls];
-            a.ntiles = ntiles_lo[cls];
-            a.pv.peps = prim_tol_fp32();
-            a.counter = d_counters + GTF_NCLASSES + cls;
-            a.wg_stat = wg_record(2 * cls + 1, std::min(a.ntiles, grid));
-            if (launch(exch ? ci->jk_tile_t_lo[bl] : ci->jk_tile_lo[bl], a, std::min(a.ntiles, grid), cs, lds))
-                return -1;
+        for (int low = 0; low < 2; low++) {
+            a.ntiles = low ? ntiles_lo[cls] : ntiles[cls];
+            if (a.ntiles == 0) continue;
+            const TileLaunch t = tile_launch(cls, a.ntiles, nd);
+            const int bl = t.staged ? 1 : 0;
+            a.tiles = low ? d_tiles_lo[cls] : d_tiles[cls];
+            a.runs = low ? d_runs_lo[cls] : d_runs[cls];
+            a.pv.peps = low ? prim_tol_fp32() : prim_tol;
+            a.counter = d_counters + cls + (low ? GTF_NCLASSES : 0);
+            a.wg_stat = wg_record(2 * cls + low, t.grid);
+            const eri_kernel_t fn = low ? (exch ? ci->jk_tile_t_lo[bl] : ci->jk_tile_lo[bl])
+                                        : (exch ? ci->jk_tile_t[bl] : ci->jk_tile[bl]);
+            if (launch(fn, a, t.grid, cs, t.lds, t.threads)) return -1;
         }
         return 0;
     }
@@ -983,7 +1226,7 @@ static int best_time(hipStream_t st, int reps, float* ms, F run)
 
 int GtfSystem::time_class(int cls, const double* D, double* J, double* K, int reps, float* ms)
 {
-    if (gtf_fill_int(stream, d_counters, 2 * GTF_NCLASSES, 0)) return -1;
+    if (reserve_jk(1) || gtf_jk_begin(stream, jkl, D, J, K, mat_total, 1, 0, d_counters, 2 * GTF_NCLASSES)) return -1;
     return best_time(stream, reps, ms, [&]() {
         return gtf_fill_int(stream, d_counters, 2 * GTF_NCLASSES, 0) || launch_class(cls, stream, D, J, K);
     });

@@ -19,6 +19,10 @@
 
 // ints per class in the tile-shape entry points
 #define GTF_SHAPE_FIELDS 7
+// tiles a class is cut into, if its work allows, for each workgroup that the
+// chip holds of it
+#define GTF_TILES_PER_WG 3
+#define GTF_MIN_TILE_UNITS 4
 // default primitive screening threshold of the J/K builds
 #define GTF_PRIM_TOL_DEFAULT 1e-15
 
@@ -49,12 +53,16 @@ struct GtfSystem {
     std::vector<int> h_s1, h_s2, h_type, h_pnprim;
     int *d_s1 = nullptr, *d_s2 = nullptr, *d_pnprim = nullptr, *d_ppoff = nullptr;
     long* d_peoff = nullptr;
+    // host copies for the tile heads
+    std::vector<int> h_ppoff, h_fstart;
+    std::vector<long> h_peoff, h_pzoff;
     double4* d_prim = nullptr;
     double* d_pq = nullptr;  // Schwarz bound per primitive pair (descending within a shell pair)
     double* d_E = nullptr;
     long* d_pzoff = nullptr;
     double* d_Ez = nullptr;
-    long nprimpairs = 0, nE = 0, nprimpairs_kept = 0;
+    float *d_Ef = nullptr, *d_Ezf = nullptr;  // rounded copies, made with the first FP32 tiles
+    long nprimpairs = 0, nE = 0, nEz = 0, nprimpairs_kept = 0;
     // primitive-pair screening threshold on max |E| of a pair block
     double prim_eps = 1e-20;
     // J/K builds skip primitive quartets whose Schwarz bound q_bra q_ket is
@@ -95,6 +103,14 @@ struct GtfSystem {
     int* d_sortrank[GTF_NPAIRTYPES] = {nullptr};
     int* d_seg_start[GTF_NPAIRTYPES] = {nullptr};
     int* d_seg_len[GTF_NPAIRTYPES] = {nullptr};
+    // ket records of each list (KetView)
+    KetView kv[GTF_NPAIRTYPES] = {};
+    int pack_kets();
+    // list-ordered density elements and J_PQ accumulators, for jk_nd densities
+    JkLists jkl = {};
+    double* d_jkl = nullptr;
+    int jk_nd = 0;
+    int reserve_jk(int nd);
     // ---- quartet rows and tiles per class: a row is (bra pair, ket segment
     // of the bra's molecule)
     long nq[GTF_NCLASSES] = {0};      // screened unique quartets
@@ -108,10 +124,28 @@ struct GtfSystem {
     std::vector<long> h_exact[GTF_NCLASSES];
     double nprimq[GTF_NCLASSES] = {0};  // sum over quartets of nprim(bra) nprim(ket)
     int ntiles[GTF_NCLASSES] = {0}, ntiles_lo[GTF_NCLASSES] = {0};
-    int4* d_tiles[GTF_NCLASSES] = {nullptr};     // FP64 tiles
-    int4* d_tiles_lo[GTF_NCLASSES] = {nullptr};  // FP32 tiles
-    size_t tile_lds[GTF_NCLASSES] = {0};       // one density
-    size_t tile_lds_work[GTF_NCLASSES] = {0};  // of that, the work area each further density adds
+    TileHead* d_tiles[GTF_NCLASSES] = {nullptr};     // FP64 tiles
+    TileHead* d_tiles_lo[GTF_NCLASSES] = {nullptr};  // FP32 tiles
+    // their runs of kets, and the bra row of each run
+    int4 *d_runs[GTF_NCLASSES] = {nullptr}, *d_runs_lo[GTF_NCLASSES] = {nullptr};
+    int *d_run_row[GTF_NCLASSES] = {nullptr}, *d_run_row_lo[GTF_NCLASSES] = {nullptr};
+    int nruns[GTF_NCLASSES] = {0}, nruns_lo[GTF_NCLASSES] = {0};
+    struct TileList {
+        std::vector<TileHead> tiles;
+        std::vector<int4> runs;
+        std::vector<int> run_row;
+    };
+    // launch of a class's n tiles digesting nd densities; staged: with the Boys
+    // slab and the density rows in LDS (asked for by the shape and within
+    // max_lds)
+    struct TileLaunch {
+        bool staged;
+        size_t lds;
+        int threads, grid;  // grid 0: does not fit
+    };
+    TileLaunch tile_launch(int cls, int n, int nd) const;
+    int ncu = 256;                            // CUs of the device
+    int tile_regs[2 * GTF_NCLASSES] = {0};    // VGPRs of the tile kernels: standard, exchanged
     size_t max_lds = 65536;
     bool use_tiles = true;
     // Tile shape of each class (the autotuner's search space): at most
@@ -119,7 +153,8 @@ struct GtfSystem {
     // about `unit_pq` primitive quartets per unit (how finely a quartet's bra
     // primitives are chunked), `grid` persistent workgroups per launch, each
     // taking tiles from the class counter until none are left,
-    // `boys_lds` whether the workgroups stage the Boys slab in LDS, and
+    // `boys_lds` whether the workgroups stage the Boys slab and the bra
+    // shells' density rows in LDS (where they fit), and
     // `fp32` whether the class evaluates its quartets below the Schwarz
     // bound tau in FP32 (with 0 it stays FP64 throughout, which is never
     // less accurate; only the speed differs from class to class).  The
@@ -131,16 +166,16 @@ struct GtfSystem {
         int unit_pq = GTF_UNIT_PQ;
         int tile_pq = GTF_TILE_PQ;
         int grid = 2048;
-        int boys_lds = 0;
+        int boys_lds = 1;
         int fp32 = 1;
     };
     TileShape shape[GTF_NCLASSES];
     // classes run by the bra/ket-exchanged tile kernel (bit = class index;
-    // only classes that have one).  Default: the two classes where it was
-    // measured faster on MI355X, (pp|ps) and (dp|ps); in the others the large
-    // pair's coefficients move into the inner primitive loop and the kernel
-    // loses more than the shared Boys/R work saves.
-    unsigned exchanged_mask = (1u << 4) | (1u << 11);
+    // only classes that have one).  Default: the classes where it is faster on
+    // MI355X, because it needs fewer threads per quartet and so forms R less
+    // often.
+    unsigned exchanged_mask = (1u << 4) | (1u << 12) | (1u << 13) | (1u << 16) | (1u << 17) |
+                              (1u << 18) | (1u << 19);
     bool exchanged(int cls) const;
     // mixed precision: Schwarz bound threshold tau (0 = plain FP64)
     double tau = 0.0;
@@ -197,8 +232,9 @@ struct GtfSystem {
     // of one class
     int build_tiles();
     int build_class_tiles(int cls);
-    void cut_class_tiles(int cls, std::vector<int4>& hv, std::vector<int4>& lv);
-    int upload_class_tiles(int cls, const std::vector<int4>& hv, const std::vector<int4>& lv);
+    void cut_class_tiles(int cls, TileList& hv, TileList& lv);
+    int upload_tiles(const TileList* hv, const TileList* lv, int c0, int c1);
+    void* tile_mem[GTF_NCLASSES] = {nullptr};  // the allocation that holds a class's tiles
     // CSR of molecule 0 in the reference layout (host)
     void csr(std::vector<int>& shellptr, std::vector<int>& shellid, std::vector<int>& shellrid,
              std::vector<double>& shellvalue) const;
@@ -212,7 +248,7 @@ struct GtfSystem {
     }
     PairView pair_view() const;
     // fused ERI + J/K digestion over all screened quartets of every class;
-    // D, J, K are the packed blocks of all molecules
+    // D, J, K are the packed blocks of all molecules, J and K cleared first
     // nd densities (and J, K) dstride elements apart, digested from each
     // integral; nd > 1 needs fits_densities(nd) (LDS work areas per density)
     int jk(const double* D, double* J, double* K, int nd = 1, long dstride = 0);

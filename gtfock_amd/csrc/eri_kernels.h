@@ -31,7 +31,7 @@ struct EriArgs {
     int ntasks;
     PairView pv;
     const int* fstart;
-    const double* boys8;  // compact Taylor tables, BOYS8_NM slabs of BOYS8_SLAB
+    const double* boys8;  // compact Taylor tables, BOYS8_NM slabs of BOYS8_SLAB, exp(-T0)
     // EPI_JK: nd densities (and their J, K) dstride elements apart, all
     // digested from each integral (pfock/fock_task.c:46 loops num_dmat)
     const double* D;
@@ -43,8 +43,15 @@ struct EriArgs {
     unsigned long long* vbits;
     // EPI_STORE
     double* out;
-    // bra-row tiles of the LDS-strip J/K kernel: (bra row, first ket, end ket)
-    const int4* tiles;
+    // tiles of the LDS-strip J/K kernel and their runs of kets (gtf_internal.h)
+    const TileHead* tiles;
+    const int4* runs;
+    // per density and ket component, by position in the ket list: the density
+    // elements of the kets, and the accumulators of their J_PQ (JkList)
+    const double* dk;
+    double* jk;
+    long nket;  // list length
+    KetView kv;  // the ket list, for the tile kernels
     int ntiles;
     int nbf;  // LDS strip capacity (largest molecule)
     // exact screening of the block-padded rows
@@ -108,11 +115,9 @@ __device__ __forceinline__ int find_row(const long* __restrict__ off, int nrows,
     return lo;
 }
 
-template <int LA, int LB, int LC, int LD, int NC, bool STRIP>
+template <int LA, int LB, int LC, int LD, int NC>
 __device__ __forceinline__ void digest(const EriArgs& a, int bra, int ket, int c0,
-                                       const double (&acc)[NC][EriShape<LA, LB, LC, LD>::NCD], double* jmn,
-                                       double* strip, int nbf, double* jpq, double* jmn_reg = nullptr,
-                                       long doff = 0);
+                                       const double (&acc)[NC][EriShape<LA, LB, LC, LD>::NCD], long doff);
 
 template <int LA, int LB, int LC, int LD, int NC, int EPI>
 __device__ __forceinline__ void eri_unit(const EriArgs& a, long u)
@@ -162,27 +167,19 @@ __device__ __forceinline__ void eri_unit(const EriArgs& a, long u)
         atomicMax(a.vbits + bra, (unsigned long long)__double_as_longlong(mx));
     } else {
         for (int d = 0; d < a.nd; d++)
-            digest<LA, LB, LC, LD, NC, false>(a, bra, ket, c0, acc, nullptr, nullptr, 0, nullptr, nullptr,
-                                              d * a.dstride);
+            digest<LA, LB, LC, LD, NC>(a, bra, ket, c0, acc, d * a.dstride);
     }
 }
 
-// update_F digestion of one thread's NC bra components of quartet (bra|ket).
-// STRIP = false: FP64 atomics straight into J and K.
-// STRIP = true:  the bra-side blocks (J_MN and the exchange blocks K_MP, K_NP,
-// K_MQ, K_NQ, which all lie in the rows of shells M and N) go to LDS
-// (jmn[NA*NB], strip[(NA+NB) * nbf], row r < NA is function fM + r, row
-// NA + r is fN + r); J_PQ goes to the ket's LDS row jpq[NCD] when one is
-// given (the threads sharing a quartet then meet in LDS), else to HBM.  With
-// jmn_reg (a thread that owns all bra components of its quartets) J_MN is
-// summed in those registers and added to LDS once per tile.
-template <int LA, int LB, int LC, int LD, int NC, bool STRIP>
+// update_F digestion of one thread's NC bra components of quartet (bra|ket)
+// by FP64 atomics straight into J and K (the classes whose LDS strips do not
+// fit).
+template <int LA, int LB, int LC, int LD, int NC>
 __device__ __forceinline__ void digest(const EriArgs& a, int bra, int ket, int c0,
-                                       const double (&acc)[NC][EriShape<LA, LB, LC, LD>::NCD], double* jmn,
-                                       double* strip, int nbf, double* jpq, double* jmn_reg, long doff)
+                                       const double (&acc)[NC][EriShape<LA, LB, LC, LD>::NCD], long doff)
 {
     using S = EriShape<LA, LB, LC, LD>;
-    constexpr int NCD = S::NCD, ND = S::ND, NB = S::NB, NA = S::NA;
+    constexpr int NCD = S::NCD, ND = S::ND, NB = S::NB;
     const int M = a.pv.s1[bra], N = a.pv.s2[bra], P = a.pv.s1[ket], Q = a.pv.s2[ket];
     const int f1 = (M != N), f2 = (P != Q), f3 = (bra != ket);
     const double cJ1 = 2.0 * (1 + f1) * (1 + f2);
@@ -211,12 +208,7 @@ __device__ __forceinline__ void digest(const EriArgs& a, int bra, int ket, int c
             constexpr int cd = decltype(d_)::value;
             s += D[(long)(oP + cd / ND) * ld + oQ + cd % ND] * acc[c][cd];
         });
-        if constexpr (STRIP) {
-            if (jmn_reg) jmn_reg[c] += cJ1 * s;
-            else atomicAdd(&jmn[mloc[c] * NB + nloc[c]], cJ1 * s);
-        } else {
-            GTF_ATOMIC_ADD(&J[(long)(oM + mloc[c]) * ld + oN + nloc[c]], cJ1 * s);
-        }
+        GTF_ATOMIC_ADD(&J[(long)(oM + mloc[c]) * ld + oN + nloc[c]], cJ1 * s);
     });
     if (f3) {
         static_for<0, NCD>([&](auto d_) {
@@ -226,11 +218,7 @@ __device__ __forceinline__ void digest(const EriArgs& a, int bra, int ket, int c
                 constexpr int c = decltype(c_)::value;
                 s += dmn[c] * acc[c][cd];
             });
-            if (jpq) {
-                atomicAdd(&jpq[cd], cJ2 * s);
-            } else {
-                GTF_ATOMIC_ADD(&J[(long)(oP + cd / ND) * ld + oQ + cd % ND], cJ2 * s);
-            }
+            GTF_ATOMIC_ADD(&J[(long)(oP + cd / ND) * ld + oQ + cd % ND], cJ2 * s);
         });
     }
     // K_MP -= cMP sum_q D_nq I,  K_NP -= cNP sum_q D_mq I
@@ -238,8 +226,6 @@ __device__ __forceinline__ void digest(const EriArgs& a, int bra, int ket, int c
     static_for<0, NC>([&](auto c_) {
         constexpr int c = decltype(c_)::value;
         const long rm = (long)(oM + mloc[c]) * ld, rn = (long)(oN + nloc[c]) * ld;
-        double* km = STRIP ? strip + (long)mloc[c] * nbf : K + rm;
-        double* kn = STRIP ? strip + (long)(NA + nloc[c]) * nbf : K + rn;
         static_for<0, S::NCc>([&](auto p_) {
             constexpr int p = decltype(p_)::value;
             double smp = 0.0, snp = 0.0;
@@ -249,13 +235,8 @@ __device__ __forceinline__ void digest(const EriArgs& a, int bra, int ket, int c
                 smp += D[rn + oQ + qq] * x;
                 snp += D[rm + oQ + qq] * x;
             });
-            if constexpr (STRIP) {
-                atomicAdd(&km[oP + p], -cMP * smp);
-                if (f1) atomicAdd(&kn[oP + p], -cNP * snp);
-            } else {
-                GTF_ATOMIC_ADD(&km[oP + p], -cMP * smp);
-                if (f1) GTF_ATOMIC_ADD(&kn[oP + p], -cNP * snp);
-            }
+            GTF_ATOMIC_ADD(&K[rm + oP + p], -cMP * smp);
+            if (f1) GTF_ATOMIC_ADD(&K[rn + oP + p], -cNP * snp);
         });
         if (f2) {
             static_for<0, ND>([&](auto q_) {
@@ -267,13 +248,8 @@ __device__ __forceinline__ void digest(const EriArgs& a, int bra, int ket, int c
                     smq += D[rn + oP + p] * x;
                     snq += D[rm + oP + p] * x;
                 });
-                if constexpr (STRIP) {
-                    atomicAdd(&km[oQ + qq], -cMQ * smq);
-                    if (f1) atomicAdd(&kn[oQ + qq], -cNQ * snq);
-                } else {
-                    GTF_ATOMIC_ADD(&km[oQ + qq], -cMQ * smq);
-                    if (f1) GTF_ATOMIC_ADD(&kn[oQ + qq], -cNQ * snq);
-                }
+                GTF_ATOMIC_ADD(&K[rm + oQ + qq], -cMQ * smq);
+                if (f1) GTF_ATOMIC_ADD(&K[rn + oQ + qq], -cNQ * snq);
             });
         }
     });
@@ -299,43 +275,60 @@ __global__ __launch_bounds__(256) void eri_kernel(EriArgs a)
     }
 }
 
-// Fused ERI + J/K digestion over bra-row tiles.  A tile is a bounded number
-// of work units of one bra row; the workgroup accumulates J_MN and
-// the exchange blocks of the bra shells in LDS and flushes them with one HBM
-// atomic per touched element when the tile is done.  The J_PQ block of
-// every ket of the tile is also kept in LDS and flushed at the end, so no
-// HBM atomic (whose completion the next loads would wait for) sits in the
-// quartet loop.  Dynamic LDS: GTF_BOYS_LDS (the Boys slab, BLDS only) +
-// (NA + NB) * nbf + NA * NB + kmax * NCD doubles, nbf = the largest molecule's size, kmax =
-// the most kets a tile of the class may hold (units per tile / NSPLIT).
+// Fused ERI + J/K digestion over bra-row tiles.  A workgroup takes a tile --
+// one bra pair and runs of its kets -- and accumulates J_MN and the exchange
+// blocks of the bra shells in LDS, flushed with one HBM atomic per touched
+// element when the tile is done.  The flush was half of the (ps|ps) kernel on
+// C54H18 when a tile held at most 320 kets (21.7 ms, 13.1 without digestion),
+// so a tile takes as much of its bra's row as the balance allows.  Dynamic
+// LDS: the Boys slab (BLDS only) + per density tile_work() doubles, and with
+// BLDS the density rows, (NA + NB) * nbf.
 //
-// A tile is (bra row, first ket, end ket, nic): each of its quartets is split
-// into nic bra-primitive chunks (sizes differing by at most one) times NSPLIT
-// bra-component chunks, so
-// that a unit holds about unit_pq primitive quartets however contracted
-// the pairs are, and a tile holds at most `units` units and about tile_pq
-// primitive quartets (per class, chosen on the host; the defaults below).
-// Digestion is linear in the integrals, so every unit digests its partial
-// sum on its own.
+// The tile's work is cut into wavefront units: 64 lanes over (ket, ket
+// primitive class), one chunk of the ket primitives, one chunk of the split
+// side's components.  The bra pair and the component chunk are the same for
+// all lanes of a unit; the kets are consecutive in their list.  2^lic chunks
+// of the ket primitives (primitives ic, ic + 2^lic, ...: the primitives are
+// ordered by their bound, so an interleaved chunk holds its share of the ones
+// that screening drops) keep a unit near unit_pq primitive quartets per lane;
+// chunks of the ket's rather than the bra's primitives, so that a ket record
+// is read by one unit only.  Where a run has few kets, 2^ljc lanes share a ket
+// and take every 2^ljc-th of the chunk; they add their integrals with lane
+// shuffles and the first one digests.  Digestion is linear in the integrals,
+// so every unit digests its partial sum on its own.
+//
+// A wavefront takes all units of a run's 64 kets one after another, from a
+// counter in LDS (their costs differ; dealt in turn, the wavefronts waited
+// for the slowest at the tile's end).  It sums J_PQ of those kets in a buffer
+// of its own and adds it to the list's accumulators with one coalesced atomic
+// per component: scattered into the matrix it was 64 cache lines each.
 #define GTF_TILE_UNITS 1024
 #define GTF_UNIT_PQ 64
-#define GTF_TILE_PQ 65536
+#define GTF_TILE_PQ 1048576
+// J_MN is the same few addresses for every lane of a unit: 16 copies, picked
+// by lane, leave 4 lanes to an address (64 lanes adding to one are served
+// one after another)
+#define GTF_JMN_COPIES 16
 
 // The Boys Taylor slab of order L copied from HBM into the first
-// GTF_BOYS_LDS doubles of dynamic LDS.  A persistent workgroup copies it
-// once; every primitive quartet of every tile it takes then reads its Taylor
-// row from LDS instead of a dependent global load.  The barrier that follows
-// each tile's clearing of its LDS work area orders the copy before the first
-// read.  It costs 23 KB of LDS per workgroup, which lowers the occupancy of
-// classes whose strips are already large, so it is a per-class choice (the
-// tile shape's boys_lds).  FP32 tiles use the same FP64 slab: the Boys
-// function is FP64 in both precisions.
-#define GTF_BOYS_LDS BOYS8_SLAB
+// GTF_BOYS_LDS doubles of dynamic LDS, as columns (boys_eval8).  A persistent
+// workgroup copies it once; every primitive quartet of every tile it takes
+// then reads its Taylor row from LDS instead of from up to 64 lines per load.
+// The barrier before the first tile orders the copy before the first
+// read.  It costs 26 KB of LDS per workgroup, which
+// lowers the occupancy of classes whose strips are already large, so it is a
+// per-class choice (the tile shape's boys_lds).  FP32 tiles use the same FP64
+// slab: the Boys function is FP64 in both precisions.
+#define GTF_BOYS_LDS (BOYS8_SLAB + BOYS8_EXP)
 template <int L>
 __device__ __forceinline__ const double* boys_to_lds(const EriArgs& a, double* smem)
 {
-    const double* src = a.boys8 + L * BOYS8_SLAB;
-    for (int k = threadIdx.x; k < BOYS8_SLAB; k += 256) smem[k] = src[k];
+    const double2* src = reinterpret_cast<const double2*>(a.boys8 + L * BOYS8_SLAB);
+    double2* dst = reinterpret_cast<double2*>(smem);
+    constexpr int C = BOYS8_NTERM / 2;
+    for (int k = threadIdx.x; k < BOYS8_SLAB / 2; k += blockDim.x) dst[(k % C) * BOYS8_NGRID + k / C] = src[k];
+    const double2* ex = reinterpret_cast<const double2*>(a.boys8 + BOYS8_NM * BOYS8_SLAB);
+    for (int k = threadIdx.x; k < BOYS8_EXP / 2; k += blockDim.x) dst[BOYS8_SLAB / 2 + k] = ex[k];
     return smem;
 }
 
@@ -354,355 +347,480 @@ __device__ __forceinline__ const double* tile_boys(const EriArgs& a, double* sme
     }
 }
 
-// Minimum waves per SIMD asked of the compiler for a class's tile kernel.
-// (ps|ss) in FP64 takes 152 VGPRs (3 waves) when left alone and fits 127
-// with none spilled at 4, 8 % faster on MI355X; the same cap makes (pp|ss)
-// and (pp|pp) spill and run 2.5x slower, so the others are left alone.
-template <int LA, int LB, int LC, int LD>
-constexpr int tile_min_waves()
+// f(std::integral_constant<int, s>) for the run-time s in [0, N)
+template <int N, int S = 0, typename F>
+__device__ __forceinline__ void split_switch(int s, F&& f)
 {
-    return (LA == 1 && LB == 0 && LC == 0 && LD == 0) ? 4 : 1;
+    if constexpr (S + 1 == N) {
+        f(std::integral_constant<int, S>{});
+    } else {
+        if (s == S) f(std::integral_constant<int, S>{});
+        else split_switch<N, S + 1>(s, f);
+    }
 }
 
-template <int LA, int LB, int LC, int LD, int NC, typename Real, bool BLDS>
-__global__ __launch_bounds__(256, (tile_min_waves<LA, LB, LC, LD>())) void eri_jk_tile_kernel(EriArgs a)
+// what a unit's digestion reads and writes
+struct DigestCtx {
+    const_as<double>* Dm;  // rows of shell M, uniform reads (D_mn)
+    const double *rm, *rn;  // D rows of shells M and N
+    int ld, oN, oP, oQ;
+    int f1, f2, f3;
+    double* strip;          // LDS: row r < NA is function M + r, row NA + r is N + r
+    int nbf;
+    double* jmn;            // LDS: this lane's copy of J_MN
+    const double* dk;       // the ket's density elements, a component every nk
+    long nk;
+    double* jpq;            // LDS: the ket's J_PQ, a component every 64; null: in jk
+    double* jk;             // the list's J_PQ, a component every nk
+};
+
+// update_F digestion (pfock/fock_task.c:29-117) of bra components A0 .. A0 +
+// NAr - 1 and ket components C0 .. C0 + NCr - 1 of a lane's quartet; get(ab,
+// cd) reads an integral.  With jreg (the thread owns every bra component of
+// its quartets) J_MN is summed there over the tile.  Contributions to the
+// same element of the strip are summed over the thread's components first.
+// crt: the run-time component of a kernel that has one bra component (A0 < 0)
+// or one ket component (C0 < 0) per thread.
+template <int LA, int LB, int LC, int LD, int A0, int NAr, int C0, int NCr, bool JREG, typename Get>
+__device__ __forceinline__ void digest_unit(const DigestCtx& x, int crt, Get&& get, double* jreg)
 {
     using S = EriShape<LA, LB, LC, LD>;
-    constexpr int NSPLIT = S::NAB / NC;
-    constexpr int NA = S::NA, NB = S::NB, NCD = S::NCD;
-    constexpr bool LOW = std::is_same<Real, float>::value;
-    constexpr bool JPQ_LDS = true;
+    constexpr int NA = S::NA, NB = S::NB, ND = S::ND;
+    constexpr bool RT = A0 < 0, KRT = C0 < 0;
+    constexpr int AB0 = RT ? 0 : A0, CD0 = KRT ? 0 : C0;
+    constexpr int M0 = AB0 / NB, M1 = (AB0 + NAr - 1) / NB + 1;
+    constexpr int P0 = KRT ? 0 : CD0 / ND, P1 = KRT ? 1 : (CD0 + NCr - 1) / ND + 1, QN = KRT ? 1 : ND;
+    const int mrt = RT ? crt / NB : 0, nrt = RT ? crt - mrt * NB : 0;
+    const int prt = KRT ? crt / ND : 0, qrt = KRT ? crt - prt * ND : 0;
+    const int oP = x.oP + prt, oQ = x.oQ + qrt;  // of the run-time ket component, else of the shells
+    const double cJ1 = 2.0 * (1 + x.f1) * (1 + x.f2);
+    const double cJ2 = 2.0 * x.f3 * (1 + x.f1) * (1 + x.f2);
+    // J_MN += cJ1 sum_pq D_pq I,  J_PQ += cJ2 sum_mn D_mn I
+    {
+        double dpq[NCr];
+        static_for<0, NCr>([&](auto d_) GTF_INLINE {
+            constexpr int cd = CD0 + decltype(d_)::value;
+            dpq[decltype(d_)::value] = x.dk[((KRT ? crt : 0) + cd) * x.nk];
+        });
+        static_for<0, NAr>([&](auto c_) GTF_INLINE {
+            constexpr int c = decltype(c_)::value;
+            double s = 0.0;
+            static_for<0, NCr>([&](auto d_) GTF_INLINE { s += dpq[decltype(d_)::value] * get(c_, d_); });
+            if constexpr (JREG) jreg[c] += cJ1 * s;
+            else atomicAdd(&x.jmn[RT ? crt : AB0 + c], cJ1 * s);
+        });
+    }
+    if (x.f3) {
+        double dmn[NAr];
+        static_for<0, NAr>([&](auto c_) GTF_INLINE {
+            constexpr int c = decltype(c_)::value;
+            const int m = RT ? mrt : (AB0 + c) / NB, n = RT ? nrt : (AB0 + c) % NB;
+            dmn[c] = x.Dm[(long)m * x.ld + x.oN + n];
+        });
+        static_for<0, NCr>([&](auto d_) GTF_INLINE {
+            double s = 0.0;
+            static_for<0, NAr>([&](auto c_) GTF_INLINE { s += dmn[decltype(c_)::value] * get(c_, d_); });
+            const int cd = (KRT ? crt : CD0) + decltype(d_)::value;
+            if (x.jpq) x.jpq[cd * 64] += cJ2 * s;
+            else GTF_ATOMIC_ADD(&x.jk[cd * x.nk], cJ2 * s);
+        });
+    }
+    // K_MP -= cMP sum_nq D_nq I,  K_MQ -= cMQ sum_np D_np I  for each m, and
+    // K_NP -= cNP sum_mq D_mq I,  K_NQ -= cNQ sum_mp D_mp I  for each n
+    const double c3 = -(double)(1 + x.f3);
+    auto bra_side = [&](auto side_) GTF_INLINE {
+        constexpr bool ROWM = decltype(side_)::value == 0;  // rows of M, sums over n
+        constexpr int R0 = RT ? 0 : ROWM ? M0 : 0, R1 = RT ? 1 : ROWM ? M1 : NB;
+        static_for<R0, R1>([&](auto r_) GTF_INLINE {
+            constexpr int r = decltype(r_)::value;
+            constexpr int O0 = RT ? 0 : ROWM ? 0 : M0, O1 = RT ? 1 : ROWM ? NB : M1;
+            auto in_chunk = [](int o) {
+                const int ab = ROWM ? r * NB + o : o * NB + r;
+                return RT || (ab >= AB0 && ab < AB0 + NAr);
+            };
+            constexpr bool any = [&]() GTF_INLINE {
+                for (int o = O0; o < O1; o++)
+                    if (in_chunk(o)) return true;
+                return false;
+            }();
+            if constexpr (any) {
+                const int row = RT ? (ROWM ? mrt : NA + nrt) : (ROWM ? r : NA + r);
+                double* out = x.strip + row * x.nbf;
+                double sp[P1 - P0], sq[QN];
+                static_for<0, P1 - P0>([&](auto p_) GTF_INLINE { sp[decltype(p_)::value] = 0.0; });
+                static_for<0, QN>([&](auto q_) GTF_INLINE { sq[decltype(q_)::value] = 0.0; });
+                static_for<O0, O1>([&](auto o_) GTF_INLINE {
+                    constexpr int o = decltype(o_)::value;
+                    constexpr int ab = ROWM ? r * NB + o : o * NB + r;
+                    if constexpr (RT || (ab >= AB0 && ab < AB0 + NAr)) {
+                        const double* dr = ROWM ? x.rn + (long)(RT ? nrt : o) * x.ld : x.rm + (long)(RT ? mrt : o) * x.ld;
+                        using C = std::integral_constant<int, RT ? 0 : ab - AB0>;
+                        static_for<P0, P1>([&](auto p_) GTF_INLINE {
+                            constexpr int p = decltype(p_)::value;
+                            const double dp = dr[oP + p];
+                            static_for<0, QN>([&](auto q_) GTF_INLINE {
+                                constexpr int q = decltype(q_)::value;
+                                constexpr int cd = p * ND + q;
+                                if constexpr (cd >= CD0 && cd < CD0 + NCr) {
+                                    const double v = get(C{}, std::integral_constant<int, cd - CD0>{});
+                                    sp[p - P0] += dr[oQ + q] * v;
+                                    sq[q] += dp * v;
+                                }
+                            });
+                        });
+                    }
+                });
+                static_for<P0, P1>([&](auto p_) GTF_INLINE {
+                    constexpr int p = decltype(p_)::value;
+                    atomicAdd(&out[oP + p], c3 * sp[p - P0]);
+                });
+                if (x.f2)
+                    static_for<0, QN>([&](auto q_) GTF_INLINE {
+                        constexpr int q = decltype(q_)::value;
+                        constexpr bool has = [&]() GTF_INLINE {
+                            for (int p = P0; p < P1; p++)
+                                if (p * ND + q >= CD0 && p * ND + q < CD0 + NCr) return true;
+                            return false;
+                        }();
+                        if constexpr (has) atomicAdd(&out[oQ + q], c3 * sq[q]);
+                    });
+            }
+        });
+    };
+    bra_side(std::integral_constant<int, 0>{});
+    if (x.f1) bra_side(std::integral_constant<int, 1>{});
+}
+
+// Largest workgroup of a class's tile kernel (the host takes it or 256, see
+// GtfSystem::tile_threads).  A kernel compiled for 512 threads has at most 256
+// VGPRs; the classes of L >= 5 need more, run one wavefront per SIMD and take
+// 256 threads.
+template <int LA, int LB, int LC, int LD>
+__host__ __device__ constexpr int tile_threads()
+{
+    return LA + LB + LC + LD <= 4 ? 512 : 256;
+}
+
+// Wavefronts per SIMD asked of the compiler.  Left alone it keeps addresses of
+// the digestion in registers across the primitive loops.
+template <int LA, int LB, int LC, int LD>
+__host__ __device__ constexpr int tile_min_waves()
+{
     constexpr int L = LA + LB + LC + LD;
-    constexpr int ND = S::ND;
-    extern __shared__ double smem[];
-    __shared__ int s_task;
+    return L <= 1 ? 4 : L == 2 ? 3 : L <= 4 ? 2 : 1;
+}
+
+// LDS doubles of one density's work area: the strips, the J_MN copies and, for
+// a single density, the wavefronts' J_PQ buffers (several densities add J_PQ
+// straight to the accumulators: the buffers would not fit for the d classes)
+__host__ __device__ constexpr int tile_work(int rows, int nbf, int nab, int ncd, int waves)
+{
+    return rows * nbf + GTF_JMN_COPIES * nab + waves * ncd * 64;
+}
+
+// One class's tile kernel.  EX = false: a thread owns NC bra components and
+// every ket component of its quartet; EX = true: NC ket components and every
+// bra component, the ket contracted first.
+template <int LA, int LB, int LC, int LD, int NC, typename Real, bool BLDS, bool EX>
+__device__ __forceinline__ void tile_kernel_body(const EriArgs& a)
+{
+    using S = EriShape<LA, LB, LC, LD>;
+    constexpr int NA = S::NA, NB = S::NB, NCD = S::NCD, NAB = S::NAB, ND = S::ND;
+    constexpr int SIDE = EX ? NCD : NAB;
+    constexpr int NSPLIT = (SIDE + NC - 1) / NC;
+    constexpr bool LOW = std::is_same<Real, float>::value;
+    constexpr int L = S::L;
+    constexpr int KREC = KetView::rec(NzTab<LC, LD>::data.nnz);
+    // compile-time component chunks, or (one component of very many) run-time
+    constexpr bool STATIC = tile_static(SIDE, NC);
+    constexpr bool JREG_ABLE = NSPLIT == 1 && NAB <= 3;
+    extern __shared__ __attribute__((aligned(16))) double smem[];
+    __shared__ int s_task, s_unit;
+    const int NT = blockDim.x;
     double* work;
     const double* boys = tile_boys<L, BLDS>(a, smem, work);
+    // the bra shells' density rows beside the work areas (BLDS): the digestion
+    // gathers from them at the kets' columns
+    const bool buffered = a.nd == 1;
+    const int wsz = tile_work(NA + NB, a.nbf, NAB, NCD, buffered ? NT / 64 : 0);
+    double* drow = work + (long)a.nd * wsz;
     const long long t_begin = (long long)wall_clock64();
+    const int lane = threadIdx.x & 63;
     int taken = 0;
-    for (;;) {
-        if (threadIdx.x == 0) s_task = atomicAdd(a.counter, 1);
-        __syncthreads();
-        const int task = s_task;
-        if (task >= a.ntiles) break;
-        taken++;
-        const int4 t = a.tiles[task];
-        const int bra = a.bra_list[t.x];
-        if (!bra_active(a, bra)) {
-            __syncthreads();  // every thread has read s_task before it is rewritten
-            continue;
-        }
-        const int nbp = a.pv.nprim[bra];
-        const int nic = t.w;  // bra-primitive chunks per quartet
+    // the current tile, wave-uniform
+    int run0, nrun, bra, oM, oN, f1, nbf, rb;
+    long mat;
+    double vb;
+    BraRef<Real> br;
+    br.peps = a.pv.peps;
+    // reads tile `task` (and its density rows); false when there is none
+    auto open_tile = [&](int task) GTF_INLINE {
+        if (task >= a.ntiles) return false;
+        const_as<TileHead>& h = *as_const(a.tiles + task);
+        run0 = h.run0;
+        // a molecule that takes no part in this build (mol_active is written
+        // between builds only)
+        nrun = !a.mol_active || as_const(a.mol_active)[h.mol] ? h.nrun : 0;
+        bra = h.bra;
         // strip rows are as wide as the bra's molecule (at most a.nbf)
-        const int nbf = a.mld[a.pv.s1[bra]];
+        nbf = h.nbf;
+        mat = h.mat;
+        oM = h.oM;
+        oN = h.oN;
+        f1 = h.two;
+        rb = h.rank;
+        vb = as_const(a.vbra)[h.row];
+        br.n = h.nprim;
+        br.prim = as_const((const double*)(a.pv.prim + h.prim));
+        br.q = as_const(a.pv.q + h.prim);
+        if constexpr (LOW) br.E = as_const(STATIC || EX ? a.pv.Ezf : a.pv.Ef) + h.E;
+        else br.E = as_const(STATIC || EX ? a.pv.Ez : a.pv.E) + h.E;
+        if constexpr (BLDS)
+            for (int d = 0; d < a.nd; d++) {
+                const double* D = a.D + d * a.dstride + mat;
+                for (int r = 0; r < NA + NB; r++) {
+                    const double* Dr = D + (long)(r < NA ? oM + r : oN + (r - NA)) * nbf;
+                    for (int k = threadIdx.x; k < nbf; k += NT) drow[(d * (NA + NB) + r) * nbf + k] = Dr[k];
+                }
+            }
+        return true;
+    };
+    if (threadIdx.x == 0) {
+        s_task = atomicAdd(a.counter, 1);
+        s_unit = 0;
+    }
+    // the work areas are zero whenever a tile starts: here, and the flush
+    // clears what it read
+    for (int k = threadIdx.x; k < a.nd * wsz; k += NT) work[k] = 0.0;
+    __syncthreads();
+    bool open = open_tile(__builtin_amdgcn_readfirstlane(s_task));
+    __syncthreads();
+    while (open) {
+        int next = 0;  // taken now, needed at the end
+        if (threadIdx.x == 0) next = atomicAdd(a.counter, 1);
+        taken++;
         const int nstrip = (NA + NB) * nbf;
         double* strip = work;
         double* jmn = work + nstrip;
-        double* jpq = jmn + NA * NB;
-        const int njpq = JPQ_LDS ? (t.z - t.y) * NCD : 0;
-        // one work area (strip, J_MN, J_PQ) per density
-        const int wsz = nstrip + NA * NB + njpq;
-        for (int k = threadIdx.x; k < a.nd * wsz; k += 256) work[k] = 0.0;
-        __syncthreads();
-        // Unit order.  NSPLIT == 1: the nic chunks of one quartet sit in
-        // neighbouring lanes (nic is a power of two, so a group never spans
-        // two wavefronts); the group adds its partial integrals with lane
-        // shuffles and its first lane digests the sum.  NSPLIT > 1: component
-        // chunk fastest, then ket, then bra-primitive chunk, so neighbouring
-        // lanes digest into different ket columns.
-        const int nkt = t.z - t.y;
-        const int nunits = nkt * nic * NSPLIT;
-        double jreg[NC];
-        static_for<0, NC>([&](auto c_) { jreg[decltype(c_)::value] = 0.0; });
-        for (int u = threadIdx.x; u < nunits; u += 256) {
-            int q, ic, c0;
-            if constexpr (NSPLIT == 1) {
-                q = u / nic;
-                ic = u - q * nic;
-                c0 = 0;
-            } else {
-                const int rest = u / NSPLIT;
-                c0 = (u - rest * NSPLIT) * NC;
-                ic = rest / nkt;
-                q = rest - ic * nkt;
+        double* jpq = jmn + GTF_JMN_COPIES * NAB + (threadIdx.x >> 6) * (NCD * 64);
+        const bool jreg_on = JREG_ABLE && a.nd == 1;
+        double jreg[JREG_ABLE ? NAB : 1];
+        if constexpr (JREG_ABLE) static_for<0, NAB>([&](auto c_) { jreg[decltype(c_)::value] = 0.0; });
+        // cursor: block `at` of the tile is block `blk` of run `r`
+        int r = -1, left = 0, kbeg = 0, nkt = 0, lic = 0, ljc = 0, sp0 = 0, spn = 1, ic0 = 0, icn = 1;
+        int blk = 0, at = -1;
+        auto take = [&]() GTF_INLINE {
+            int u = 0;
+            if (lane == 0) u = atomicAdd(&s_unit, 1);
+            return __builtin_amdgcn_readfirstlane(u);
+        };
+        auto seek = [&](int unit) GTF_INLINE {
+            int d = unit - at;  // >= 1
+            at = unit;
+            while (d > left) {  // into the next run (left: blocks after the current one)
+                d -= left + 1;
+                if (++r >= nrun) return false;
+                const_as<int>* rp = as_const((const int*)(a.runs + run0 + r));
+                kbeg = rp[0];
+                const int span = rp[1], chunks = rp[2];
+                nkt = GTF_RUN_KETS(span), sp0 = GTF_RUN_SP0(span), spn = GTF_RUN_SPN(span);
+                lic = GTF_RUN_LIC(chunks), ljc = GTF_RUN_LJC(chunks);
+                ic0 = GTF_RUN_IC0(chunks), icn = GTF_RUN_ICN(chunks);
+                left = (((nkt << ljc) + 63) >> 6) - 1;
+                blk = 0;
             }
-            const int i0 = ic * nbp / nic, i1 = (ic + 1) * nbp / nic;
-            const int j = t.y + q;
-            if (!quartet_valid(a, t.x, j)) continue;
-            // precision split on the Schwarz bound sqrt(v_bra v_ket) vs tau
-            if ((a.vbra[t.x] * a.vket[j] >= a.tau2) == LOW) continue;
-            const int ket = a.ket_list[j];
-            double acc[NC][NCD];
-            if constexpr (LOW) {
-                float accf[NC][NCD];
-                eri_block<LA, LB, LC, LD, NC, float>(a.pv, bra, ket, c0, boys, accf, i0, i1);
-                static_for<0, NC>([&](auto c_) {
-                    static_for<0, NCD>([&](auto d_) {
-                        acc[decltype(c_)::value][decltype(d_)::value] = (double)accf[decltype(c_)::value][decltype(d_)::value];
+            left -= d;
+            blk += d;
+            return true;
+        };
+        for (int unit = take(); seek(unit);) {
+            unit = take();
+            const int u = blk * 64 + lane;
+            const int q = u >> ljc, jc = u & ((1 << ljc) - 1);
+            const int j = kbeg + q;
+            bool on = q < nkt;
+            if (on) {
+                const double vk = a.vket[j];
+                // the Schwarz test of pfock/fock_task.c:192, the one-orientation
+                // rule of a diagonal class, and the precision split on the
+                // bound sqrt(v_bra v_ket) against tau
+                on = vb * vk >= a.tol2 && (!a.same || a.rank_ket[j] <= rb) && (vb * vk >= a.tau2) != LOW;
+            }
+            if (__ballot(on) == 0) continue;
+            KetRef kr{a.kv.d, a.kv.q, 0};
+            int4 ki = make_int4(0, 0, 0, -1);
+            int kb = 0;
+            if (on) {
+                kb = a.kv.base[j];
+                ki = a.kv.info[j];
+                kr.d = a.kv.d + (long)(kb >> 6) * (KREC * 64) + (kb & 63);
+                kr.q = a.kv.q + kb;
+                kr.n = a.kv.nprim[j];
+            }
+            const int js = 1 << (lic + ljc);
+            auto finish = [&](auto a0_, auto nar_, auto c0_, auto ncr_, auto& acc, int crt) GTF_INLINE {
+                constexpr int A0 = decltype(a0_)::value, NAr = decltype(nar_)::value;
+                constexpr int C0 = decltype(c0_)::value, NCr = decltype(ncr_)::value;
+                // acc is [NAr][NCr], or [NCr][NAr] in the exchanged form
+                auto cell = [&](auto c_, auto d_) GTF_INLINE -> Real& {
+                    constexpr int c = decltype(c_)::value, d = decltype(d_)::value;
+                    if constexpr (EX) return acc[d][c];
+                    else return acc[c][d];
+                };
+                for (int s = 1; s < (1 << ljc); s <<= 1)
+                    static_for<0, NAr>([&](auto c_) GTF_INLINE {
+                        static_for<0, NCr>([&](auto d_) GTF_INLINE { cell(c_, d_) += __shfl_xor(cell(c_, d_), s, 64); });
                     });
-                });
-            } else {
-                eri_block<LA, LB, LC, LD, NC, double>(a.pv, bra, ket, c0, boys, acc, i0, i1);
-            }
-            if constexpr (NSPLIT == 1) {
-                // sum the group's partial integrals into its first lane
-                for (int w = 1; w < nic; w <<= 1)
-                    static_for<0, NC>([&](auto c_) {
-                        static_for<0, NCD>([&](auto d_) {
-                            constexpr int c = decltype(c_)::value, cd = decltype(d_)::value;
-                            acc[c][cd] += __shfl_xor(acc[c][cd], w, 64);
-                        });
-                    });
-                if (ic != 0) continue;
-            }
-            for (int d = 0; d < a.nd; d++)
-                digest<LA, LB, LC, LD, NC, true>(a, bra, ket, c0, acc, jmn + d * wsz, strip + d * wsz, nbf,
-                                                 JPQ_LDS ? jpq + d * wsz + q * NCD : nullptr,
-                                                 NSPLIT == 1 && a.nd == 1 ? jreg : nullptr, d * a.dstride);
-        }
-        if constexpr (NSPLIT == 1) {
-            static_for<0, NC>([&](auto c_) {
-                constexpr int c = decltype(c_)::value;
-                if (jreg[c] != 0.0) atomicAdd(&jmn[(c / NB) * NB + c % NB], jreg[c]);
-            });
-        }
-        __syncthreads();
-        const int M = a.pv.s1[bra], N = a.pv.s2[bra];
-        const int oM = a.fstart[M], oN = a.fstart[N];
-        const long base = a.mbase[M];
-        const int ld = a.mld[M];
-        for (int d = 0; d < a.nd; d++) {
-            const double* sd = strip + d * wsz;
-            const double* jd = jmn + d * wsz;
-            double* Kd = a.K + d * a.dstride + base;
-            double* Jd = a.J + d * a.dstride + base;
-            for (int k = threadIdx.x; k < nstrip; k += 256) {
-                const double v = sd[k];
-                if (v != 0.0) {
-                    const int r = k / nbf, col = k - r * nbf;
-                    const int row = r < NA ? oM + r : oN + (r - NA);
-                    GTF_ATOMIC_ADD(&Kd[(long)row * ld + col], v);
+                if (!on || jc != 0) return;
+                // (opaque, or the digestion's addresses would be formed ahead of
+                // the primitive loops and held across them)
+                int ox = ki.x, oy = ki.y, oj = j, onbf = nbf, orow = oM, ocol = oN;
+                asm volatile("" : "+v"(ox), "+v"(oy), "+v"(oj), "+s"(onbf), "+s"(orow), "+s"(ocol));
+                for (int d = 0; d < a.nd; d++) {
+                    const double* D = a.D + d * a.dstride + mat;
+                    DigestCtx x;
+                    x.Dm = as_const(D + (long)orow * onbf);
+                    x.rm = BLDS ? drow + d * (NA + NB) * onbf : D + (long)orow * onbf;
+                    x.rn = BLDS ? drow + d * (NA + NB) * onbf + NA * onbf : D + (long)ocol * onbf;
+                    x.ld = onbf;
+                    x.oN = ocol;
+                    x.oP = ox;
+                    x.oQ = oy;
+                    x.f1 = f1;
+                    x.f2 = ki.z;
+                    x.f3 = bra != ki.w;
+                    x.strip = strip + d * wsz;
+                    x.nbf = onbf;
+                    x.jmn = jmn + d * wsz + (lane & (GTF_JMN_COPIES - 1)) * NAB;
+                    x.dk = a.dk + d * NCD * a.nket + oj;
+                    x.nk = a.nket;
+                    x.jpq = buffered ? jpq + lane : nullptr;
+                    x.jk = a.jk + d * NCD * a.nket + oj;
+                    auto get = [&](auto c_, auto d_) GTF_INLINE { return (double)cell(c_, d_); };
+                    if constexpr (JREG_ABLE) {
+                        if (jreg_on) {
+                            digest_unit<LA, LB, LC, LD, A0, NAr, C0, NCr, true>(x, crt, get, jreg);
+                            continue;
+                        }
+                    }
+                    digest_unit<LA, LB, LC, LD, A0, NAr, C0, NCr, false>(x, crt, get, nullptr);
                 }
-            }
-            for (int k = threadIdx.x; k < NA * NB; k += 256) {
-                const double v = jd[k];
-                if (v != 0.0) GTF_ATOMIC_ADD(&Jd[(long)(oM + k / NB) * ld + oN + k % NB], v);
-            }
-            if constexpr (JPQ_LDS) {
-                const double* pd = jpq + d * wsz;
-                for (int k = threadIdx.x; k < njpq; k += 256) {
-                    const double v = pd[k];
+            };
+            for (int sp = sp0; sp < sp0 + spn; sp++)
+                for (int ic = ic0; ic < ic0 + icn; ic++) {
+                    const int j0 = ic + (jc << lic);
+                    if constexpr (!STATIC && EX) {
+                        const double* kf = on ? a.kv.f + ((long)(kb >> 6) * S::ESZ_CD + sp * S::HCD) * 64 + (kb & 63) : nullptr;
+                        Real acc[1][NAB];
+                        eri_lane_t<LA, LB, LC, LD, -1, 1, Real, BLDS>(br, kr, j0, js, kf, boys, acc);
+                        finish(std::integral_constant<int, 0>{}, std::integral_constant<int, NAB>{},
+                               std::integral_constant<int, -1>{}, std::integral_constant<int, 1>{}, acc, sp);
+                    } else if constexpr (!STATIC) {
+                        BraRef<Real> b1 = br;
+                        b1.E += sp * S::HAB;
+                        Real acc[1][NCD];
+                        eri_lane<LA, LB, LC, LD, -1, 1, Real, BLDS>(b1, kr, j0, js, boys, acc);
+                        finish(std::integral_constant<int, -1>{}, std::integral_constant<int, 1>{},
+                               std::integral_constant<int, 0>{}, std::integral_constant<int, NCD>{}, acc, sp);
+                    } else {
+                        split_switch<NSPLIT>(sp, [&](auto s_) GTF_INLINE {
+                            constexpr int F0 = decltype(s_)::value * NC;
+                            constexpr int FN = SIDE - F0 < NC ? SIDE - F0 : NC;
+                            if constexpr (EX) {
+                                Real acc[FN][NAB];
+                                eri_lane_t<LA, LB, LC, LD, F0, FN, Real, BLDS>(br, kr, j0, js, nullptr, boys, acc);
+                                finish(std::integral_constant<int, 0>{}, std::integral_constant<int, NAB>{},
+                                       std::integral_constant<int, F0>{}, std::integral_constant<int, FN>{}, acc, 0);
+                            } else {
+                                Real acc[FN][NCD];
+                                eri_lane<LA, LB, LC, LD, F0, FN, Real, BLDS>(br, kr, j0, js, boys, acc);
+                                finish(std::integral_constant<int, F0>{}, std::integral_constant<int, FN>{},
+                                       std::integral_constant<int, 0>{}, std::integral_constant<int, NCD>{}, acc, 0);
+                            }
+                        });
+                    }
+                }
+            // the block's J_PQ
+            if (buffered && on && jc == 0)
+                for (int cd = 0; cd < NCD; cd++) {
+                    double* p = jpq + cd * 64 + lane;
+                    const double v = *p;
                     if (v != 0.0) {
-                        const int q = k / NCD, cd = k - q * NCD;
-                        const int ket = a.ket_list[t.y + q];
-                        const int oP = a.fstart[a.pv.s1[ket]], oQ = a.fstart[a.pv.s2[ket]];
-                        GTF_ATOMIC_ADD(&Jd[(long)(oP + cd / ND) * ld + oQ + cd % ND], v);
+                        GTF_ATOMIC_ADD(&a.jk[cd * a.nket + j], v);
+                        *p = 0.0;
+                    }
+                }
+        }
+        if constexpr (JREG_ABLE) {
+            if (jreg_on)
+                static_for<0, NAB>([&](auto c_) GTF_INLINE {
+                    constexpr int c = decltype(c_)::value;
+                    if (jreg[c] != 0.0) atomicAdd(&jmn[(lane & (GTF_JMN_COPIES - 1)) * NAB + c], jreg[c]);
+                });
+        }
+        if (threadIdx.x == 0) s_task = next;
+        __syncthreads();
+        for (int d = 0; d < a.nd; d++) {
+            double* sd = strip + d * wsz;
+            double* jd = jmn + d * wsz;
+            double* Kd = a.K + d * a.dstride + mat;
+            double* Jd = a.J + d * a.dstride + mat;
+            for (int o = 0; o < NA + NB; o++) {
+                double* Kr = Kd + (long)(o < NA ? oM + o : oN + (o - NA)) * nbf;
+                for (int k = threadIdx.x; k < nbf; k += NT) {
+                    const double v = sd[o * nbf + k];
+                    if (v != 0.0) {
+                        GTF_ATOMIC_ADD(&Kr[k], v);
+                        sd[o * nbf + k] = 0.0;
                     }
                 }
             }
+            for (int k = threadIdx.x; k < NAB; k += NT) {
+                double v = 0.0;
+                for (int c = 0; c < GTF_JMN_COPIES; c++) {
+                    v += jd[c * NAB + k];
+                    jd[c * NAB + k] = 0.0;
+                }
+                if (v != 0.0) GTF_ATOMIC_ADD(&Jd[(long)(oM + k / NB) * nbf + oN + k % NB], v);
+            }
         }
+        if (threadIdx.x == 0) s_unit = 0;
+        open = open_tile(__builtin_amdgcn_readfirstlane(s_task));
         __syncthreads();
     }
     record_workgroup(a, t_begin, taken);
 }
 
-// update_F digestion of a quartet evaluated with bra and ket exchanged: the
-// thread holds (cd | ab) for its NCT ket components cd0.. and every bra
-// component ab, acc[k][ab].  Same contributions as digest<..., true>: J_MN
-// summed in jmn_reg[NAB] (registers, all bra components), J_PQ to the ket's
-// LDS row, the exchange blocks K_MP, K_NP, K_MQ, K_NQ to the bra rows of the
-// LDS strip.
-template <int LA, int LB, int LC, int LD, int NCT>
-__device__ __forceinline__ void digest_t(const EriArgs& a, int bra, int ket, int cd0,
-                                         const double (&acc)[NCT][EriShape<LA, LB, LC, LD>::NAB],
-                                         double* jmn_reg, double* strip, int nbf, double* jpq, double* jmn_lds,
-                                         long doff)
+template <int LA, int LB, int LC, int LD, int NC, typename Real, bool BLDS>
+__global__ __launch_bounds__((tile_threads<LA, LB, LC, LD>()), (tile_min_waves<LA, LB, LC, LD>())) void eri_jk_tile_kernel(EriArgs a)
 {
-    using S = EriShape<LA, LB, LC, LD>;
-    constexpr int NAB = S::NAB, NA = S::NA, NB = S::NB, ND = S::ND;
-    const int M = a.pv.s1[bra], N = a.pv.s2[bra], P = a.pv.s1[ket], Q = a.pv.s2[ket];
-    const int f1 = (M != N), f2 = (P != Q), f3 = (bra != ket);
-    const double cJ1 = 2.0 * (1 + f1) * (1 + f2);
-    const double cJ2 = 2.0 * f3 * (1 + f1) * (1 + f2);
-    const double cMP = (1 + f3), cNP = f1 * (1 + f3), cMQ = f2 * (1 + f3), cNQ = f1 * f2 * (1 + f3);
-    const int ld = a.mld[M];
-    const long base = a.mbase[M];
-    const int oM = a.fstart[M], oN = a.fstart[N], oP = a.fstart[P], oQ = a.fstart[Q];
-    const double* __restrict__ D = a.D + doff + base;
-    static_for<0, NCT>([&](auto k_) {
-        constexpr int k = decltype(k_)::value;
-        const int cd = cd0 + k;
-        const int p = cd / ND, q = cd - (cd / ND) * ND;
-        const double dpq = D[(long)(oP + p) * ld + oQ + q];
-        // J_MN += cJ1 D_pq I (registers, or LDS with several densities) and
-        // J_PQ += cJ2 sum_mn D_mn I
-        double jpq_s = 0.0;
-        static_for<0, NAB>([&](auto ab_) {
-            constexpr int ab = decltype(ab_)::value;
-            constexpr int m = ab / NB, n = ab % NB;
-            if (jmn_lds) atomicAdd(&jmn_lds[ab], cJ1 * dpq * acc[k][ab]);
-            else jmn_reg[ab] += cJ1 * dpq * acc[k][ab];
-            jpq_s += D[(long)(oM + m) * ld + oN + n] * acc[k][ab];
-        });
-        if (f3) atomicAdd(&jpq[cd], cJ2 * jpq_s);
-        // K_MP[m][p] -= cMP sum_n D_nq I,  K_MQ[m][q] -= cMQ sum_n D_np I
-        static_for<0, NA>([&](auto m_) {
-            constexpr int m = decltype(m_)::value;
-            double smp = 0.0, smq = 0.0;
-            static_for<0, NB>([&](auto n_) {
-                constexpr int n = decltype(n_)::value;
-                const double x = acc[k][m * NB + n];
-                smp += D[(long)(oN + n) * ld + oQ + q] * x;
-                smq += D[(long)(oN + n) * ld + oP + p] * x;
-            });
-            atomicAdd(&strip[m * nbf + oP + p], -cMP * smp);
-            if (f2) atomicAdd(&strip[m * nbf + oQ + q], -cMQ * smq);
-        });
-        // K_NP[n][p] -= cNP sum_m D_mq I,  K_NQ[n][q] -= cNQ sum_m D_mp I
-        if (f1) {
-            static_for<0, NB>([&](auto n_) {
-                constexpr int n = decltype(n_)::value;
-                double snp = 0.0, snq = 0.0;
-                static_for<0, NA>([&](auto m_) {
-                    constexpr int m = decltype(m_)::value;
-                    const double x = acc[k][m * NB + n];
-                    snp += D[(long)(oM + m) * ld + oQ + q] * x;
-                    snq += D[(long)(oM + m) * ld + oP + p] * x;
-                });
-                atomicAdd(&strip[(NA + n) * nbf + oP + p], -cNP * snp);
-                if (f2) atomicAdd(&strip[(NA + n) * nbf + oQ + q], -cNQ * snq);
-            });
-        }
-    });
+    tile_kernel_body<LA, LB, LC, LD, NC, Real, BLDS, false>(a);
 }
 
-// The bra-row tile kernel for classes evaluated with bra and ket exchanged:
-// a thread owns NCT ket components and every bra component of its quartet,
-// so the Boys function and the R recursion of a primitive quartet are
-// computed by NCD / NCT threads instead of NAB / NC.  Units: (ket, ket
-// component chunk), no bra-primitive chunks.  LDS as eri_jk_tile_kernel.
 template <int LA, int LB, int LC, int LD, int NCT, typename Real, bool BLDS>
-__global__ __launch_bounds__(256) void eri_jk_tile_t_kernel(EriArgs a)
+__global__ __launch_bounds__((tile_threads<LA, LB, LC, LD>()), (tile_min_waves<LA, LB, LC, LD>())) void eri_jk_tile_t_kernel(EriArgs a)
 {
-    using S = EriShape<LA, LB, LC, LD>;
-    constexpr int NSPLIT = S::NCD / NCT;
-    constexpr int NA = S::NA, NB = S::NB, NCD = S::NCD, NAB = S::NAB, ND = S::ND;
-    constexpr bool LOW = std::is_same<Real, float>::value;
-    constexpr int L = LA + LB + LC + LD;
-    extern __shared__ double smem[];
-    __shared__ int s_task;
-    double* work;
-    const double* boys = tile_boys<L, BLDS>(a, smem, work);
-    const long long t_begin = (long long)wall_clock64();
-    int taken = 0;
-    for (;;) {
-        if (threadIdx.x == 0) s_task = atomicAdd(a.counter, 1);
-        __syncthreads();
-        const int task = s_task;
-        if (task >= a.ntiles) break;
-        taken++;
-        const int4 t = a.tiles[task];
-        const int bra = a.bra_list[t.x];
-        if (!bra_active(a, bra)) {
-            __syncthreads();  // every thread has read s_task before it is rewritten
-            continue;
-        }
-        const int nbf = a.mld[a.pv.s1[bra]];
-        const int nstrip = (NA + NB) * nbf;
-        double* strip = work;
-        double* jmn = work + nstrip;
-        double* jpq = jmn + NA * NB;
-        const int nkt = t.z - t.y;
-        const int njpq = nkt * NCD;
-        const int wsz = nstrip + NA * NB + njpq;  // work area per density
-        for (int k = threadIdx.x; k < a.nd * wsz; k += 256) work[k] = 0.0;
-        __syncthreads();
-        double jreg[NAB];
-        static_for<0, NAB>([&](auto c_) { jreg[decltype(c_)::value] = 0.0; });
-        const int nunits = nkt * NSPLIT;
-        for (int u = threadIdx.x; u < nunits; u += 256) {
-            const int q = u / NSPLIT;
-            const int cd0 = (u - q * NSPLIT) * NCT;
-            const int j = t.y + q;
-            if (!quartet_valid(a, t.x, j)) continue;
-            if ((a.vbra[t.x] * a.vket[j] >= a.tau2) == LOW) continue;
-            const int ket = a.ket_list[j];
-            double acc[NCT][NAB];
-            if constexpr (LOW) {
-                float accf[NCT][NAB];
-                eri_block<LC, LD, LA, LB, NCT, float>(a.pv, ket, bra, cd0, boys, accf);
-                static_for<0, NCT>([&](auto c_) {
-                    static_for<0, NAB>([&](auto d_) {
-                        acc[decltype(c_)::value][decltype(d_)::value] =
-                            (double)accf[decltype(c_)::value][decltype(d_)::value];
-                    });
-                });
-            } else {
-                eri_block<LC, LD, LA, LB, NCT, double>(a.pv, ket, bra, cd0, boys, acc);
-            }
-            for (int d = 0; d < a.nd; d++)
-                digest_t<LA, LB, LC, LD, NCT>(a, bra, ket, cd0, acc, jreg, strip + d * wsz, nbf,
-                                              jpq + d * wsz + q * NCD, a.nd == 1 ? nullptr : jmn + d * wsz,
-                                              d * a.dstride);
-        }
-        if (a.nd == 1)
-            static_for<0, NAB>([&](auto c_) {
-                constexpr int c = decltype(c_)::value;
-                if (jreg[c] != 0.0) atomicAdd(&jmn[c], jreg[c]);
-            });
-        __syncthreads();
-        const int M = a.pv.s1[bra], N = a.pv.s2[bra];
-        const int oM = a.fstart[M], oN = a.fstart[N];
-        const long base = a.mbase[M];
-        const int ld = a.mld[M];
-        for (int d = 0; d < a.nd; d++) {
-            const double* sd = strip + d * wsz;
-            const double* jd = jmn + d * wsz;
-            const double* pd = jpq + d * wsz;
-            double* Kd = a.K + d * a.dstride + base;
-            double* Jd = a.J + d * a.dstride + base;
-            for (int k = threadIdx.x; k < nstrip; k += 256) {
-                const double v = sd[k];
-                if (v != 0.0) {
-                    const int r = k / nbf, col = k - r * nbf;
-                    const int row = r < NA ? oM + r : oN + (r - NA);
-                    GTF_ATOMIC_ADD(&Kd[(long)row * ld + col], v);
-                }
-            }
-            for (int k = threadIdx.x; k < NA * NB; k += 256) {
-                const double v = jd[k];
-                if (v != 0.0) GTF_ATOMIC_ADD(&Jd[(long)(oM + k / NB) * ld + oN + k % NB], v);
-            }
-            for (int k = threadIdx.x; k < njpq; k += 256) {
-                const double v = pd[k];
-                if (v != 0.0) {
-                    const int q = k / NCD, cd = k - q * NCD;
-                    const int ket = a.ket_list[t.y + q];
-                    const int oP = a.fstart[a.pv.s1[ket]], oQ = a.fstart[a.pv.s2[ket]];
-                    GTF_ATOMIC_ADD(&Jd[(long)(oP + cd / ND) * ld + oQ + cd % ND], v);
-                }
-            }
-        }
-        __syncthreads();
-    }
-    record_workgroup(a, t_begin, taken);
+    tile_kernel_body<LA, LB, LC, LD, NCT, Real, BLDS, true>(a);
 }
 
 // launch helpers (eri_table.cpp)
 typedef void (*eri_kernel_t)(EriArgs);
 struct EriClassInfo {
     int la, lb, lc, ld;
-    int nc;         // bra components per thread
-    int nsplit;     // threads per quartet
+    int nc;         // bra components per thread of the unit kernels (jk, diag, store)
+    int nsplit;     // and threads per quartet
+    int tile_threads;  // largest workgroup of the tile kernels
+    int nc_tile;       // bra components per thread of the tile kernels
+    int nsplit_tile;
+    bool full_E;       // the standard tile kernel reads the full coefficients
     int nints;      // integrals per quartet
     eri_kernel_t jk, diag, store;
     // tile kernels, [0] Boys slab read from HBM, [1] staged in LDS
     eri_kernel_t jk_tile[2];     // FP64 quartets (v_bra v_ket >= tau2)
     eri_kernel_t jk_tile_lo[2];  // FP32 quartets (v_bra v_ket < tau2)
-    // classes evaluated with bra and ket exchanged (nsplit_t > 0): threads
-    // per quartet and the two tile kernels
-    int nsplit_t;
+    // classes that have a tile kernel with the contractions exchanged
+    // (nsplit_t > 0): threads per quartet, ket components per thread
+    int nsplit_t, nc_t;
     eri_kernel_t jk_tile_t[2], jk_tile_t_lo[2];
 };
 const EriClassInfo* gtf_eri_class(int cls);

@@ -20,6 +20,38 @@
 // ket-list block re-sorted by primitive count (one wavefront)
 #define GTF_KET_BLOCK 64
 
+// A tile of the J/K kernels is one bra pair and several runs of its kets:
+// TileHead.  A run is int4 (first ket, span word, chunk word, 0).
+// span word: kets, first component chunk and number of them
+#define GTF_RUN_SPAN(kets, sp0, spn) ((kets) | (sp0) << 15 | (spn) << 20)
+#define GTF_RUN_KETS(y) ((y) & 32767)
+#define GTF_RUN_SP0(y) (((y) >> 15) & 31)
+#define GTF_RUN_SPN(y) ((y) >> 20)
+#define GTF_RUN_MAX_KETS 32767
+// chunk word: log2 of the ket-primitive chunks, log2 of the lanes that share a
+// ket, first ket-primitive chunk and number of them
+#define GTF_RUN_CHUNKS(lic, ljc, ic0, icn) ((lic) | (ljc) << 4 | (ic0) << 8 | (icn) << 20)
+#define GTF_RUN_LIC(z) ((z) & 15)
+#define GTF_RUN_LJC(z) (((z) >> 4) & 15)
+#define GTF_RUN_IC0(z) (((z) >> 8) & 4095)
+#define GTF_RUN_ICN(z) ((z) >> 20)
+#define GTF_MAX_LIC 9  // at most 512 chunks
+// Everything of the bra that a workgroup needs to start a tile, read with one
+// scalar load (looked up through the pair and shell arrays it was a chain of
+// five dependent loads, several microseconds a tile).
+struct TileHead {
+    int row, run0, nrun;  // bra row, runs
+    int bra;              // pair id
+    int prim, nprim;      // first primitive pair, primitive pairs
+    int oM, oN;           // function offsets
+    int two;              // 1 if the shells differ
+    int nbf, mol;         // size of the molecule's matrices, molecule
+    int rank;
+    long mat;             // the molecule's matrix block
+    long E;               // first coefficient, in the layout that the kernel reads
+};
+static_assert(sizeof(TileHead) == 64, "read as 16 dwords");
+
 // Boys-function grid: F_m(T0) for T0 = i * BOYS_DELTA, i = 0..BOYS_NGRID-1,
 // m = 0..BOYS_NCOL-1; T >= BOYS_TMAX uses the asymptotic form.
 #define BOYS_DELTA 0.05
@@ -36,6 +68,9 @@
 #define BOYS8_NTERM 8
 #define BOYS8_NM 9
 #define BOYS8_SLAB (BOYS8_NGRID * BOYS8_NTERM)
+// the slabs, then exp(-T0) of the grid points (padded to whole double2)
+#define BOYS8_EXP (BOYS8_NGRID + 1)
+#define BOYS8_TOTAL (BOYS8_NM * BOYS8_SLAB + BOYS8_EXP)
 
 #define GTF_CHECK(call)                                                                    \
     do {                                                                                   \
@@ -103,6 +138,9 @@ __device__ __forceinline__ float rsqrt_nr(float s)
     return y;
 }
 
+// for lambdas whose arrays must stay in registers
+#define GTF_INLINE __attribute__((always_inline))
+
 // compile-time loop: f(std::integral_constant<int, i>) for i in [B, E)
 template <int B, int E, typename F>
 __host__ __device__ __forceinline__ void static_for(F&& f)
@@ -125,7 +163,42 @@ struct PairView {
     const long* zoff;    // offset into Ez[]
     const double* Ez;    // the same, structural nonzeros only (herm_nz_pos order)
     const double* q;     // Schwarz bound per primitive pair (a pair's primitives in descending order)
+    const float *Ef, *Ezf;  // E and Ez rounded to FP32 (systems with FP32 tiles)
     double peps;         // primitive quartets with q_bra q_ket < peps are skipped (0: none)
+};
+
+// Ket side of one pair type's significant-pair list, in list order, for the
+// tile kernels: 64 kets of a segment form a block whose primitive pairs are
+// stored primitive by primitive, each as rec(nnz) rows of 64 double2 -- (p,
+// Px), (Py, Pz) and the compact Hermite coefficients two by two -- so that the
+// lanes of a wavefront, which hold consecutive kets, read whole lines.
+// base[j] = 64 * (first primitive row of ket j's block) + (place in the block).
+struct KetView {
+    const int* base;
+    const double2* d;
+    const double* f;    // pair types with a chunked ket side: the full coefficients, rows of 64 doubles
+    const double* q;    // Schwarz bound per primitive pair, rows of 64
+    const int4* info;   // function offsets of the two shells, 1 if they differ, pair id
+    const int* nprim;
+    __host__ __device__ static constexpr int rec(int nnz) { return 2 + (nnz + 1) / 2; }
+    // pair types whose full coefficients are stored (pp, ds, dp)
+    __host__ __device__ static constexpr bool full(int type) { return type >= 2 && type <= 4; }
+};
+
+// One pair type's list in the density's and J_PQ's list-ordered copies: [density]
+// [component][list position].
+struct JkList {
+    int n;             // list length
+    int nc, nd;        // functions of the two shells
+    const int4* info;  // KetView::info
+    double* dk;
+    double* jk;
+};
+struct JkLists {
+    JkList t[GTF_NPAIRTYPES];
+    const int* s1;      // first shell of each pair
+    const long* mbase;  // per shell: matrix block and leading dimension
+    const int* mld;
 };
 
 struct BasisView {

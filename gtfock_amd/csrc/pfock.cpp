@@ -337,8 +337,6 @@ PFockStatus_t PFock_computeFock(BasisSet_t basis, PFock_t pf)
     const long nn = (long)pf->nbf * pf->nbf;
     PF_HIP(hipEventRecord(pf->ev0, pf->stream), "hipEventRecord");
     const int nd = pf->num_dmat;
-    if (gtf_fill(pf->stream, pf->d_J[0], nn * nd, 0.0) || gtf_fill(pf->stream, pf->d_K[0], nn * nd, 0.0))
-        return PFOCK_STATUS_EXECUTION_FAILED;
     // every density from each integral (update_F's num_dmat loop,
     // pfock/fock_task.c:46) when the per-density LDS work areas fit, else
     // one build per density
@@ -596,14 +594,14 @@ int gtf_pfock_class_info(PFock_t pf, int cls, int* info)
     info[1] = ci->lb;
     info[2] = ci->lc;
     info[3] = ci->ld;
-    info[4] = ci->nc;
-    info[5] = ci->nsplit;
+    info[4] = pf->sys.ntiles[cls] > 0 ? ci->nc_tile : ci->nc;
+    info[5] = pf->sys.ntiles[cls] > 0 ? ci->nsplit_tile : ci->nsplit;
     info[6] = pf->sys.ntiles[cls];
     info[7] = pf->sys.ntiles_lo[cls];
     // the exchanged tile kernel runs the class: ket components per thread
     const bool ex = pf->sys.exchanged(cls);
     info[8] = ex ? 1 : 0;
-    info[9] = ex ? (2 * ci->lc + 1) * (2 * ci->ld + 1) / ci->nsplit_t : 0;
+    info[9] = ex ? ci->nc_t : 0;
     info[10] = pf->sys.shape[cls].boys_lds;
     return 0;
 }

@@ -9,10 +9,34 @@
 int gtf_build_pairs(hipStream_t st, const BasisView& b, int npairs, const int* s1, const int* s2,
                     const int* poff, const long* eoff, double4* prim, double* E, const long* zoff, double* Ez,
                     int* nprim_out, double* qout, double prim_eps);
-// primitive quartets evaluated over a tile list (prim_census_kernel)
+// the ket records of one type list (KetView): base, info and nprim are per
+// list position, d and q as base lays them out
+struct KetPack {
+    int n;            // list length
+    const int* sig;   // pair ids in list order
+    const int* base;
+    int nnz;          // compact Hermite coefficients per primitive pair
+    int nfull;        // full Hermite coefficients per primitive pair (0: not stored)
+    double2* d;
+    double* f;
+    double* q;
+    int4* info;
+    int* nprim;
+};
+// Before the class launches of a build: J and K of nd densities (total
+// elements each, dstride apart) and the n counters cleared, the lists' density
+// elements gathered and their J_PQ cleared.  After them: J_PQ added to J.
+int gtf_jk_begin(hipStream_t st, const JkLists& l, const double* D, double* J, double* K, long total, int nd,
+                 long dstride, int* counters, int n);
+int gtf_jk_end(hipStream_t st, const JkLists& l, double* J, int nd, long dstride);
+int gtf_round_f32(hipStream_t st, const double* x, long n, float* y);
+int gtf_pack_kets(hipStream_t st, const PairView& pv, const int* fstart, const KetPack& k);
+// primitive quartets evaluated over a run list (prim_census_kernel); of the
+// runs over the same kets only the one holding chunk 0 of both kinds counts
 struct CensusArgs {
-    const int4* tiles;
-    int ntiles;
+    const int4* runs;
+    const int* run_row;  // bra row of each run
+    int nruns;
     const int* bra_list;
     const int* ket_list;
     const double* vbra;

@@ -8,6 +8,8 @@
 // and  E^{i,j+1}_t = E^{ij}_{t-1}/(2p) + X_PB E^{ij}_t + (t+1) E^{ij}_{t+1}
 // (Helgaker, Jorgensen, Olsen, Molecular Electronic-Structure Theory 9.5),
 // transformed to real solid harmonics and scaled by c_a c_b exp(-mu AB^2)/p.
+#include <algorithm>
+
 #include "gtf_internal.h"
 #include "screen.h"
 
@@ -316,24 +318,26 @@ __global__ void fill_qlist_diag_kernel(int n, const int* __restrict__ ids, int2*
     if (k < n) q[k] = make_int2(ids[k], ids[k]);
 }
 
-// Primitive quartets the J/K kernels evaluate over a list of tiles (bra
-// row, first ket, end ket): for each quartet of a tile that passes the
+// Primitive quartets the J/K kernels evaluate over the runs of a tile list
+// (run, bra row): for each quartet of a run that passes the
 // kernels' tests (Schwarz, one orientation in a diagonal class, the
 // precision split), the pairs (i, j) of bra and ket primitives with
 // q_i q_j >= peps when the class screens primitives, else all of them.
 // With both lists in descending order of q that is what the kernels' loops
-// visit, whichever pair they take as the bra.  One workgroup per tile, one
+// visit, whichever pair they take as the bra.  One workgroup per run, one
 // thread per ket; the total is added to *out.
 __global__ __launch_bounds__(256) void prim_census_kernel(CensusArgs c)
 {
-    const int4 t = c.tiles[blockIdx.x];
-    const int bra = c.bra_list[t.x];
+    const int4 t = c.runs[blockIdx.x];
+    if (GTF_RUN_IC0(t.z) != 0 || GTF_RUN_SP0(t.y) != 0) return;
+    const int row = c.run_row[blockIdx.x];
+    const int bra = c.bra_list[row];
     const int nbp = c.pv.nprim[bra];
     const double* __restrict__ qb = c.pv.q + c.pv.poff[bra];
-    const double vb = c.vbra[t.x];
+    const double vb = c.vbra[row];
     unsigned long long cnt = 0;
-    for (int j = t.y + threadIdx.x; j < t.z; j += blockDim.x) {
-        if (!(vb * c.vket[j] >= c.tol2) || (c.same && c.rank_ket[j] > c.rank_bra[t.x])) continue;
+    for (int j = t.x + threadIdx.x; j < t.x + GTF_RUN_KETS(t.y); j += blockDim.x) {
+        if (!(vb * c.vket[j] >= c.tol2) || (c.same && c.rank_ket[j] > c.rank_bra[row])) continue;
         if ((vb * c.vket[j] >= c.tau2) == (c.low != 0)) continue;
         const int ket = c.ket_list[j];
         const int nk = c.pv.nprim[ket];
@@ -356,6 +360,85 @@ __global__ __launch_bounds__(256) void prim_census_kernel(CensusArgs c)
     }
     for (int off = 32; off > 0; off >>= 1) cnt += __shfl_xor(cnt, off);
     if ((threadIdx.x & 63) == 0 && cnt) atomicAdd(c.out, cnt);
+}
+
+// Ket records of a type list: one thread per ket copies its primitive pairs
+// into the 64-ket blocks, so a wavefront's writes are whole rows; the reads
+// are the pairs' own records.
+__global__ __launch_bounds__(256) void pack_kets_kernel(PairView pv, const int* __restrict__ fstart, KetPack k)
+{
+    const int j = blockIdx.x * 256 + threadIdx.x;
+    if (j >= k.n) return;
+    const int id = k.sig[j], np = pv.nprim[id], b = k.base[j], rec = KetView::rec(k.nnz);
+    const int s1 = pv.s1[id], s2 = pv.s2[id];
+    k.info[j] = make_int4(fstart[s1], fstart[s2], s1 != s2, id);
+    k.nprim[j] = np;
+    const double* z = pv.Ez + pv.zoff[id];
+    const int po = pv.poff[id];
+    double2* d = k.d + (long)(b >> 6) * (rec * 64) + (b & 63);
+    for (int i = 0; i < np; i++, d += rec * 64, z += k.nnz) {
+        const double4 p = pv.prim[po + i];
+        d[0] = make_double2(p.x, p.y);
+        d[64] = make_double2(p.z, p.w);
+        for (int c = 0; c < k.nnz; c += 2) d[(2 + c / 2) * 64] = make_double2(z[c], c + 1 < k.nnz ? z[c + 1] : 0.0);
+        k.q[b + 64L * i] = pv.q[po + i];
+        if (k.nfull) {
+            const double* e = pv.E + pv.eoff[id] + (long)i * k.nfull;
+            double* f = k.f + ((long)(b >> 6) + i) * k.nfull * 64 + (b & 63);
+            for (int c = 0; c < k.nfull; c++) f[c * 64] = e[c];
+        }
+    }
+}
+
+__global__ __launch_bounds__(256) void round_f32_kernel(const double* __restrict__ x, long n, float* __restrict__ y)
+{
+    for (long k = blockIdx.x * 256L + threadIdx.x; k < n; k += gridDim.x * 256L) y[k] = (float)x[k];
+}
+
+// f(list, position, density) over the lists' positions, one thread each
+template <typename F>
+__device__ __forceinline__ void each_ket(const JkLists& l, int nd, F&& f)
+{
+    for (long k = blockIdx.x * 256L + threadIdx.x;; k += gridDim.x * 256L) {
+        long i = k;
+        int t = 0;
+        while (t < GTF_NPAIRTYPES && i >= (long)nd * l.t[t].n) i -= (long)nd * l.t[t++].n;
+        if (t == GTF_NPAIRTYPES) return;
+        const int d = (int)(i / l.t[t].n);
+        f(l.t[t], (int)(i - (long)d * l.t[t].n), d);
+    }
+}
+
+__global__ __launch_bounds__(256) void jk_begin_kernel(JkLists l, const double* __restrict__ D, double* __restrict__ J,
+                                                       double* __restrict__ K, long total, int nd, long dstride,
+                                                       int* __restrict__ counters, int n)
+{
+    const long t0 = blockIdx.x * 256L + threadIdx.x, step = gridDim.x * 256L;
+    if (t0 < n) counters[t0] = 0;
+    for (int d = 0; d < nd; d++)
+        for (long k = t0; k < total; k += step) J[d * dstride + k] = K[d * dstride + k] = 0.0;
+    each_ket(l, nd, [&](const JkList& t, int j, int d) {
+        const int4 ki = t.info[j];
+        const int s = l.s1[ki.w], ld = l.mld[s];
+        const double* b = D + d * dstride + l.mbase[s] + (long)ki.x * ld + ki.y;
+        const long o = (long)d * t.nc * t.nd * t.n + j;
+        for (int c = 0; c < t.nc * t.nd; c++) {
+            t.dk[o + (long)c * t.n] = b[(long)(c / t.nd) * ld + c % t.nd];
+            t.jk[o + (long)c * t.n] = 0.0;
+        }
+    });
+}
+
+// every (pair, component) is one element of J, so plain additions
+__global__ __launch_bounds__(256) void jk_end_kernel(JkLists l, double* __restrict__ J, int nd, long dstride)
+{
+    each_ket(l, nd, [&](const JkList& t, int j, int d) {
+        const int4 ki = t.info[j];
+        const int s = l.s1[ki.w], ld = l.mld[s];
+        double* b = J + d * dstride + l.mbase[s] + (long)ki.x * ld + ki.y;
+        const long o = (long)d * t.nc * t.nd * t.n + j;
+        for (int c = 0; c < t.nc * t.nd; c++) b[(long)(c / t.nd) * ld + c % t.nd] += t.jk[o + (long)c * t.n];
+    });
 }
 
 // ---- host launchers -------------------------------------------------------
@@ -392,10 +475,49 @@ int gtf_fill_qlist_diag(hipStream_t st, int n, const int* ids, int2* q)
     return 0;
 }
 
+static int jk_blocks(const JkLists& l, long most, int nd)
+{
+    long n = 0;
+    for (const JkList& t : l.t) n += (long)nd * t.n;
+    return (int)std::max<long>(1, std::min<long>(2048, (std::max(n, most) + 255) / 256));
+}
+
+int gtf_jk_begin(hipStream_t st, const JkLists& l, const double* D, double* J, double* K, long total, int nd,
+                 long dstride, int* counters, int n)
+{
+    jk_begin_kernel<<<jk_blocks(l, std::max<long>(total / 4, n), nd), 256, 0, st>>>(l, D, J, K, total, nd, dstride,
+                                                                                   counters, n);
+    GTF_CHECK(hipGetLastError());
+    return 0;
+}
+
+int gtf_jk_end(hipStream_t st, const JkLists& l, double* J, int nd, long dstride)
+{
+    jk_end_kernel<<<jk_blocks(l, 1, nd), 256, 0, st>>>(l, J, nd, dstride);
+    GTF_CHECK(hipGetLastError());
+    return 0;
+}
+
+int gtf_round_f32(hipStream_t st, const double* x, long n, float* y)
+{
+    if (n <= 0) return 0;
+    round_f32_kernel<<<(int)std::min<long>(8192, (n + 255) / 256), 256, 0, st>>>(x, n, y);
+    GTF_CHECK(hipGetLastError());
+    return 0;
+}
+
+int gtf_pack_kets(hipStream_t st, const PairView& pv, const int* fstart, const KetPack& k)
+{
+    if (k.n <= 0) return 0;
+    pack_kets_kernel<<<(k.n + 255) / 256, 256, 0, st>>>(pv, fstart, k);
+    GTF_CHECK(hipGetLastError());
+    return 0;
+}
+
 int gtf_prim_census(hipStream_t st, const CensusArgs& c)
 {
-    if (c.ntiles <= 0) return 0;
-    prim_census_kernel<<<c.ntiles, 256, 0, st>>>(c);
+    if (c.nruns <= 0) return 0;
+    prim_census_kernel<<<c.nruns, 256, 0, st>>>(c);
     GTF_CHECK(hipGetLastError());
     return 0;
 }
