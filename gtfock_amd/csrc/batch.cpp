@@ -72,6 +72,7 @@ struct GtfBatch {
     double *p_X = nullptr, *p_S = nullptr, *p_F = nullptr, *p_D = nullptr;      // padded
     double *p_D2 = nullptr, *p_D3 = nullptr, *p_W = nullptr, *p_W2 = nullptr;  // padded work
     double *evecs = nullptr, *Fvecs = nullptr;                                  // B_MAX_DIIS padded sets
+    double* d_ppart = nullptr;
     double *d_stats = nullptr, *d_dots = nullptr, *d_coef = nullptr, *d_energy = nullptr;
     int *d_iters = nullptr, *d_skip = nullptr, *d_nvec = nullptr, *d_slot = nullptr, *d_skip2 = nullptr;
     // host sources of asynchronous copies (alive until the stream syncs)
@@ -260,6 +261,7 @@ int GtfBatch::scf_setup(const GtfBatch* from, const int* from_idx)
     evecs = s.dalloc<double>((size_t)ptotal * B_MAX_DIIS);
     Fvecs = s.dalloc<double>((size_t)ptotal * B_MAX_DIIS);
     d_stats = s.dalloc<double>(3 * nmol);
+    d_ppart = s.dalloc<double>(gtf_bpurif_part(nmol, maxpld));
     d_dots = s.dalloc<double>((size_t)BMAX_DOTS * nmol);
     d_coef = s.dalloc<double>((size_t)BMAX_DOTS * nmol);
     d_energy = s.dalloc<double>(nmol);
@@ -272,7 +274,7 @@ int GtfBatch::scf_setup(const GtfBatch* from, const int* from_idx)
     d_pcoef = s.dalloc<double>(2 * (size_t)nmol);
     d_low = s.dalloc<int>(nmol);
     if (!d_part || !d_pcoef || !d_low) return -2;
-    if (!d_H || !d_S || !d_F || !T || !V || !evecs || !Fvecs || !d_stats || !d_dots || !d_coef || !d_energy ||
+    if (!d_H || !d_S || !d_F || !T || !V || !evecs || !Fvecs || !d_stats || !d_ppart || !d_dots || !d_coef || !d_energy ||
         !d_iters || !d_skip || !d_skip2 || !d_nvec || !d_slot)
         return -2;
     for (double** p : pads)
@@ -648,13 +650,15 @@ int GtfBatch::purify(const std::vector<int>& active)
     for (it = 0; it < 200; it++) {
         // molecules already converged skip their GEMMs through d_iters >= 0;
         // those in the split-BF16 phase take the ozaki.h products instead
-        if (gtf_bgemm(stream, L, skip, d_iters, p_D, p_D, p_D2, 0, d_low) ||
-            gtf_bgemm(stream, L, skip, d_iters, p_D, p_D2, p_D3, 0, d_low))
+        if (purif_mode == GTF_LOW_FP64) {
+            if (gtf_bpurif_iterate(stream, L, skip, d_iters, d_ppart, 1e-11, p_D, p_D2, p_D3, it)) return -1;
+        } else if (gtf_bgemm(stream, L, skip, d_iters, p_D, p_D, p_D2, 0, d_low) ||
+                   gtf_bgemm(stream, L, skip, d_iters, p_D, p_D2, p_D3, 0, d_low) ||
+                   (purif_mode == GTF_LOW_SPLIT && gtf_oz_square_cube(stream, o, oz, p_D, p_D2, p_D3)) ||
+                   gtf_bpurif_stats(stream, L, skip, p_D, p_D2, p_D3, d_iters, d_stats, it, 1e-11, d_low, purif_until) ||
+                   gtf_bpurif_update(stream, L, skip, d_iters, d_stats, p_D, p_D2, p_D3, it)) {
             return -1;
-        if (purif_mode == GTF_LOW_SPLIT && gtf_oz_square_cube(stream, o, oz, p_D, p_D2, p_D3)) return -1;
-        if (gtf_bpurif_stats(stream, L, skip, p_D, p_D2, p_D3, d_iters, d_stats, it, 1e-11, d_low, purif_until))
-            return -1;
-        if (gtf_bpurif_update(stream, L, skip, d_iters, d_stats, p_D, p_D2, p_D3, it)) return -1;
+        }
         if (it % 2 == 1) {
             B_CHECK(hipMemcpyAsync(it_h.data(), d_iters, sizeof(int) * nmol, hipMemcpyDeviceToHost, stream));
             B_CHECK(hipStreamSynchronize(stream));

@@ -38,6 +38,13 @@ int gtf_bpurif_stats(hipStream_t st, const BatchLayout& L, const int* skip, cons
                      double fp32_until = 0.0, int* low_iters = nullptr);
 int gtf_bpurif_update(hipStream_t st, const BatchLayout& L, const int* skip, const int* iters, const double* stats,
                       double* D, const double* D2, const double* D3, int it);
+// One FP64 purification iteration: D2 = D D, D3 = D D2 and the update of D
+// (which must be symmetric); iters[m] = it for a molecule whose ||D - D2||_F is
+// below tol, after its update, also in host_iters (pinned host memory, may be
+// null).  part: gtf_bpurif_part doubles.
+int gtf_bpurif_iterate(hipStream_t st, const BatchLayout& L, const int* skip, int* iters, double* part, double tol,
+                       double* D, double* D2, double* D3, int it, int* host_iters = nullptr);
+size_t gtf_bpurif_part(int nmol, int maxpld);
 int gtf_bantisym(hipStream_t st, const BatchLayout& L, const int* skip, const double* W, double* E);
 int gtf_bmultidot(hipStream_t st, const BatchLayout& L, const int* skip, const int* nvec, const double* x,
                   const double* vecs, long stride, double* dots);

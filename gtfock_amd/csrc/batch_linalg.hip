@@ -35,6 +35,94 @@ __global__ __launch_bounds__(256) void bgemm_kernel(const long* __restrict__ pof
     else gemm_tile<TRANSB, false>(ld, A0 + o, B0 + o, C0 + o, row0, col0);
 }
 
+// fixed-order tree reduction of one value per thread of a block of NT threads
+template <int NT = 256, typename Op>
+__device__ __forceinline__ double block_reduce(double v, double* sh, Op op)
+{
+    sh[threadIdx.x] = v;
+    __syncthreads();
+    for (int s = NT / 2; s > 0; s >>= 1) {
+        if (threadIdx.x < s) sh[threadIdx.x] = op(sh[threadIdx.x], sh[threadIdx.x + s]);
+        __syncthreads();
+    }
+    const double r = sh[0];
+    __syncthreads();
+    return r;
+}
+
+// C_m = A_m * B_m^T, every tile
+__global__ __launch_bounds__(ROWS_THREADS) void bgemm_rows_kernel(const long* __restrict__ poff, const int* __restrict__ pld,
+                                                         const int* __restrict__ skip, const int* __restrict__ done,
+                                                         const double* __restrict__ A0, const double* __restrict__ B0,
+                                                         double* __restrict__ C0)
+{
+    __shared__ double red[ROWS_W][ROWS_T * ROWS_T];
+    const int m = blockIdx.z, ld = pld[m], row0 = blockIdx.y * ROWS_T, col0 = blockIdx.x * ROWS_T;
+    if (row0 >= ld || col0 >= ld || (skip && skip[m]) || (done && done[m] >= 0)) return;
+    const long o = poff[m];
+    rows_tile(ld, A0 + o, B0 + o, row0, col0, red);
+    for (int k = threadIdx.x; k < ROWS_T * ROWS_T; k += ROWS_THREADS) C0[o + (long)(row0 + k / ROWS_T) * ld + col0 + k % ROWS_T] = red[0][k];
+}
+
+// tiles of the lower triangle
+__host__ __device__ constexpr int tri_tiles(int ld) { return (ld / ROWS_T) * (ld / ROWS_T + 1) / 2; }
+
+// One product of the purification, C_m = D_m * B_m of symmetric commuting
+// matrices (B is D, then D^2): the tiles of the lower triangle, each also
+// written transposed.  The partial sums of the statistics come from the tiles:
+// with B = D (CUBE false) {||D - C||_F^2, tr(D - C)}, with B = D^2 tr(B - C).
+template <bool CUBE>
+__global__ __launch_bounds__(ROWS_THREADS) void bpurif_product_kernel(const long* __restrict__ poff,
+                                                             const int* __restrict__ pld, const int* __restrict__ skip,
+                                                             const int* __restrict__ done,
+                                                             const double* __restrict__ D0,
+                                                             const double* __restrict__ B0, double* __restrict__ C0,
+                                                             double* __restrict__ part, int mtiles)
+{
+    __shared__ double red[ROWS_W][ROWS_T * ROWS_T];
+    const int m = blockIdx.y, t = blockIdx.x, ld = pld[m];
+    if (t >= tri_tiles(ld) || (skip && skip[m]) || done[m] >= 0) return;
+    int ti = (int)((sqrtf(8.0f * t + 1.0f) - 1.0f) * 0.5f);
+    while ((ti + 1) * (ti + 2) / 2 <= t) ti++;
+    while (ti * (ti + 1) / 2 > t) ti--;
+    const int tj = t - ti * (ti + 1) / 2;
+    const int row0 = ti * ROWS_T, col0 = tj * ROWS_T;
+    const long o = poff[m];
+    rows_tile(ld, D0 + o, B0 + o, row0, col0, red);
+    double* C = C0 + o;
+    const double* S = (CUBE ? B0 : D0) + o;  // what C is subtracted from
+    double e = 0.0, tr = 0.0;
+    for (int k = threadIdx.x; k < ROWS_T * ROWS_T; k += ROWS_THREADS) {
+        const int i = k / ROWS_T, j = k % ROWS_T;
+        const double low = red[0][k], up = red[0][j * ROWS_T + i];
+        double v = low;
+        if (ti == tj) v = 0.5 * (low + up);
+        else C[(long)(col0 + i) * ld + row0 + j] = up;
+        C[(long)(row0 + i) * ld + col0 + j] = v;
+        if (!CUBE || (ti == tj && i == j)) {
+            const double x = S[(long)(row0 + i) * ld + col0 + j] - v;
+            e += x * x;
+            if (ti == tj && i == j) tr += x;
+        }
+    }
+    if (CUBE && ti != tj) return;  // tr alone
+    __syncthreads();
+    double* sh = red[1];
+    auto add = [](double a, double b) { return a + b; };
+    if (!CUBE) e = block_reduce<ROWS_THREADS>(e, sh, add);
+    if (ti == tj) tr = block_reduce<ROWS_THREADS>(tr, sh, add);
+    if (threadIdx.x == 0) {
+        double* p = part + ((long)m * mtiles + t) * 3;
+        if (CUBE) {
+            p[2] = tr;
+        } else {
+            p[0] = ti == tj ? e : 2.0 * e;
+            p[1] = ti == tj ? tr : 0.0;
+            p[2] = 0.0;
+        }
+    }
+}
+
 // packed -> padded (zero padding) and padded -> packed
 __global__ void bpad_kernel(const long* __restrict__ off, const int* __restrict__ nn, const long* __restrict__ poff,
                             const int* __restrict__ pld, const int* __restrict__ skip, const double* __restrict__ src,
@@ -65,21 +153,6 @@ __global__ void bunpad_kernel(const long* __restrict__ off, const int* __restric
     }
 }
 
-// fixed-order tree reduction of one value per thread of a 256-thread block
-template <typename Op>
-__device__ __forceinline__ double block_reduce(double v, double* sh, Op op)
-{
-    sh[threadIdx.x] = v;
-    __syncthreads();
-    for (int s = 128; s > 0; s >>= 1) {
-        if (threadIdx.x < s) sh[threadIdx.x] = op(sh[threadIdx.x], sh[threadIdx.x + s]);
-        __syncthreads();
-    }
-    const double r = sh[0];
-    __syncthreads();
-    return r;
-}
-
 // Reductions over one molecule's matrix run in BPART workgroups per molecule
 // (grid BPART x nmol), each writing its partial to part[(m * BPART + p) * w
 // + v]; a finishing kernel (one thread per molecule) adds the partials in
@@ -96,14 +169,18 @@ __global__ __launch_bounds__(256) void bgersh_part_kernel(const long* __restrict
     const int n = nn[m], ld = pld[m];
     const double* F = F0 + poff[m];
     double mn = 1e300, mx = -1e300, tr = 0.0;
-    for (int i = p * 256 + threadIdx.x; i < n; i += BPART * 256) {
+    // a wavefront per row (F is symmetric); a thread per column walked the
+    // matrix with one workgroup at n = 250, 100 us
+    const int lane = threadIdx.x & 63;
+    for (int i = p * 4 + (threadIdx.x >> 6); i < n; i += BPART * 4) {
         double off = 0.0;
-        for (int j = 0; j < n; j++) off += fabs(F[(long)j * ld + i]);
+        for (int j = lane; j < n; j += 64) off += fabs(F[(long)i * ld + j]);
+        for (int w = 32; w > 0; w >>= 1) off += __shfl_xor(off, w, 64);
         const double dg = F[(long)i * ld + i];
         off -= fabs(dg);
         mn = fmin(mn, dg - off);
         mx = fmax(mx, dg + off);
-        tr += dg;
+        if (lane == 0) tr += dg;
     }
     mn = block_reduce(mn, sh, [](double a, double b) { return fmin(a, b); });
     mx = block_reduce(mx, sh, [](double a, double b) { return fmax(a, b); });
@@ -139,7 +216,7 @@ __global__ void bgersh_fin_kernel(int nmol, const int* __restrict__ nn, const in
     coef[2 * m + 1] = lambda * mu / n + no / n;
 }
 
-// D0 = coef0 F + coef1 I on the n x n block, zero padding
+// D0 = coef0 (F + F^T)/2 + coef1 I on the n x n block, zero padding
 __global__ void bpurif_init_kernel(const long* __restrict__ poff, const int* __restrict__ nn,
                                    const int* __restrict__ pld, const int* __restrict__ skip,
                                    const double* __restrict__ coef, const double* __restrict__ F0,
@@ -153,7 +230,7 @@ __global__ void bpurif_init_kernel(const long* __restrict__ poff, const int* __r
     double* D = D0 + poff[m];
     for (long k = (long)blockIdx.x * blockDim.x + threadIdx.x; k < (long)ld * ld; k += (long)gridDim.x * blockDim.x) {
         const int i = (int)(k / ld), j = (int)(k - (long)i * ld);
-        D[k] = (i < n && j < n) ? a * F[k] + (i == j ? dshift : 0.0) : 0.0;
+        D[k] = (i < n && j < n) ? a * (0.5 * (F[k] + F[(long)j * ld + i])) + (i == j ? dshift : 0.0) : 0.0;
     }
 }
 
@@ -239,6 +316,48 @@ __global__ void bpurif_update_kernel(const long* __restrict__ poff, const int* _
     for (long k = (long)blockIdx.x * blockDim.x + threadIdx.x; k < (long)ld * ld; k += (long)gridDim.x * blockDim.x) {
         if (c < 0.5) D[k] = ((1.0 - 2.0 * c) * D[k] + (1.0 + c) * D2[k] - D3[k]) / (1.0 - c);
         else D[k] = ((1.0 + c) * D2[k] - D3[k]) / c;
+    }
+}
+
+// The same after bpurif_product_kernel: every workgroup adds up the molecule's
+// partials (in one fixed order), and the first one records the end of the
+// iterations, so a purification iteration is three launches.
+__global__ __launch_bounds__(256) void bpurif_step_kernel(const long* __restrict__ poff, const int* __restrict__ pld,
+                                                          const int* __restrict__ skip, int* __restrict__ iters,
+                                                          const double* __restrict__ part, int mtiles, double tol,
+                                                          int* host_iters, double* __restrict__ D0, const double* __restrict__ D20,
+                                                          const double* __restrict__ D30, int it)
+{
+    __shared__ double sh[256];
+    const int m = blockIdx.y;
+    // a molecule that ends at `it` still takes this update: its flag may be
+    // set already by the time a workgroup reads it
+    if ((skip && skip[m]) || (iters[m] >= 0 && iters[m] != it)) return;
+    const int ld = pld[m], nt = tri_tiles(ld);
+    double e = 0.0, t2 = 0.0, t1 = 0.0;
+    for (int k = threadIdx.x; k < nt; k += 256) {
+        const double* p = part + ((long)m * mtiles + k) * 3;
+        e += p[0];
+        t2 += p[1];
+        t1 += p[2];
+    }
+    auto add = [](double a, double b) { return a + b; };
+    e = block_reduce(e, sh, add);
+    t2 = block_reduce(t2, sh, add);
+    t1 = block_reduce(t1, sh, add);
+    if (blockIdx.x == 0 && threadIdx.x == 0 && sqrt(e) < tol) {
+        iters[m] = it;
+        if (host_iters) __hip_atomic_store(host_iters + m, it, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+    }
+    const double c = t1 / t2;
+    double2* D = (double2*)(D0 + poff[m]);
+    const double2* D2 = (const double2*)(D20 + poff[m]);
+    const double2* D3 = (const double2*)(D30 + poff[m]);
+    const double x = c < 0.5 ? (1.0 - 2.0 * c) / (1.0 - c) : 0.0, r = c < 0.5 ? 1.0 / (1.0 - c) : 1.0 / c;
+    const double y = (1.0 + c) * r;
+    for (long k = (long)blockIdx.x * 256 + threadIdx.x; k < (long)ld * ld / 2; k += (long)gridDim.x * 256) {
+        const double2 d = D[k], d2 = D2[k], d3 = D3[k];
+        D[k] = make_double2(x * d.x + y * d2.x - r * d3.x, x * d.y + y * d2.y - r * d3.y);
     }
 }
 
@@ -352,6 +471,12 @@ int gtf_bgemm(hipStream_t st, const BatchLayout& L, const int* skip, const int* 
               const double* B, double* C, int transB, const int* fp32)
 {
     if (L.nmol <= 0) return 0;
+    if (transB && !fp32 && L.maxpld <= ROWS_MAX_LD) {
+        dim3 tiles(L.maxpld / ROWS_T, L.maxpld / ROWS_T, L.nmol);
+        bgemm_rows_kernel<<<tiles, ROWS_THREADS, 0, st>>>(L.poff, L.pld, skip, done, A, B, C);
+        GTF_CHECK(hipGetLastError());
+        return 0;
+    }
     dim3 grid(L.maxpld / GEMM_GT, L.maxpld / GEMM_GT, L.nmol);
     if (transB) bgemm_kernel<1><<<grid, 256, 0, st>>>(L.poff, L.pld, skip, done, fp32, A, B, C);
     else bgemm_kernel<0><<<grid, 256, 0, st>>>(L.poff, L.pld, skip, done, fp32, A, B, C);
@@ -404,6 +529,23 @@ int gtf_bpurif_update(hipStream_t st, const BatchLayout& L, const int* skip, con
 {
     bpurif_update_kernel<<<per_mol_grid(L.maxpld * L.maxpld, L.nmol), 256, 0, st>>>(L.poff, L.pld, skip, iters, stats,
                                                                                   D, D2, D3, it);
+    GTF_CHECK(hipGetLastError());
+    return 0;
+}
+
+size_t gtf_bpurif_part(int nmol, int maxpld) { return (size_t)nmol * tri_tiles(maxpld) * 3; }
+
+int gtf_bpurif_iterate(hipStream_t st, const BatchLayout& L, const int* skip, int* iters, double* part, double tol,
+                       double* D, double* D2, double* D3, int it, int* host_iters)
+{
+    const int mt = tri_tiles(L.maxpld);
+    const dim3 grid(mt, L.nmol);
+    bpurif_product_kernel<false><<<grid, ROWS_THREADS, 0, st>>>(L.poff, L.pld, skip, iters, D, D, D2, part, mt);
+    GTF_CHECK(hipGetLastError());
+    bpurif_product_kernel<true><<<grid, ROWS_THREADS, 0, st>>>(L.poff, L.pld, skip, iters, D, D2, D3, part, mt);
+    GTF_CHECK(hipGetLastError());
+    bpurif_step_kernel<<<per_mol_grid(L.maxpld * L.maxpld / 4, L.nmol), 256, 0, st>>>(L.poff, L.pld, skip, iters, part,
+                                                                                     mt, tol, host_iters, D, D2, D3, it);
     GTF_CHECK(hipGetLastError());
     return 0;
 }

@@ -189,3 +189,66 @@ __device__ __forceinline__ void gemm_tile(int ld, const double* __restrict__ A, 
     if constexpr (F32) gemm_tile_f32<TRANSB>(ld, A, B, C, row0, col0);
     else gemm_tile_f64<TRANSB>(ld, A, B, C, row0, col0);
 }
+
+// A 32 x 32 tile of C = A * B^T by ROWS_W wavefronts that take every ROWS_W-th
+// 16-deep K block, straight from global memory to the FP64 MFMA's operands, and
+// add their sums in LDS.  A lane holds four consecutive k of its row (k = k0 +
+// 4 (lane / 16) + e for the e-th MFMA; the order of k is free as long as A and B
+// agree), so a row's 128-byte line is used whole and 8 loads of 1 KB feed 16
+// MFMAs.  No LDS in the loop and no barrier: at n = 250 the 64 x 64 LDS tiles
+// ran 16 workgroups of 16 K blocks, 14.6 us a product, and at n = 846 196
+// workgroups on 256 CUs, 45 us.
+#define ROWS_T 32
+#define ROWS_W 8
+#define ROWS_THREADS (64 * ROWS_W)
+// A * B^T products take these tiles up to this leading dimension; beyond it the
+// 64 x 64 LDS tiles reuse an operand twice as often and fill the chip as well
+// (ld 256: 7 against 15 us a product, 896: 54 against 45)
+#define ROWS_MAX_LD 512
+__device__ __forceinline__ void rows_tile(int ld, const double* __restrict__ A, const double* __restrict__ B, int row0,
+                                          int col0, double (*red)[ROWS_T * ROWS_T])
+{
+    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, li = lane & 15, lk = lane >> 4;
+    const double* pa = A + (long)(row0 + li) * ld + 4 * lk;
+    const double* pb = B + (long)(col0 + li) * ld + 4 * lk;
+    const long half = 16L * ld;
+    gtf_double4_t acc[2][2];
+    for (int i = 0; i < 2; i++)
+        for (int j = 0; j < 2; j++)
+            for (int r = 0; r < 4; r++) acc[i][j][r] = 0.0;
+    gtf_double4_t a[2], b[2], na[2], nb[2];
+    auto load = [&](gtf_double4_t(&x)[2], gtf_double4_t(&y)[2], int k) {
+        for (int t = 0; t < 2; t++) {
+            x[t] = *(const gtf_double4_t*)(pa + t * half + k);
+            y[t] = *(const gtf_double4_t*)(pb + t * half + k);
+        }
+    };
+    auto mul = [&](const gtf_double4_t(&x)[2], const gtf_double4_t(&y)[2]) {
+        for (int e = 0; e < 4; e++)
+            for (int i = 0; i < 2; i++)
+                for (int j = 0; j < 2; j++)
+                    acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(x[i][e], y[j][e], acc[i][j], 0, 0, 0);
+    };
+    const int step = 16 * ROWS_W;
+    int k = 16 * w;
+    if (k < ld) load(a, b, k);
+    for (; k + step < ld; k += 2 * step) {
+        load(na, nb, k + step);
+        mul(a, b);
+        if (k + 2 * step < ld) load(a, b, k + 2 * step);
+        mul(na, nb);
+    }
+    if (k < ld) mul(a, b);
+    for (int i = 0; i < 2; i++)
+        for (int j = 0; j < 2; j++)
+            for (int r = 0; r < 4; r++) red[w][(i * 16 + lk + 4 * r) * ROWS_T + j * 16 + li] = acc[i][j][r];
+    __syncthreads();
+    for (int q = threadIdx.x; q < ROWS_T * ROWS_T; q += ROWS_THREADS) {
+        double v[ROWS_W];
+        for (int x = 0; x < ROWS_W; x++) v[x] = red[x][q];
+        for (int x = 1; x < ROWS_W; x *= 2)
+            for (int y = 0; y < ROWS_W; y += 2 * x) v[y] += v[y + x];
+        red[0][q] = v[0];
+    }
+    __syncthreads();
+}

@@ -17,12 +17,27 @@ __global__ __launch_bounds__(256) void dgemm_mfma_kernel(int ld, const double* _
     gemm_tile<TRANSB, F32>(ld, A, B, C, blockIdx.y * GEMM_GT, blockIdx.x * GEMM_GT);
 }
 
+__global__ __launch_bounds__(ROWS_THREADS) void dgemm_rows_kernel(int ld, const double* __restrict__ A,
+                                                         const double* __restrict__ B, double* __restrict__ C)
+{
+    __shared__ double red[ROWS_W][ROWS_T * ROWS_T];
+    const int row0 = blockIdx.y * ROWS_T, col0 = blockIdx.x * ROWS_T;
+    rows_tile(ld, A, B, row0, col0, red);
+    for (int k = threadIdx.x; k < ROWS_T * ROWS_T; k += ROWS_THREADS)
+        C[(long)(row0 + k / ROWS_T) * ld + col0 + k % ROWS_T] = red[0][k];
+}
+
 int gtf_gemm(hipStream_t st, int n, int ld, const double* A, const double* B, double* C, int transB, int fp32)
 {
     (void)n;
     if (ld % GEMM_GT != 0) {
         fprintf(stderr, "gtf_gemm: leading dimension %d is not a multiple of %d\n", ld, GEMM_GT);
         return -1;
+    }
+    if (transB && !fp32 && ld <= ROWS_MAX_LD) {
+        dgemm_rows_kernel<<<dim3(ld / ROWS_T, ld / ROWS_T), ROWS_THREADS, 0, st>>>(ld, A, B, C);
+        GTF_CHECK(hipGetLastError());
+        return 0;
     }
     dim3 grid(ld / GEMM_GT, ld / GEMM_GT);
     if (fp32) {

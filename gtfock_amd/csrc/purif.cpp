@@ -25,6 +25,8 @@
 struct purif_dev {
     hipStream_t stream = nullptr;
     hipEvent_t e0 = nullptr, e1 = nullptr;
+    hipEvent_t group[2] = {nullptr, nullptr};  // ends of PURIF_CHECK purification iterations
+    int* h_end = nullptr;  // pinned: the iteration at which the purification ended, or -1
     PinnedStage stage;  // F, D in and out
     int n = 0, ld = 0;
     double *F = nullptr, *D = nullptr, *D2 = nullptr, *D3 = nullptr, *X = nullptr, *S = nullptr;
@@ -52,7 +54,7 @@ struct purif_dev {
     long *d_off = nullptr, *d_poff = nullptr;
     int *d_n = nullptr, *d_pld = nullptr, *d_nocc = nullptr, *d_iters = nullptr, *d_low = nullptr,
         *d_lowit = nullptr;
-    double *d_part = nullptr, *d_pcoef = nullptr, *d_stats = nullptr;
+    double *d_part = nullptr, *d_pcoef = nullptr, *d_stats = nullptr, *ppart = nullptr;
     BatchLayout layout() const { return BatchLayout{1, n, ld, d_off, d_n, d_poff, d_pld, d_part, d_pcoef}; }
 };
 
@@ -151,7 +153,10 @@ purif_t* create_purif(BasisSet_t basis, int nprow_purif, int npcol_purif, int np
     d->ld = ((n + 63) / 64) * 64;
     const size_t m = (size_t)d->ld * d->ld;
     bool ok = hipStreamCreate(&d->stream) == hipSuccess && hipEventCreate(&d->e0) == hipSuccess &&
-              hipEventCreate(&d->e1) == hipSuccess;
+              hipEventCreate(&d->e1) == hipSuccess &&
+              hipEventCreateWithFlags(&d->group[0], hipEventDisableTiming) == hipSuccess &&
+              hipEventCreateWithFlags(&d->group[1], hipEventDisableTiming) == hipSuccess &&
+              hipHostMalloc((void**)&d->h_end, sizeof(int), hipHostMallocDefault) == hipSuccess;
     double** bufs[] = {&d->F, &d->D, &d->D2, &d->D3, &d->X, &d->S, &d->W, &d->W2};
     for (double** b : bufs) ok = ok && hipMalloc((void**)b, sizeof(double) * m) == hipSuccess;
     ok = ok && hipMalloc((void**)&d->evecs, sizeof(double) * m * MAX_DIIS) == hipSuccess;
@@ -166,6 +171,7 @@ purif_t* create_purif(BasisSet_t basis, int nprow_purif, int npcol_purif, int np
     ok = ok && hipMalloc((void**)&d->d_part, sizeof(double) * BPART * BMAX_DOTS) == hipSuccess;
     ok = ok && hipMalloc((void**)&d->d_pcoef, sizeof(double) * 2) == hipSuccess;
     ok = ok && hipMalloc((void**)&d->d_stats, sizeof(double) * 3) == hipSuccess;
+    ok = ok && hipMalloc((void**)&d->ppart, sizeof(double) * gtf_bpurif_part(1, d->ld)) == hipSuccess;
     if (!ok) { destroy_purif(p); return nullptr; }
     {
         const long zero = 0;
@@ -193,11 +199,14 @@ void destroy_purif(purif_t* p)
         if (d->stream) (void)hipStreamSynchronize(d->stream);
         void* bufs[] = {d->F, d->D, d->D2, d->D3, d->X, d->S, d->W, d->W2, d->evecs, d->Fvecs,
                         d->scal, d->coef, d->partial, d->oz_mem, d->d_off, d->d_poff, d->d_n, d->d_pld,
-                        d->d_nocc, d->d_iters, d->d_low, d->d_lowit, d->d_part, d->d_pcoef, d->d_stats};
+                        d->d_nocc, d->d_iters, d->d_low, d->d_lowit, d->d_part, d->d_pcoef, d->d_stats, d->ppart};
         for (void* b : bufs)
             if (b) (void)hipFree(b);
         if (d->e0) (void)hipEventDestroy(d->e0);
         if (d->e1) (void)hipEventDestroy(d->e1);
+        for (hipEvent_t g : d->group)
+            if (g) (void)hipEventDestroy(g);
+        if (d->h_end) (void)hipHostFree(d->h_end);
         if (d->stream) (void)hipStreamDestroy(d->stream);
         delete d;
     }
@@ -234,33 +243,57 @@ static int purify(purif_t* p, double* F_block, double* D_block, int* iters)
     o.done = d->d_iters;
     o.sel = d->d_low;
     int it_done = -1, it = 0;
-    for (it = 0; it < 200; it++) {
-        if (gtf_bgemm(d->stream, L, nullptr, d->d_iters, d->D, d->D, d->D2, 0, d->d_low) ||
-            gtf_bgemm(d->stream, L, nullptr, d->d_iters, d->D, d->D2, d->D3, 0, d->d_low))
-            return -1;
-        if (mode == GTF_LOW_SPLIT && gtf_oz_square_cube(d->stream, o, d->oz, d->D, d->D2, d->D3)) return -1;
-        if (gtf_bpurif_stats(d->stream, L, nullptr, d->D, d->D2, d->D3, d->d_iters, d->d_stats, it, 1e-11, d->d_low,
-                             d->low_until, d->d_lowit))
-            return -1;
-        if (gtf_bpurif_update(d->stream, L, nullptr, d->d_iters, d->d_stats, d->D, d->D2, d->D3, it)) return -1;
-        if (it % PURIF_CHECK == PURIF_CHECK - 1) {
-            PD_CHECK(hipMemcpyAsync(&it_done, d->d_iters, sizeof(int), hipMemcpyDeviceToHost, d->stream));
-            PD_CHECK(hipStreamSynchronize(d->stream));
-            if (it_done >= 0) break;
+    if (mode == GTF_LOW_FP64) {
+        // The last kernel of an iteration writes the end to pinned host memory,
+        // so the host looks without stopping the stream; it stays at most two
+        // groups of PURIF_CHECK iterations ahead (launches after the end return
+        // at once).  A copy and a synchronisation every PURIF_CHECK iterations
+        // left the GPU idle for about one iteration in four at n = 250.
+        volatile int* end = d->h_end;
+        *end = -1;
+        for (it = 0; it < 200 && *end < 0; it++) {
+            if (gtf_bpurif_iterate(d->stream, L, nullptr, d->d_iters, d->ppart, 1e-11, d->D, d->D2, d->D3, it, d->h_end))
+                return -1;
+            if (it % PURIF_CHECK == PURIF_CHECK - 1) {
+                const int g = it / PURIF_CHECK;
+                PD_CHECK(hipEventRecord(d->group[g % 2], d->stream));
+                if (g > 0) PD_CHECK(hipEventSynchronize(d->group[(g + 1) % 2]));
+            }
+        }
+    } else {
+        for (it = 0; it < 200; it++) {
+            if (gtf_bgemm(d->stream, L, nullptr, d->d_iters, d->D, d->D, d->D2, 0, d->d_low) ||
+                gtf_bgemm(d->stream, L, nullptr, d->d_iters, d->D, d->D2, d->D3, 0, d->d_low) ||
+                (mode == GTF_LOW_SPLIT && gtf_oz_square_cube(d->stream, o, d->oz, d->D, d->D2, d->D3)) ||
+                gtf_bpurif_stats(d->stream, L, nullptr, d->D, d->D2, d->D3, d->d_iters, d->d_stats, it, 1e-11, d->d_low,
+                                 d->low_until, d->d_lowit) ||
+                gtf_bpurif_update(d->stream, L, nullptr, d->d_iters, d->d_stats, d->D, d->D2, d->D3, it))
+                return -1;
+            if (it % PURIF_CHECK == PURIF_CHECK - 1) {
+                PD_CHECK(hipMemcpyAsync(&it_done, d->d_iters, sizeof(int), hipMemcpyDeviceToHost, d->stream));
+                PD_CHECK(hipStreamSynchronize(d->stream));
+                if (it_done >= 0) break;
+            }
         }
     }
-    int lowit = 0;
-    PD_CHECK(hipMemcpyAsync(&it_done, d->d_iters, sizeof(int), hipMemcpyDeviceToHost, d->stream));
-    PD_CHECK(hipMemcpyAsync(&lowit, d->d_lowit, sizeof(int), hipMemcpyDeviceToHost, d->stream));
+    // D = X D X (pscf/purif.c:469-476)
+    if (gtf_gemm(d->stream, d->n, d->ld, d->X, d->D, d->W, 1, 0) ||
+        gtf_gemm(d->stream, d->n, d->ld, d->W, d->X, d->D, 1, 0))
+        return -1;
     PD_CHECK(hipEventRecord(d->e1, d->stream));
-    PD_CHECK(hipEventSynchronize(d->e1));
+    int lowit = 0;
+    if (mode == GTF_LOW_FP64) {
+        if (d2h(d, D_block, d->D, p->ldx)) return -1;
+        it_done = *d->h_end;
+    } else {
+        PD_CHECK(hipMemcpyAsync(&it_done, d->d_iters, sizeof(int), hipMemcpyDeviceToHost, d->stream));
+        PD_CHECK(hipMemcpyAsync(&lowit, d->d_lowit, sizeof(int), hipMemcpyDeviceToHost, d->stream));
+        if (d2h(d, D_block, d->D, p->ldx)) return -1;
+    }
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, d->e0, d->e1);
     p->timedgemm += 1e-3 * ms;
     d->low_iters = mode != 0 ? (lowit > 0 ? lowit : (it_done >= 0 ? it_done + 1 : 200)) : 0;
-    // D = X D X (pscf/purif.c:469-476)
-    if (gemm_pair(d, d->X, d->D, d->W, 1, d->W, d->X, d->D, 1, &p->timedgemm)) return -1;
-    if (d2h(d, D_block, d->D, p->ldx)) return -1;
     *iters = it_done >= 0 ? it_done : 200;
     return 0;
 }
