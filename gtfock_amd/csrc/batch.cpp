@@ -291,7 +291,7 @@ int GtfBatch::scf_setup(const GtfBatch* from, const int* from_idx)
         if (carried(m)) continue;
         const int ns = s.mol_nshells[m];
         om.push_back(OneelMol{nblk, s.mol_shell_off[m], ns, atom_off[m], bases[m]->natoms, n[m], off[m]});
-        nblk += (ns * ns + 63) / 64;
+        nblk += gtf_oneel_blocks(ns, nmol);
     }
     const int nom = (int)om.size();
     om.push_back(OneelMol{nblk, 0, 0, 0, 0, 0, 0});

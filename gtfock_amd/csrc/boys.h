@@ -78,13 +78,15 @@ __device__ __forceinline__ void boys_eval8(double T, double* F, const double* __
     }
 }
 
-// runtime-order variant for the one-electron kernels (m <= mmax <= 8)
-__device__ inline void boys_eval_rt(int mmax, double T, double* F, const double* __restrict__ tab)
+// F_0..F_M(T) for the one-electron kernels (M <= 8) from the full table
+template <int M>
+__device__ __forceinline__ void boys_eval(double T, double* F, const double* __restrict__ tab)
 {
+    const double e = M > 0 ? exp(-T) : 0.0;
     if (T < BOYS_TMAX) {
-        int i = (int)(T * BOYS_INV_DELTA + 0.5);
-        double dt = i * BOYS_DELTA - T;
-        const double* row = tab + i * BOYS_NCOL + mmax;
+        const int i = (int)(T * BOYS_INV_DELTA + 0.5);
+        const double dt = i * BOYS_DELTA - T;
+        const double* row = tab + i * BOYS_NCOL + M;
         double f = row[6];
         f = row[5] + dt * (1.0 / 6.0) * f;
         f = row[4] + dt * (1.0 / 5.0) * f;
@@ -92,12 +94,16 @@ __device__ inline void boys_eval_rt(int mmax, double T, double* F, const double*
         f = row[2] + dt * (1.0 / 3.0) * f;
         f = row[1] + dt * (1.0 / 2.0) * f;
         f = row[0] + dt * f;
-        F[mmax] = f;
-        double e = exp(-T);
-        for (int m = mmax - 1; m >= 0; --m) F[m] = (2.0 * T * F[m + 1] + e) / (2 * m + 1);
+        F[M] = f;
+        static_for<0, M>([&](auto k) {
+            constexpr int m = M - 1 - decltype(k)::value;
+            F[m] = (2.0 * T * F[m + 1] + e) / (2 * m + 1);
+        });
     } else {
         F[0] = 0.88622692545275801365 / sqrt(T);
-        double e = exp(-T);
-        for (int m = 1; m <= mmax; ++m) F[m] = ((2 * m - 1) * F[m - 1] - e) / (2.0 * T);
+        static_for<1, M + 1>([&](auto k) {
+            constexpr int m = decltype(k)::value;
+            F[m] = ((2 * m - 1) * F[m - 1] - e) / (2.0 * T);
+        });
     }
 }

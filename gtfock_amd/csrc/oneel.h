@@ -4,7 +4,10 @@
 
 int gtf_oneel(hipStream_t st, const BasisView& b, const double* boys, int ld, double* S, double* T, double* V);
 
-// one molecule of a batched one-electron launch: its first 64-thread block,
+// workgroups of 64 threads for a molecule of nshells, of nmol in the launch
+int gtf_oneel_blocks(int nshells, int nmol);
+
+// one molecule of a batched one-electron launch: its first workgroup,
 // shell and atom offsets into the shared basis arrays, sizes, the leading
 // dimension of its matrices and their offset in S / T / V
 struct OneelMol {

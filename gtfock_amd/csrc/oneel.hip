@@ -1,152 +1,272 @@
 // oneel.hip -- overlap, kinetic and nuclear-attraction matrices by the
-// McMurchie-Davidson scheme (one thread per ordered shell pair; setup work,
-// replaces pfock/one_electron.c:28-119 and the closed OED library):
-//   S_ab = E^x_0 E^y_0 E^z_0 (pi/p)^(3/2)
-//   T_ab = sum over directions of  -2b^2 S_{i,j+2} + b(2j+1) S_{ij} - j(j-1)/2 S_{i,j-2}
+// McMurchie-Davidson scheme (setup work, replaces
+// pfock/one_electron.c:28-119 and the closed OED library):
+//   S_ab = s^x_ab s^y_ab s^z_ab, s the one-dimensional overlaps
+//   T_ab = sum over directions of  -2b^2 s_{i,j+2} + b(2j+1) s_{ij} - j(j-1)/2 s_{i,j-2}
 //   V_ab = -sum_C Z_C (2 pi / p) sum_tuv E^{ab}_{tuv} R_{tuv}(p, P - C)
+//
+// One wavefront per unordered shell pair, in code compiled for its two angular
+// momenta.  Its lanes are PP primitive pairs x 64 / PP shares of the nuclei
+// (PP the power of two that holds the pair's primitive pairs, at most 64); a
+// lane sums R over its nuclei, contracts once, and the 64 partial blocks are
+// added with lane shuffles.  Bound by latency: few wavefronts live (the d
+// blocks take most of the registers) and little work in each.  One thread per
+// ordered pair with sizes known at run time had its tables in scratch memory,
+// and a wavefront waited for the pair with the most primitives: 13.3 ms of the
+// 35.2 ms set-up of C24H12 (180 shells, 36 nuclei), which takes 23.5 ms now.
 #include "boys.h"
+#include "eri_md.h"
 #include "gtf_internal.h"
 #include "oneel.h"
 
-#define LKIN (GTF_LMAX + 2)
+namespace {
 
-// S, T, V of ordered shell pair pid = A * nshells + B of one molecule
-__device__ __forceinline__ void oneel_pair(const BasisView& b, const double* __restrict__ boys, int ld,
-                                           double* __restrict__ S, double* __restrict__ Tk, double* __restrict__ V,
-                                           int pid)
+// cartesian exponents of component c of order l
+__host__ __device__ constexpr int cart_x(int l, int c) { return herm_t((l == 0 ? 0 : nherm(l - 1)) + c); }
+__host__ __device__ constexpr int cart_y(int l, int c) { return herm_u((l == 0 ? 0 : nherm(l - 1)) + c); }
+__host__ __device__ constexpr int cart_z(int l, int c) { return herm_v((l == 0 ? 0 : nherm(l - 1)) + c); }
+
+// a primitive pair of the two shells
+struct PrimPair {
+    double a, b, p, cc;
+    double P[3], PA[3], PB[3], K[3];  // K: exp(-mu AB_d^2)
+};
+
+__device__ __forceinline__ PrimPair prim_pair(const BasisView& b, int A, int B, int k)
 {
-    if (pid >= b.nshells * b.nshells) return;
-    const int A = pid / b.nshells, B = pid % b.nshells;
-    const int la = b.L[A], lb = b.L[B], lab = la + lb;
-    const double* CA = b.center + 3 * A;
-    const double* CB = b.center + 3 * B;
-    double AB2 = 0.0;
-    for (int d = 0; d < 3; d++) AB2 += (CA[d] - CB[d]) * (CA[d] - CB[d]);
-    const int nca = ncart(la), ncb = ncart(lb);
-    double sc[36], tc[36], vc[36];
-    for (int k = 0; k < 36; k++) sc[k] = tc[k] = vc[k] = 0.0;
-    const int ca0 = la == 0 ? 0 : nherm(la - 1), cb0 = lb == 0 ? 0 : nherm(lb - 1);
-    for (int i = 0; i < b.nprim[A]; i++)
-        for (int j = 0; j < b.nprim[B]; j++) {
-            const double a = b.alpha[b.poff[A] + i], bb = b.alpha[b.poff[B] + j];
-            const double p = a + bb, mu = a * bb / p;
-            const double cc = b.coef[b.poff[A] + i] * b.coef[b.poff[B] + j];
-            double P[3];
-            // E1[d][x][y][t] for x <= la, y <= lb + 2
-            double E1[3][GTF_LMAX + 1][LKIN + 1][GTF_LMAX + LKIN + 2];
-            for (int d = 0; d < 3; d++) {
-                P[d] = (a * CA[d] + bb * CB[d]) / p;
-                const double XPA = P[d] - CA[d], XPB = P[d] - CB[d];
-                for (int x = 0; x <= GTF_LMAX; x++)
-                    for (int y = 0; y <= LKIN; y++)
-                        for (int t = 0; t < GTF_LMAX + LKIN + 2; t++) E1[d][x][y][t] = 0.0;
-                E1[d][0][0][0] = exp(-mu * (CA[d] - CB[d]) * (CA[d] - CB[d]));
-                for (int x = 0; x < la; x++)
-                    for (int t = 0; t <= x + 1; t++) {
-                        double v = XPA * E1[d][x][0][t] + (t + 1) * E1[d][x][0][t + 1];
-                        if (t > 0) v += E1[d][x][0][t - 1] / (2.0 * p);
-                        E1[d][x + 1][0][t] = v;
-                    }
-                for (int y = 0; y < lb + 2; y++)
-                    for (int x = 0; x <= la; x++)
-                        for (int t = 0; t <= x + y + 1; t++) {
-                            double v = XPB * E1[d][x][y][t] + (t + 1) * E1[d][x][y][t + 1];
-                            if (t > 0) v += E1[d][x][y][t - 1] / (2.0 * p);
-                            E1[d][x][y + 1][t] = v;
-                        }
+    const int nb = b.nprim[B], i = k / nb, j = k - i * nb;
+    PrimPair q;
+    q.a = b.alpha[b.poff[A] + i];
+    q.b = b.alpha[b.poff[B] + j];
+    q.p = q.a + q.b;
+    q.cc = b.coef[b.poff[A] + i] * b.coef[b.poff[B] + j];
+    const double mu = q.a * q.b / q.p;
+    for (int d = 0; d < 3; d++) {
+        const double ca = b.center[3 * A + d], cb = b.center[3 * B + d];
+        q.P[d] = (q.a * ca + q.b * cb) / q.p;
+        q.PA[d] = q.P[d] - ca;
+        q.PB[d] = q.P[d] - cb;
+        q.K[d] = exp(-mu * (ca - cb) * (ca - cb));
+    }
+    return q;
+}
+
+// cartesian block -> spherical, summed over the wavefront; lane e of the
+// first ones returns element e
+template <int LA, int LB>
+__device__ __forceinline__ double sph_sum(const double (&cart)[ncart(LA) * ncart(LB)], int lane)
+{
+    double mine = 0.0;
+    static_for<0, nsph(LA)>([&](auto as_) {
+        static_for<0, nsph(LB)>([&](auto bs_) {
+            constexpr int as = decltype(as_)::value, bs = decltype(bs_)::value;
+            double v = 0.0;
+            static_for<0, ncart(LA)>([&](auto ia_) {
+                static_for<0, ncart(LB)>([&](auto ib_) {
+                    constexpr int ia = decltype(ia_)::value, ib = decltype(ib_)::value;
+                    constexpr double w = sph_coef(LA, as, ia) * sph_coef(LB, bs, ib);
+                    if constexpr (w != 0.0) v += w * cart[ia * ncart(LB) + ib];
+                });
+            });
+            for (int m = 32; m; m >>= 1) v += __shfl_xor(v, m);
+            if (lane == as * nsph(LB) + bs) mine = v;
+        });
+    });
+    return mine;
+}
+
+// S, T, V of shells A, B (LA >= LB), both triangles
+template <int LA, int LB>
+__device__ __forceinline__ void oneel_block(const BasisView& b, const double* __restrict__ boys, int ld,
+                                            double* __restrict__ S, double* __restrict__ Tk, double* __restrict__ V,
+                                            int A, int B)
+{
+    constexpr int NCA = ncart(LA), NCB = ncart(LB), L = LA + LB, HL = nherm(L);
+    const int lane = threadIdx.x & 63;
+    const int np = b.nprim[A] * b.nprim[B];
+    int lp = 0;
+    while (lp < 6 && (1 << lp) < np) lp++;
+    const int pp = 1 << lp, share = lane >> lp, nshare = 64 >> lp;
+    const bool writes = lane < nsph(LA) * nsph(LB);
+    const int as = lane / nsph(LB), bs = lane - as * nsph(LB);
+    const long k1 = (long)(b.fstart[A] + as) * ld + b.fstart[B] + bs;
+    const long k2 = (long)(b.fstart[B] + bs) * ld + b.fstart[A] + as;
+    {
+        double vc[NCA * NCB];
+        static_for<0, NCA * NCB>([&](auto e_) { vc[decltype(e_)::value] = 0.0; });
+        for (int k = lane & (pp - 1); k < np; k += pp) {
+            const PrimPair q = prim_pair(b, A, B, k);
+            // Hermite Coulomb R_{tuv}(p, P - C), summed with -Z_C
+            double Rs[HL];
+            static_for<0, HL>([&](auto h_) { Rs[decltype(h_)::value] = 0.0; });
+            for (int c = share; c < b.natoms; c += nshare) {
+                const double X = q.P[0] - b.atom_xyz[3 * c], Y = q.P[1] - b.atom_xyz[3 * c + 1],
+                             Z = q.P[2] - b.atom_xyz[3 * c + 2], z = b.atom_Z[c];
+                double F[L + 1], R[HL];
+                boys_eval<L>(q.p * (X * X + Y * Y + Z * Z), F, boys);
+                hermite_R<L, double>(R, F, 1.0, -2.0 * q.p, X, Y, Z);
+                static_for<0, HL>([&](auto h_) { Rs[decltype(h_)::value] -= z * R[decltype(h_)::value]; });
             }
-            const double sq = sqrt(M_PI / p);
-            // Hermite Coulomb R_{tuv}(p, P - C) for every nucleus, summed with -Z_C
-            double Rsum[nherm(2 * GTF_LMAX)];
-            for (int h = 0; h < nherm(lab); h++) Rsum[h] = 0.0;
-            for (int c = 0; c < b.natoms; c++) {
-                const double X = P[0] - b.atom_xyz[3 * c], Y = P[1] - b.atom_xyz[3 * c + 1],
-                             Z = P[2] - b.atom_xyz[3 * c + 2];
-                double F[2 * GTF_LMAX + 1];
-                boys_eval_rt(lab, p * (X * X + Y * Y + Z * Z), F, boys);
-                // R^n_{tuv} table, n = 0..lab
-                double R[2 * GTF_LMAX + 1][nherm(2 * GTF_LMAX)];
-                double pw = 1.0;
-                for (int n = 0; n <= lab; n++) {
-                    R[n][0] = pw * F[n];
-                    pw *= -2.0 * p;
-                }
-                for (int k = 1; k <= lab; k++)
-                    for (int n = 0; n <= lab - k; n++)
-                        for (int h = nherm(k - 1); h < nherm(k); h++) {
-                            const int t = herm_t(h), u = herm_u(h), v = herm_v(h);
-                            double r;
-                            if (t > 0) {
-                                r = X * R[n + 1][hidx(t - 1, u, v)];
-                                if (t > 1) r += (t - 1) * R[n + 1][hidx(t - 2, u, v)];
-                            } else if (u > 0) {
-                                r = Y * R[n + 1][hidx(t, u - 1, v)];
-                                if (u > 1) r += (u - 1) * R[n + 1][hidx(t, u - 2, v)];
-                            } else {
-                                r = Z * R[n + 1][hidx(t, u, v - 1)];
-                                if (v > 1) r += (v - 1) * R[n + 1][hidx(t, u, v - 2)];
-                            }
-                            R[n][h] = r;
-                        }
-                for (int h = 0; h < nherm(lab); h++) Rsum[h] -= b.atom_Z[c] * R[0][h];
-            }
-            for (int ia = 0; ia < nca; ia++) {
-                const int ax = herm_t(ca0 + ia), ay = herm_u(ca0 + ia), az = herm_v(ca0 + ia);
-                for (int ib = 0; ib < ncb; ib++) {
-                    const int bx = herm_t(cb0 + ib), by = herm_u(cb0 + ib), bz = herm_v(cb0 + ib);
-                    const int ax_[3] = {ax, ay, az}, bx_[3] = {bx, by, bz};
-                    double s1[3], t1[3];
-                    for (int d = 0; d < 3; d++) {
-                        const int ii = ax_[d], jj = bx_[d];
-                        s1[d] = E1[d][ii][jj][0] * sq;
-                        double t = -2.0 * bb * bb * E1[d][ii][jj + 2][0] * sq + bb * (2 * jj + 1) * s1[d];
-                        if (jj >= 2) t -= 0.5 * jj * (jj - 1) * E1[d][ii][jj - 2][0] * sq;
-                        t1[d] = t;
-                    }
-                    sc[ia * ncb + ib] += cc * s1[0] * s1[1] * s1[2];
-                    tc[ia * ncb + ib] += cc * (t1[0] * s1[1] * s1[2] + s1[0] * t1[1] * s1[2] + s1[0] * s1[1] * t1[2]);
+            // E[d][x][y][t], x <= LA, y <= LB
+            double E[3][LA + 1][LB + 1][L + 1];
+            const double h = 0.5 / q.p;
+            static_for<0, 3>([&](auto d_) {
+                constexpr int d = decltype(d_)::value;
+                E[d][0][0][0] = q.K[d];
+                static_for<0, LA>([&](auto x_) {
+                    constexpr int x = decltype(x_)::value;
+                    static_for<0, x + 2>([&](auto t_) {
+                        constexpr int t = decltype(t_)::value;
+                        double v = 0.0;
+                        if constexpr (t <= x) v += q.PA[d] * E[d][x][0][t];
+                        if constexpr (t + 1 <= x) v += (t + 1) * E[d][x][0][t + 1];
+                        if constexpr (t > 0) v += h * E[d][x][0][t - 1];
+                        E[d][x + 1][0][t] = v;
+                    });
+                });
+                static_for<0, LB>([&](auto y_) {
+                    constexpr int y = decltype(y_)::value;
+                    static_for<0, LA + 1>([&](auto x_) {
+                        constexpr int x = decltype(x_)::value;
+                        static_for<0, x + y + 2>([&](auto t_) {
+                            constexpr int t = decltype(t_)::value;
+                            double v = 0.0;
+                            if constexpr (t <= x + y) v += q.PB[d] * E[d][x][y][t];
+                            if constexpr (t + 1 <= x + y) v += (t + 1) * E[d][x][y][t + 1];
+                            if constexpr (t > 0) v += h * E[d][x][y][t - 1];
+                            E[d][x][y + 1][t] = v;
+                        });
+                    });
+                });
+            });
+            const double w = q.cc * 2.0 * M_PI / q.p;
+            static_for<0, NCA>([&](auto ia_) {
+                static_for<0, NCB>([&](auto ib_) {
+                    constexpr int ia = decltype(ia_)::value, ib = decltype(ib_)::value;
+                    constexpr int ax = cart_x(LA, ia), ay = cart_y(LA, ia), az = cart_z(LA, ia);
+                    constexpr int bx = cart_x(LB, ib), by = cart_y(LB, ib), bz = cart_z(LB, ib);
                     double v = 0.0;
-                    for (int t = 0; t <= ax + bx; t++)
-                        for (int u = 0; u <= ay + by; u++)
-                            for (int w = 0; w <= az + bz; w++)
-                                v += E1[0][ax][bx][t] * E1[1][ay][by][u] * E1[2][az][bz][w] * Rsum[hidx(t, u, w)];
-                    vc[ia * ncb + ib] += cc * 2.0 * M_PI / p * v;
-                }
-            }
+                    static_for<0, ax + bx + 1>([&](auto t_) {
+                        static_for<0, ay + by + 1>([&](auto u_) {
+                            constexpr int t = decltype(t_)::value, u = decltype(u_)::value;
+                            double r = 0.0;
+                            static_for<0, az + bz + 1>([&](auto z_) {
+                                constexpr int zz = decltype(z_)::value;
+                                r += E[2][az][bz][zz] * Rs[hidx(t, u, zz)];
+                            });
+                            v += E[0][ax][bx][t] * E[1][ay][by][u] * r;
+                        });
+                    });
+                    vc[ia * NCB + ib] += w * v;
+                });
+            });
         }
-    const int na = nsph(la), nb = nsph(lb);
-    const int r0 = b.fstart[A], c0 = b.fstart[B];
-    for (int as = 0; as < na; as++)
-        for (int bs = 0; bs < nb; bs++) {
-            double s = 0.0, t = 0.0, v = 0.0;
-            for (int ia = 0; ia < nca; ia++) {
-                const double ta = sph_coef(la, as, ia);
-                if (ta == 0.0) continue;
-                for (int ib = 0; ib < ncb; ib++) {
-                    const double w = ta * sph_coef(lb, bs, ib);
-                    s += w * sc[ia * ncb + ib];
-                    t += w * tc[ia * ncb + ib];
-                    v += w * vc[ia * ncb + ib];
-                }
-            }
-            const long k = (long)(r0 + as) * ld + c0 + bs;
-            S[k] = s;
-            Tk[k] = t;
-            V[k] = v;
+        const double v = sph_sum<LA, LB>(vc, lane);
+        if (writes) {
+            V[k1] = v;
+            if (A != B) V[k2] = v;
         }
+    }
+    double sc[NCA * NCB], tc[NCA * NCB];
+    static_for<0, NCA * NCB>([&](auto e_) { sc[decltype(e_)::value] = tc[decltype(e_)::value] = 0.0; });
+    // no nuclei here: the primitive pairs are over all 64 lanes
+    for (int k = lane; k < np; k += 64) {
+        const PrimPair q = prim_pair(b, A, B, k);
+        const double sq = sqrt(M_PI / q.p), h = 0.5 / q.p;
+        // one-dimensional overlaps s[d][x][y], x <= LA, y <= LB + 2, and
+        // kinetic factors t[d][x][y], y <= LB
+        double s[3][LA + 1][LB + 3], t[3][LA + 1][LB + 1];
+        static_for<0, 3>([&](auto d_) {
+            constexpr int d = decltype(d_)::value;
+            s[d][0][0] = q.K[d] * sq;
+            static_for<0, LA>([&](auto x_) {
+                constexpr int x = decltype(x_)::value;
+                double v = q.PA[d] * s[d][x][0];
+                if constexpr (x > 0) v += x * h * s[d][x - 1][0];
+                s[d][x + 1][0] = v;
+            });
+            static_for<0, LB + 2>([&](auto y_) {
+                constexpr int y = decltype(y_)::value;
+                static_for<0, LA + 1>([&](auto x_) {
+                    constexpr int x = decltype(x_)::value;
+                    double v = q.PB[d] * s[d][x][y];
+                    if constexpr (x > 0) v += x * h * s[d][x - 1][y];
+                    if constexpr (y > 0) v += y * h * s[d][x][y - 1];
+                    s[d][x][y + 1] = v;
+                });
+            });
+            static_for<0, LA + 1>([&](auto x_) {
+                static_for<0, LB + 1>([&](auto y_) {
+                    constexpr int x = decltype(x_)::value, y = decltype(y_)::value;
+                    double v = -2.0 * q.b * q.b * s[d][x][y + 2] + q.b * (2 * y + 1) * s[d][x][y];
+                    if constexpr (y >= 2) v -= 0.5 * y * (y - 1) * s[d][x][y - 2];
+                    t[d][x][y] = v;
+                });
+            });
+        });
+        static_for<0, NCA>([&](auto ia_) {
+            static_for<0, NCB>([&](auto ib_) {
+                constexpr int ia = decltype(ia_)::value, ib = decltype(ib_)::value;
+                constexpr int ax = cart_x(LA, ia), ay = cart_y(LA, ia), az = cart_z(LA, ia);
+                constexpr int bx = cart_x(LB, ib), by = cart_y(LB, ib), bz = cart_z(LB, ib);
+                const double sx = s[0][ax][bx], sy = s[1][ay][by], sz = s[2][az][bz];
+                sc[ia * NCB + ib] += q.cc * sx * sy * sz;
+                tc[ia * NCB + ib] += q.cc * (t[0][ax][bx] * sy * sz + sx * t[1][ay][by] * sz + sx * sy * t[2][az][bz]);
+            });
+        });
+    }
+    const double s = sph_sum<LA, LB>(sc, lane), t = sph_sum<LA, LB>(tc, lane);
+    if (writes) {
+        S[k1] = s;
+        Tk[k1] = t;
+        if (A != B) {
+            S[k2] = s;
+            Tk[k2] = t;
+        }
+    }
 }
 
-__global__ void oneel_kernel(BasisView b, const double* __restrict__ boys, int ld, double* __restrict__ S,
-                             double* __restrict__ Tk, double* __restrict__ V)
+// the pairs blk, blk + nblk, ... of one molecule
+__device__ __forceinline__ void oneel_pairs(const BasisView& b, const double* __restrict__ boys, int ld,
+                                            double* __restrict__ S, double* __restrict__ Tk, double* __restrict__ V,
+                                            int blk, int nblk)
 {
-    oneel_pair(b, boys, ld, S, Tk, V, blockIdx.x * blockDim.x + threadIdx.x);
+    const long npair = (long)b.nshells * (b.nshells + 1) / 2;
+    for (long k = blk; k < npair; k += nblk) {
+        long i = (long)((sqrt(8.0 * (double)k + 1.0) - 1.0) * 0.5);
+        while (i * (i + 1) / 2 > k) i--;
+        while ((i + 1) * (i + 2) / 2 <= k) i++;
+        int A = (int)i, B = (int)(k - i * (i + 1) / 2);
+        if (b.L[A] < b.L[B]) {
+            const int t = A;
+            A = B;
+            B = t;
+        }
+        switch (b.L[A] * (b.L[A] + 1) / 2 + b.L[B]) {
+        case 0: oneel_block<0, 0>(b, boys, ld, S, Tk, V, A, B); break;
+        case 1: oneel_block<1, 0>(b, boys, ld, S, Tk, V, A, B); break;
+        case 2: oneel_block<1, 1>(b, boys, ld, S, Tk, V, A, B); break;
+        case 3: oneel_block<2, 0>(b, boys, ld, S, Tk, V, A, B); break;
+        case 4: oneel_block<2, 1>(b, boys, ld, S, Tk, V, A, B); break;
+        default: oneel_block<2, 2>(b, boys, ld, S, Tk, V, A, B); break;
+        }
+    }
+}
+static_assert(GTF_LMAX == 2, "oneel_pairs lists the pairs of l = 0..2");
+
+}  // namespace
+
+__global__ __launch_bounds__(64) void oneel_kernel(BasisView b, const double* __restrict__ boys, int ld,
+                                                   double* __restrict__ S, double* __restrict__ Tk,
+                                                   double* __restrict__ V)
+{
+    oneel_pairs(b, boys, ld, S, Tk, V, blockIdx.x, gridDim.x);
 }
 
-// Many molecules in one launch: molecule k owns the 64-thread blocks
-// [mol[k].blk0, mol[k + 1].blk0) (mol[nmol].blk0 = the grid), one thread per
-// ordered shell pair, and views the shared basis arrays from its own shell
-// and atom offsets.  Each thread computes exactly what oneel_kernel does
-// for that molecule alone.
+// Many molecules in one launch: molecule k owns the workgroups
+// [mol[k].blk0, mol[k + 1].blk0) (mol[nmol].blk0 = the grid) and views the
+// shared basis arrays from its own shell and atom offsets.  A pair's sums do
+// not depend on the grid: each molecule's matrices are those of oneel_kernel.
 __global__ __launch_bounds__(64) void oneel_batch_kernel(BasisView b, const double* __restrict__ boys,
                                                          const OneelMol* __restrict__ mol, int nmol,
                                                          double* __restrict__ S, double* __restrict__ Tk,
@@ -165,7 +285,15 @@ __global__ __launch_bounds__(64) void oneel_batch_kernel(BasisView b, const doub
                       b.fstart + m.shell_off, b.atom + m.shell_off, b.alpha,
                       b.coef,              b.center + 3 * m.shell_off, b.atom_xyz + 3 * m.atom_off,
                       b.atom_Z + m.atom_off};
-    oneel_pair(v, boys, m.ld, S + m.moff, Tk + m.moff, V + m.moff, (blk - m.blk0) * 64 + threadIdx.x);
+    oneel_pairs(v, boys, m.ld, S + m.moff, Tk + m.moff, V + m.moff, blk - m.blk0, mol[lo + 1].blk0 - m.blk0);
+}
+
+// a workgroup per pair; where the launch would hold more than a million of
+// them, fewer that each take several
+int gtf_oneel_blocks(int nshells, int nmol)
+{
+    const long pairs = (long)nshells * (nshells + 1) / 2, cap = (1L << 20) / (nmol > 0 ? nmol : 1);
+    return (int)(pairs < cap ? pairs : cap < 64 ? (pairs < 64 ? pairs : 64) : cap);
 }
 
 int gtf_oneel_batch(hipStream_t st, const BasisView& b, const double* boys, const OneelMol* d_mol, int nmol,
@@ -179,8 +307,7 @@ int gtf_oneel_batch(hipStream_t st, const BasisView& b, const double* boys, cons
 
 int gtf_oneel(hipStream_t st, const BasisView& b, const double* boys, int ld, double* S, double* T, double* V)
 {
-    const int n = b.nshells * b.nshells;
-    oneel_kernel<<<(n + 63) / 64, 64, 0, st>>>(b, boys, ld, S, T, V);
+    oneel_kernel<<<gtf_oneel_blocks(b.nshells, 1), 64, 0, st>>>(b, boys, ld, S, T, V);
     GTF_CHECK(hipGetLastError());
     return 0;
 }
