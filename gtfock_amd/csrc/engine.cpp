@@ -207,7 +207,19 @@ int GtfSystem::init(const std::vector<const BasisSet*>& mols, hipStream_t st)
     SYS_CHECK(hipMemcpyAsync(h_pnprim.data(), d_pnprim, sizeof(int) * npairs, hipMemcpyDeviceToHost, st));
     SYS_CHECK(hipStreamSynchronize(st));
     nprimpairs_kept = 0;
-    for (int id = 0; id < npairs; id++) nprimpairs_kept += h_pnprim[id];
+    // lanes that share a quartet of the unit kernels, per bra type: the largest
+    // power of two within the mean number of primitive pairs, each pair counted
+    // once per primitive pair (an uncontracted set keeps one lane)
+    double np1[GTF_NPAIRTYPES] = {}, np2[GTF_NPAIRTYPES] = {};
+    for (int id = 0; id < npairs; id++) {
+        nprimpairs_kept += h_pnprim[id];
+        np1[h_type[id]] += h_pnprim[id];
+        np2[h_type[id]] += (double)h_pnprim[id] * h_pnprim[id];
+    }
+    for (int t = 0; t < GTF_NPAIRTYPES; t++) {
+        unit_llane[t] = 0;
+        while (unit_llane[t] < 6 && (2 << unit_llane[t]) * np1[t] <= np2[t]) unit_llane[t]++;
+    }
     setup_s[1] = sys_wtime() - t0;
     return 0;
 }
@@ -286,12 +298,13 @@ int GtfSystem::screen(double tolscr)
             if (gtf_fill_qlist_diag(stream, n, d_ids + off, d_q + off)) return -1;
             const EriClassInfo* ci = gtf_eri_class(class_index(t, t));
             EriArgs a{};
-            a.nunits = (long)n * ci->nsplit;
+            a.llane = unit_llane[t];
+            a.nunits = ((long)n * ci->nsplit) << a.llane;
             a.qlist = d_q + off;
             a.pv = pv;
             a.fstart = d_fstart;
             a.boys8 = d_boys8;
-                    a.vbits = d_vbits;
+            a.vbits = d_vbits;
             if (launch(ci->diag, a, (int)((a.nunits + 255) / 256), stream)) return -1;
             off += n;
         }
@@ -1426,13 +1439,14 @@ int GtfSystem::collect_times()
     return 0;
 }
 
-int GtfSystem::store(int cls, int nq_, const int2* d_qlist, double* d_out)
+int GtfSystem::store(int cls, int nq_, const int4* d_list, double* d_out)
 {
     if (nq_ <= 0) return 0;
     const EriClassInfo* ci = gtf_eri_class(cls);
     EriArgs a{};
-    a.nunits = (long)nq_ * ci->nsplit;
-    a.qlist = d_qlist;
+    a.llane = unit_llane[pair_type(ci->la, ci->lb)];
+    a.nunits = ((long)nq_ * ci->nsplit) << a.llane;
+    a.slist = d_list;
     a.pv = pair_view();
     a.fstart = d_fstart;
     a.boys8 = d_boys8;

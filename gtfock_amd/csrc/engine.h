@@ -239,6 +239,7 @@ struct GtfSystem {
     void csr(std::vector<int>& shellptr, std::vector<int>& shellid, std::vector<int>& shellrid,
              std::vector<double>& shellvalue) const;
     // global pair id of two shells of the same molecule
+    int unit_llane[GTF_NPAIRTYPES] = {};  // log2 of the lanes per quartet of the unit kernels, by bra type
     int pair_id(int A, int B) const
     {
         const int m = h_shell_mol[A];
@@ -281,7 +282,7 @@ struct GtfSystem {
     // A <- (A + A^T)/2 per molecule block
     int symmetrize(double* A);
     // contracted integrals of a list of (bra, ket) canonical pair quartets of one class
-    int store(int cls, int nq_, const int2* d_qlist, double* d_out);
+    int store(int cls, int nq_, const int4* d_list, double* d_out);
     // screened unique quartets as canonical (M, N, P, Q) global shell ids;
     // returns the count, writes at most cap
     long quartets(int* out, long cap) const;

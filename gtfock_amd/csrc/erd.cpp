@@ -20,7 +20,7 @@ struct ERD {
     std::vector<std::vector<double>> bufs;  // per thread id
     double* d_out = nullptr;
     long out_cap = 0;
-    int2* d_q = nullptr;
+    int4* d_q = nullptr;
     long q_cap = 0;
 };
 
@@ -36,7 +36,7 @@ static int erd_reserve(ERD* e, long nq, long nout)
     if (nq > e->q_cap) {
         if (e->d_q) (void)hipFree(e->d_q);
         e->d_q = nullptr;
-        if (hipMalloc(&e->d_q, sizeof(int2) * nq) != hipSuccess) return -2;
+        if (hipMalloc(&e->d_q, sizeof(int4) * nq) != hipSuccess) return -2;
         e->q_cap = nq;
     }
     if (nout > e->out_cap) {
@@ -48,77 +48,63 @@ static int erd_reserve(ERD* e, long nq, long nout)
     return 0;
 }
 
+// quartets and doubles of one pass over the device
+#define ERD_PASS_QUARTETS (1L << 22)
+#define ERD_PASS_DOUBLES (1L << 25)
+
 // Integrals of nq quartets (M,N,P,Q), each in the reference layout
-// iM + dM*(iN + dN*(iP + dP*iQ)), concatenated in input order.
+// iM + dM*(iN + dN*(iP + dP*iQ)), concatenated in input order.  The kernels
+// write that layout themselves; a pass is one upload of its quartets sorted by
+// class, one launch per class and one copy into out.
 static int erd_batch(ERD* e, int nq, const int* q, double* out)
 {
     GtfSystem& s = e->sys;
     const BasisSet* b = e->basis;
-    std::vector<long> outoff(nq + 1, 0);
-    for (int i = 0; i < nq; i++) {
-        long d = 1;
-        for (int k = 0; k < 4; k++) {
-            const int sh = q[4 * i + k];
-            if (sh < 0 || sh >= s.nshells) return -3;
-            d *= b->fstart[sh + 1] - b->fstart[sh];
+    for (long i = 0; i < 4L * nq; i++)
+        if (q[i] < 0 || q[i] >= s.nshells) return -3;
+    std::vector<int4> list, sorted;
+    std::vector<int> cls;
+    for (long i0 = 0; i0 < nq;) {
+        list.clear();
+        cls.clear();
+        long count[GTF_NCLASSES + 1] = {}, nout = 0;
+        long i = i0;
+        for (; i < nq && i - i0 < ERD_PASS_QUARTETS; i++) {
+            const int *sh = q + 4 * i;
+            long d = 1;
+            for (int k = 0; k < 4; k++) d *= b->fstart[sh[k] + 1] - b->fstart[sh[k]];
+            if (nout + d > ERD_PASS_DOUBLES) break;
+            int p1 = s.pair_id(sh[0], sh[1]), p2 = s.pair_id(sh[2], sh[3]);
+            int f1 = s.h_s1[p1] != sh[0], f2 = s.h_s1[p2] != sh[2];
+            int t1 = s.h_type[p1], t2 = s.h_type[p2], flags = 0;
+            if (t1 < t2) {
+                std::swap(p1, p2);
+                std::swap(f1, f2);
+                std::swap(t1, t2);
+                flags = GTF_STORE_SWAPPED;
+            }
+            flags |= (f1 ? GTF_STORE_FLIP_BRA : 0) | (f2 ? GTF_STORE_FLIP_KET : 0);
+            list.push_back(make_int4(p1, p2, (int)nout, flags));
+            cls.push_back(class_index(t1, t2));
+            count[cls.back() + 1]++;
+            nout += d;
         }
-        outoff[i + 1] = outoff[i] + d;
-    }
-    std::vector<std::vector<int>> members(GTF_NCLASSES);
-    std::vector<int2> canon(nq);
-    std::vector<char> swapped(nq);
-    for (int i = 0; i < nq; i++) {
-        int p1 = s.pair_id(q[4 * i], q[4 * i + 1]), p2 = s.pair_id(q[4 * i + 2], q[4 * i + 3]);
-        int t1 = s.h_type[p1], t2 = s.h_type[p2];
-        swapped[i] = t1 < t2;
-        if (swapped[i]) { std::swap(p1, p2); std::swap(t1, t2); }
-        canon[i] = make_int2(p1, p2);
-        members[class_index(t1, t2)].push_back(i);
-    }
-    for (int cls = 0; cls < GTF_NCLASSES; cls++) {
-        const std::vector<int>& mem = members[cls];
-        if (mem.empty()) continue;
-        const EriClassInfo* ci = gtf_eri_class(cls);
-        const long n = (long)mem.size(), nint = ci->nints;
-        if (erd_reserve(e, n, n * nint)) return -2;
-        std::vector<int2> ql(n);
-        for (long k = 0; k < n; k++) ql[k] = canon[mem[k]];
-        if (hipMemcpyAsync(e->d_q, ql.data(), sizeof(int2) * n, hipMemcpyHostToDevice, e->stream) != hipSuccess)
+        const long n = i - i0;
+        if (erd_reserve(e, n, nout)) return -2;
+        for (int c = 0; c < GTF_NCLASSES; c++) count[c + 1] += count[c];
+        sorted.resize(n);
+        long pos[GTF_NCLASSES];
+        std::copy(count, count + GTF_NCLASSES, pos);
+        for (long k = 0; k < n; k++) sorted[pos[cls[k]]++] = list[k];
+        if (hipMemcpyAsync(e->d_q, sorted.data(), sizeof(int4) * n, hipMemcpyHostToDevice, e->stream) != hipSuccess)
             return -1;
-        if (s.store(cls, (int)n, e->d_q, e->d_out)) return -1;
-        std::vector<double> res(n * nint);
-        if (hipMemcpyAsync(res.data(), e->d_out, sizeof(double) * n * nint, hipMemcpyDeviceToHost, e->stream) !=
-                hipSuccess ||
+        for (int c = 0; c < GTF_NCLASSES; c++)
+            if (s.store(c, (int)(count[c + 1] - count[c]), e->d_q + count[c], e->d_out)) return -1;
+        if (hipMemcpyAsync(out, e->d_out, sizeof(double) * nout, hipMemcpyDeviceToHost, e->stream) != hipSuccess ||
             hipStreamSynchronize(e->stream) != hipSuccess)
             return -1;
-        const int NB = 2 * ci->lb + 1, NCc = 2 * ci->lc + 1, ND = 2 * ci->ld + 1;
-        const int NCD = NCc * ND;
-        for (long k = 0; k < n; k++) {
-            const int i = mem[k];
-            const int M = q[4 * i], N = q[4 * i + 1], P = q[4 * i + 2], Q = q[4 * i + 3];
-            const int dM = b->fstart[M + 1] - b->fstart[M], dN = b->fstart[N + 1] - b->fstart[N];
-            const int dP = b->fstart[P + 1] - b->fstart[P], dQ = b->fstart[Q + 1] - b->fstart[Q];
-            const int bra = canon[i].x, ket = canon[i].y;
-            const double* src = res.data() + k * nint;
-            double* dst = out + outoff[i];
-            for (int iQ = 0; iQ < dQ; iQ++)
-                for (int iP = 0; iP < dP; iP++)
-                    for (int iN = 0; iN < dN; iN++)
-                        for (int iM = 0; iM < dM; iM++) {
-                            // requested bra/ket pairs in terms of canonical pairs
-                            int x1 = M, y1 = N, ix1 = iM, iy1 = iN, x2 = P, y2 = Q, ix2 = iP, iy2 = iQ;
-                            if (swapped[i]) {
-                                std::swap(x1, x2); std::swap(y1, y2);
-                                std::swap(ix1, ix2); std::swap(iy1, iy2);
-                            }
-                            const int a = (s.h_s1[bra] == x1) ? ix1 : iy1;
-                            const int bb = (s.h_s1[bra] == x1) ? iy1 : ix1;
-                            const int c = (s.h_s1[ket] == x2) ? ix2 : iy2;
-                            const int d = (s.h_s1[ket] == x2) ? iy2 : ix2;
-                            (void)y1; (void)y2;
-                            dst[iM + dM * (iN + dN * (iP + dP * iQ))] = src[(a * NB + bb) * NCD + c * ND + d];
-                        }
-        }
+        out += nout;
+        i0 = i;
     }
     return 0;
 }

@@ -5,7 +5,7 @@
 //            the accumulators hold 2J and -K before symmetrisation.
 //  EPI_DIAG  Schwarz values max |(mn|mn)| of a shell pair
 //            (pfock/screening.c:63-89).
-//  EPI_STORE write the contracted integrals (for CInt_computeShellQuartet).
+//  EPI_STORE write the contracted integrals in the caller's order (for CInt_computeShellQuartet).
 //
 // Work is handed out by a device-wide atomic task counter (the GPU form of
 // taskq_next, pfock/taskq.c:55-62): each workgroup takes 256 consecutive work
@@ -18,6 +18,10 @@
 #endif
 
 enum { EPI_JK = 0, EPI_DIAG = 1, EPI_STORE = 2 };
+
+// flags of a quartet of EPI_STORE: how the caller's order of its shells
+// differs from the canonical one
+enum { GTF_STORE_SWAPPED = 1, GTF_STORE_FLIP_BRA = 2, GTF_STORE_FLIP_KET = 4 };
 
 struct EriArgs {
     // work decode: either bra rows (row_off over bra_list x ket_list) or qlist
@@ -41,8 +45,11 @@ struct EriArgs {
     long dstride;
     // EPI_DIAG
     unsigned long long* vbits;
-    // EPI_STORE
+    // EPI_STORE: (bra, ket, first double, GTF_STORE_* flags) per quartet
+    const int4* slist;
     double* out;
+    // EPI_DIAG, EPI_STORE: 2^llane lanes share a quartet's bra primitive pairs
+    int llane;
     // tiles of the LDS-strip J/K kernel and their runs of kets (gtf_internal.h)
     const TileHead* tiles;
     const int4* runs;
@@ -119,16 +126,33 @@ template <int LA, int LB, int LC, int LD, int NC>
 __device__ __forceinline__ void digest(const EriArgs& a, int bra, int ket, int c0,
                                        const double (&acc)[NC][EriShape<LA, LB, LC, LD>::NCD], long doff);
 
+// One component chunk of one quartet.  EPI_DIAG and EPI_STORE, whose lists hold
+// a pair's or a quartet's whole primitive work, deal the bra primitive pairs to
+// 2^llane lanes that add their integrals with lane shuffles: in one thread, a
+// pair of 8-primitive shells took 4096 primitive quartets one after another
+// while the wavefronts were too few to fill the chip.  Schwarz values of
+// C24H12's pairs 2.5 -> 0.5 ms, of water's 1.8 -> 0.3 ms.
 template <int LA, int LB, int LC, int LD, int NC, int EPI>
 __device__ __forceinline__ void eri_unit(const EriArgs& a, long u)
 {
     using S = EriShape<LA, LB, LC, LD>;
     constexpr int NSPLIT = S::NAB / NC;
     constexpr int NCD = S::NCD, ND = S::ND, NB = S::NB;
+    int li = 0, nl = 1;
+    if constexpr (EPI != EPI_JK) {
+        nl = 1 << a.llane;
+        li = (int)u & (nl - 1);
+        u >>= a.llane;
+    }
     const long q = u / NSPLIT;
     const int c0 = (int)(u - q * NSPLIT) * NC;
     int bra, ket;
-    if (a.qlist) {
+    int4 dst;
+    if constexpr (EPI == EPI_STORE) {
+        dst = a.slist[q];
+        bra = dst.x;
+        ket = dst.y;
+    } else if (a.qlist) {
         const int2 bk = a.qlist[q];
         bra = bk.x;
         ket = bk.y;
@@ -144,15 +168,33 @@ __device__ __forceinline__ void eri_unit(const EriArgs& a, long u)
         if (!bra_active(a, bra)) return;
     }
     double acc[NC][NCD];
-    eri_block<LA, LB, LC, LD, NC, double>(a.pv, bra, ket, c0, a.boys8 + (LA + LB + LC + LD) * BOYS8_SLAB, acc);
+    eri_block<LA, LB, LC, LD, NC, double>(a.pv, bra, ket, c0, a.boys8 + (LA + LB + LC + LD) * BOYS8_SLAB, acc, li, nl);
+    if constexpr (EPI != EPI_JK) {
+        for (int m = nl >> 1; m; m >>= 1)
+            static_for<0, NC>([&](auto c_) {
+                static_for<0, NCD>([&](auto d_) {
+                    double& x = acc[decltype(c_)::value][decltype(d_)::value];
+                    x += __shfl_xor(x, m);
+                });
+            });
+    }
 
     if constexpr (EPI == EPI_STORE) {
-        double* o = a.out + q * (long)(S::NAB * NCD) + (long)c0 * NCD;
+        // strides of the components in the caller's order: a flipped pair has
+        // its second shell first, a swapped quartet its ket pair first
+        const int f = dst.w;
+        const int sb = f & GTF_STORE_SWAPPED ? NCD : 1, sk = f & GTF_STORE_SWAPPED ? 1 : S::NAB;
+        const int sa_ = f & GTF_STORE_FLIP_BRA ? sb * NB : sb, sb_ = f & GTF_STORE_FLIP_BRA ? sb : sb * (S::NAB / NB);
+        const int sc_ = f & GTF_STORE_FLIP_KET ? sk * ND : sk, sd_ = f & GTF_STORE_FLIP_KET ? sk : sk * S::NCc;
+        double* o = a.out + (unsigned)dst.z;
         static_for<0, NC>([&](auto c_) {
             constexpr int c = decltype(c_)::value;
+            const int ia = (c0 + c) / NB, ib = (c0 + c) - ia * NB;
+            const int ob = ia * sa_ + ib * sb_;
             static_for<0, NCD>([&](auto d_) {
                 constexpr int cd = decltype(d_)::value;
-                o[c * NCD + cd] = acc[c][cd];
+                constexpr int e = c * NCD + cd;
+                if ((e & (nl - 1)) == li) o[ob + (cd / ND) * sc_ + (cd % ND) * sd_] = acc[c][cd];
             });
         });
     } else if constexpr (EPI == EPI_DIAG) {
@@ -164,7 +206,7 @@ __device__ __forceinline__ void eri_unit(const EriArgs& a, long u)
                 if (cd == c0 + c) mx = fmax(mx, fabs(acc[c][cd]));
             });
         });
-        atomicMax(a.vbits + bra, (unsigned long long)__double_as_longlong(mx));
+        if (li == 0) atomicMax(a.vbits + bra, (unsigned long long)__double_as_longlong(mx));
     } else {
         for (int d = 0; d < a.nd; d++)
             digest<LA, LB, LC, LD, NC>(a, bra, ket, c0, acc, d * a.dstride);

@@ -130,7 +130,7 @@ __host__ __device__ constexpr bool prim_screened()
 
 // Contracted integrals (bra components c0..c0+NC-1, all ket components) of
 // the quartet (bra pair | ket pair), summed over the bra primitive pairs
-// [i0, i1) (i1 < 0: all) and, in the classes of prim_screened, the
+// i0, i0 + istep, ... and, in the classes of prim_screened, the
 // primitive quartets whose Schwarz bound q_bra q_ket is at least pv.peps.  acc[c][cd], cd = c_sph * nsph(LD) + d_sph.
 // The ket coefficients are read in the compact nonzero-only layout and the
 // structurally zero terms are skipped at compile time; when a thread owns the
@@ -138,8 +138,7 @@ __host__ __device__ constexpr bool prim_screened()
 template <int LA, int LB, int LC, int LD, int NC, typename Real>
 __device__ __forceinline__ void eri_block(const PairView& pv, int bra, int ket, int c0,
                                           const double* __restrict__ boys_slab,
-                                          Real (&acc)[NC][EriShape<LA, LB, LC, LD>::NCD], int i0 = 0,
-                                          int i1 = -1)
+                                          Real (&acc)[NC][EriShape<LA, LB, LC, LD>::NCD], int i0, int istep)
 {
     using S = EriShape<LA, LB, LC, LD>;
     constexpr int L = S::L, HAB = S::HAB, HCD = S::HCD, HL = S::HL, NCD = S::NCD;
@@ -162,8 +161,7 @@ __device__ __forceinline__ void eri_block(const PairView& pv, int bra, int ket, 
     // q_i q_j >= peps are a prefix, found by bisection once per i, and once
     // one bra primitive has none the later ones have none either
     constexpr bool PSCREEN = prim_screened<LA, LB, LC, LD>();
-    const int ie = i1 < 0 ? nb : i1;
-    for (int i = i0; i < ie; ++i) {
+    for (int i = i0; i < nb; i += istep) {
         int nke = nk;
         if constexpr (PSCREEN) {
             if (pv.peps > 0.0) {

@@ -1,0 +1,130 @@
+"""The kernels at the sizes where their work splits change, against the CPU
+oracle: contractions beyond one wavefront of primitive pairs, one atom and more
+nuclei than lanes, ket lists around the 64-ket blocks, matrices around the
+32 x 32 product tiles and the largest size of the row products."""
+import numpy as np
+import pytest
+
+import oracle
+
+gpu = pytest.mark.gpu
+FOCK_TOL = 1e-10
+
+
+@pytest.fixture(scope="module")
+def g():
+    import gtfock_amd
+    gtfock_amd.lib()
+    return gtfock_amd
+
+
+def _basis(path, nprim):
+    """s, p and d shells on hydrogen with the given numbers of primitives."""
+    with open(path, "w") as fh:
+        fh.write("spherical\n\n****\nH     0\n")
+        for l, n in zip("SPD", nprim):
+            fh.write("%s   %d   1.00\n" % (l, n))
+            for k in range(n):
+                fh.write("  %.10f  %.10f\n" % (0.25 * 2.2 ** k, 1.0 / (1 + k)))
+        fh.write("****\n")
+    return str(path)
+
+
+def _hydrogens(path, n):
+    """n hydrogens in H2 pairs along a folded line (a wide gap, no symmetry)."""
+    with open(path, "w") as fh:
+        fh.write("%d\n\n" % n)
+        for k in range(n):
+            x, row = (k // 2) % 24, k // 48
+            fh.write("H %.6f %.6f %.6f\n" % (2.3 * x + 0.75 * (k % 2), 2.6 * (row % 8) + 0.05 * x, 2.9 * (row // 8) + 0.03 * (k % 5)))
+    return str(path)
+
+
+# primitives per s, p, d shell; nuclei: 81 primitive pairs and one nucleus,
+# the splits between, one primitive and more nuclei than lanes
+@gpu
+@pytest.mark.parametrize("nprim,natoms", [((9, 5, 2), 1), ((9, 3, 1), 2), ((3, 2, 3), 6), ((1, 1, 1), 66)])
+def test_one_electron_edges(g, tmp_path, nprim, natoms):
+    gbs, xyz = _basis(tmp_path / "b.gbs", nprim), _hydrogens(tmp_path / "m.xyz", natoms)
+    b, ob = g.BasisSet(gbs, xyz), oracle.Basis(gbs, xyz)
+    pf = g.PFock(b)
+    S, H, Hr = pf.overlap(), pf.core_hamiltonian(), ob.core_hamiltonian()
+    pf.close()
+    print("one-electron %s %d: %.2e %.2e" % (nprim, natoms, np.abs(S - ob.overlap()).max(), np.abs(H - Hr).max()))
+    assert np.abs(S - ob.overlap()).max() < 1e-12
+    assert np.abs(H - Hr).max() < 1e-12 * max(10.0, np.abs(Hr).max())
+
+
+# every order and orientation of the shells; the lanes per quartet follow the
+# primitives, from one to all 64 of a wavefront
+@gpu
+@pytest.mark.parametrize("nprim", [(1, 1, 1), (3, 2, 1), (9, 3, 2)])
+def test_quartets_in_every_order(g, tmp_path, nprim):
+    gbs, xyz = _basis(tmp_path / "b.gbs", nprim), _hydrogens(tmp_path / "m.xyz", 2)
+    b, ob = g.BasisSet(gbs, xyz), oracle.Basis(gbs, xyz)
+    erd = g.ERD(b)
+    ns = b.nshells
+    q = np.array([(M, N, P, Q) for M in range(ns) for N in range(ns) for P in range(ns) for Q in range(ns)], dtype=np.int32)
+    worst = 0.0
+    for quartet, r in zip(q, erd.quartets(q)):
+        ref = ob.eri_quartet(*quartet).reshape(-1)
+        worst = max(worst, np.abs(r - ref).max() / max(1.0, np.abs(ref).max()))
+    print("quartets %s: %.2e" % (nprim, worst))
+    assert worst < 1e-12
+    one = erd.quartet(*[int(x) for x in q[-2]])
+    assert np.abs(one - ob.eri_quartet(*q[-2]).reshape(-1)).max() < 1e-12 * max(1.0, np.abs(one).max())
+
+
+# long contractions in every class; STO-3G hydrogens put 55, 66 and 136 kets
+# in the (ss| list, around the 64-ket blocks; one and two densities
+@gpu
+@pytest.mark.parametrize("nprim,natoms", [((9, 5, 2), 1), ((9, 3, 1), 2), ((1, 1, 1), 4),
+                                          (None, 2), (None, 10), (None, 11), (None, 16)])
+def test_fock_edges(g, sto3g, tmp_path, nprim, natoms):
+    gbs = _basis(tmp_path / "b.gbs", nprim) if nprim else sto3g
+    xyz = _hydrogens(tmp_path / "m.xyz", natoms)
+    b, ob = g.BasisSet(gbs, xyz), oracle.Basis(gbs, xyz)
+    rng = np.random.default_rng(77)
+    Ds = [0.1 * (a + a.T) for a in rng.normal(size=(2, b.nbf, b.nbf))]
+    refs = [sum(ob.fock(D)[:2]) for D in Ds]
+    pf = g.PFock(b, tolscr=1e-11, max_numdmat=2)
+    err = np.abs(pf.fock(Ds[0]) - refs[0]).max()
+    pf.set_num_den_mat(2)
+    for k, D in enumerate(Ds):
+        pf.put_den_mat(D, index=k)
+    pf.commit()
+    pf.compute_fock()
+    err2 = max(np.abs(pf.get_mat(g.MAT_F, index=k) - refs[k]).max() for k in range(2))
+    pf.close()
+    print("fock %s %d: %.2e, two densities %.2e" % (nprim, natoms, err, err2))
+    assert max(err, err2) < FOCK_TOL
+
+
+# one tile, a remainder of two, exact tiles, several tiles
+@gpu
+@pytest.mark.parametrize("n", [2, 32, 34, 64, 66, 130])
+def test_purification_edges(g, sto3g, tmp_path, n):
+    xyz = _hydrogens(tmp_path / "m.xyz", n)
+    b, ob = g.BasisSet(sto3g, xyz), oracle.Basis(sto3g, xyz)
+    S = ob.overlap()
+    X = oracle.inv_sqrt(S)
+    F = X @ ob.core_hamiltonian() @ X
+    F = 0.5 * (F + F.T)
+    Dref, _ = oracle.purification(F, X, ob.nocc)
+    pu = g.Purif(b)
+    pu.set_xs(X, S)
+    D, _ = pu.purify(F)
+    pu.close()
+    print("purification n = %d: %.2e" % (n, np.abs(D - Dref).max()))
+    assert np.abs(D - Dref).max() < 1e-10
+
+
+# A B^T: below, at and above a tile, and both sides of the largest size of the
+# row products; each element within the rounding of its sum of k products
+@gpu
+@pytest.mark.parametrize("n", [1, 31, 33, 64, 100, 511, 512, 513])
+def test_dgemm_edges(g, n):
+    rng = np.random.default_rng(n)
+    A, B = rng.normal(size=(2, n, n))
+    bound = 2.0 * (n + 1) * np.finfo(float).eps * (np.abs(A) @ np.abs(B.T)) + 1e-300
+    assert (np.abs(g.dgemm(A, B, transB=True) - A @ B.T) <= bound).all()
