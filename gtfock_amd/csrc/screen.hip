@@ -362,21 +362,25 @@ __global__ __launch_bounds__(256) void prim_census_kernel(CensusArgs c)
     if ((threadIdx.x & 63) == 0 && cnt) atomicAdd(c.out, cnt);
 }
 
-// Ket records of a type list: one thread per ket copies its primitive pairs
+// Ket records of a type list: PACK_Y threads per ket copy its primitive pairs
 // into the 64-ket blocks, so a wavefront's writes are whole rows; the reads
-// are the pairs' own records.
+// are the pairs' own records.  Bound by the latency of
+// those reads: with one thread per ket the six lists of C24H12 took 1.0 ms.
+#define PACK_Y 16
 __global__ __launch_bounds__(256) void pack_kets_kernel(PairView pv, const int* __restrict__ fstart, KetPack k)
 {
     const int j = blockIdx.x * 256 + threadIdx.x;
     if (j >= k.n) return;
     const int id = k.sig[j], np = pv.nprim[id], b = k.base[j], rec = KetView::rec(k.nnz);
     const int s1 = pv.s1[id], s2 = pv.s2[id];
-    k.info[j] = make_int4(fstart[s1], fstart[s2], s1 != s2, id);
-    k.nprim[j] = np;
-    const double* z = pv.Ez + pv.zoff[id];
+    if (blockIdx.y == 0) {
+        k.info[j] = make_int4(fstart[s1], fstart[s2], s1 != s2, id);
+        k.nprim[j] = np;
+    }
     const int po = pv.poff[id];
-    double2* d = k.d + (long)(b >> 6) * (rec * 64) + (b & 63);
-    for (int i = 0; i < np; i++, d += rec * 64, z += k.nnz) {
+    for (int i = blockIdx.y; i < np; i += PACK_Y) {
+        const double* z = pv.Ez + pv.zoff[id] + (long)i * k.nnz;
+        double2* d = k.d + ((long)(b >> 6) + i) * (rec * 64) + (b & 63);
         const double4 p = pv.prim[po + i];
         d[0] = make_double2(p.x, p.y);
         d[64] = make_double2(p.z, p.w);
@@ -509,7 +513,7 @@ int gtf_round_f32(hipStream_t st, const double* x, long n, float* y)
 int gtf_pack_kets(hipStream_t st, const PairView& pv, const int* fstart, const KetPack& k)
 {
     if (k.n <= 0) return 0;
-    pack_kets_kernel<<<(k.n + 255) / 256, 256, 0, st>>>(pv, fstart, k);
+    pack_kets_kernel<<<dim3((k.n + 255) / 256, PACK_Y), 256, 0, st>>>(pv, fstart, k);
     GTF_CHECK(hipGetLastError());
     return 0;
 }
