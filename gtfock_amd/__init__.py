@@ -476,10 +476,10 @@ class ERD:
         q = np.ascontiguousarray(q, dtype=np.int32).reshape(-1, 4)
         d = np.array(self.basis.shell_dim)
         sizes = d[q[:, 0]] * d[q[:, 1]] * d[q[:, 2]] * d[q[:, 3]]
-        out = np.zeros(int(sizes.sum()))
+        out = np.empty(int(sizes.sum()))
         _check(lib().gtf_erd_quartets(self.h, len(q), q.ctypes.data_as(_ip), _p(out)), "gtf_erd_quartets")
-        offs = np.concatenate([[0], np.cumsum(sizes)])
-        return [out[offs[i]:offs[i + 1]] for i in range(len(q))]
+        offs = np.concatenate([[0], np.cumsum(sizes)]).tolist()  # plain ints: numpy ones double the slicing
+        return [out[i:j] for i, j in zip(offs, offs[1:])]
 
 
 def dgemm(A, B, transB=False, fp32=False, split=0):
