@@ -270,10 +270,13 @@ int GtfSystem::screen(double tolscr)
             const EriClassInfo* ci = gtf_eri_class(c);
             for (int ex = 0; ex < 2; ex++) {
                 hipFuncAttributes fa{};
-                const eri_kernel_t fn = ex ? ci->jk_tile_t[1] : ci->jk_tile[1];
-                tile_regs[2 * c + ex] = 256;
-                if (fn && hipFuncGetAttributes(&fa, (const void*)fn) == hipSuccess && fa.numRegs > 0)
-                    tile_regs[2 * c + ex] = (fa.numRegs + 7) / 8 * 8;
+                const eri_kernel_t fn[2] = {ex ? ci->jk_tile_t[1] : ci->jk_tile[1],
+                                            ex ? ci->jk_tile_t_lo : ci->jk_tile_lo};
+                for (int lo = 0; lo < 2; lo++) {
+                    tile_regs[4 * c + 2 * lo + ex] = 256;
+                    if (fn[lo] && hipFuncGetAttributes(&fa, (const void*)fn[lo]) == hipSuccess && fa.numRegs > 0)
+                        tile_regs[4 * c + 2 * lo + ex] = (fa.numRegs + 7) / 8 * 8;
+                }
             }
         }
     }
@@ -1014,19 +1017,24 @@ bool GtfSystem::fits_densities(int nd) const
 // register limits, 256 threads on a tie (shorter waits at a tile's end).  The
 // grid is what the chip holds at once, at most the shape's: more workgroups
 // would only start later and set up their LDS again.
-GtfSystem::TileLaunch GtfSystem::tile_launch(int cls, int n, int nd) const
+// FP64 tiles of one density stage the Boys slab and the density rows in LDS
+// where the shape says so (C54H18 183 ms, 195 without).  FP32 tiles and several
+// densities never do: their registers leave room for more wavefronts than the
+// staged LDS does (C24H12 mixed 24.6 ms, 27.6 staged; seven waters, two
+// densities 1.36 ms, 1.45 staged).
+GtfSystem::TileLaunch GtfSystem::tile_launch(int cls, int n, int nd, bool low) const
 {
     TileLaunch t{};
     const EriClassInfo* ci = gtf_eri_class(cls);
     const int NA = 2 * ci->la + 1, NB = 2 * ci->lb + 1, NCD = (2 * ci->lc + 1) * (2 * ci->ld + 1);
-    const int simd_waves = std::max(1, 512 / std::max(1, tile_regs[2 * cls + (exchanged(cls) ? 1 : 0)]));
+    const int simd_waves = std::max(1, 512 / std::max(1, tile_regs[4 * cls + 2 * low + exchanged(cls)]));
     const size_t rows = (size_t)(NA + NB) * nbf;
     int best = 0;
     for (int threads = 256; threads <= ci->tile_threads; threads *= 2) {
         const int w = threads / 64;
         const size_t plain = sizeof(double) * (size_t)nd * tile_work(NA + NB, nbf, NA * NB, NCD, nd == 1 ? w : 0);
-        const size_t with = plain + sizeof(double) * ((size_t)nd * rows + GTF_BOYS_LDS);
-        const bool staged = shape[cls].boys_lds && with <= max_lds;
+        const size_t with = plain + sizeof(double) * (rows + GTF_BOYS_LDS);
+        const bool staged = shape[cls].boys_lds && !low && nd == 1 && with <= max_lds;
         const size_t lds = staged ? with : plain;
         const int wgs = (int)std::min<size_t>(max_lds / lds, std::max(1, 4 * simd_waves / w));
         if (wgs * w > best) {
@@ -1074,7 +1082,7 @@ int GtfSystem::jk(const double* D, double* J, double* K, int nd, long dstride)
             for (int lo = 0; lo < 2; lo++) {
                 const int n = nq[cls] == 0 ? 0 : lo ? ntiles_lo[cls] : ntiles[cls];
                 wg_off[2 * cls + lo] = tot;
-                wg_n[2 * cls + lo] = n > 0 ? tile_launch(cls, n, nd).grid : 0;
+                wg_n[2 * cls + lo] = n > 0 ? tile_launch(cls, n, nd, lo).grid : 0;
                 tot += wg_n[2 * cls + lo];
             }
         if (tot > wgstat_cap) {
@@ -1162,14 +1170,14 @@ int GtfSystem::launch_class(int cls, hipStream_t cs, const double* D, double* J,
         for (int low = 0; low < 2; low++) {
             a.ntiles = low ? ntiles_lo[cls] : ntiles[cls];
             if (a.ntiles == 0) continue;
-            const TileLaunch t = tile_launch(cls, a.ntiles, nd);
+            const TileLaunch t = tile_launch(cls, a.ntiles, nd, low);
             const int bl = t.staged ? 1 : 0;
             a.tiles = low ? d_tiles_lo[cls] : d_tiles[cls];
             a.runs = low ? d_runs_lo[cls] : d_runs[cls];
             a.pv.peps = low ? prim_tol_fp32() : prim_tol;
             a.counter = d_counters + cls + (low ? GTF_NCLASSES : 0);
             a.wg_stat = wg_record(2 * cls + low, t.grid);
-            const eri_kernel_t fn = low ? (exch ? ci->jk_tile_t_lo[bl] : ci->jk_tile_lo[bl])
+            const eri_kernel_t fn = low ? (exch ? ci->jk_tile_t_lo : ci->jk_tile_lo)
                                         : (exch ? ci->jk_tile_t[bl] : ci->jk_tile[bl]);
             if (launch(fn, a, t.grid, cs, t.lds, t.threads)) return -1;
         }

@@ -143,9 +143,9 @@ struct GtfSystem {
         size_t lds;
         int threads, grid;  // grid 0: does not fit
     };
-    TileLaunch tile_launch(int cls, int n, int nd) const;
+    TileLaunch tile_launch(int cls, int n, int nd, bool low = false) const;
     int ncu = 256;                            // CUs of the device
-    int tile_regs[2 * GTF_NCLASSES] = {0};    // VGPRs of the tile kernels: standard, exchanged
+    int tile_regs[4 * GTF_NCLASSES] = {0};    // VGPRs of the tile kernels: FP64 standard, exchanged, FP32 the same
     size_t max_lds = 65536;
     bool use_tiles = true;
     // Tile shape of each class (the autotuner's search space): at most
@@ -153,14 +153,14 @@ struct GtfSystem {
     // about `unit_pq` primitive quartets per unit (how finely a quartet's bra
     // primitives are chunked), `grid` persistent workgroups per launch, each
     // taking tiles from the class counter until none are left,
-    // `boys_lds` whether the workgroups stage the Boys slab and the bra
-    // shells' density rows in LDS (where they fit), and
+    // `boys_lds` whether the workgroups of FP64 tiles and one density stage
+    // the Boys slab and the bra shells' density rows in LDS (where they fit), and
     // `fp32` whether the class evaluates its quartets below the Schwarz
     // bound tau in FP32 (with 0 it stays FP64 throughout, which is never
     // less accurate; only the speed differs from class to class).  The
-    // defaults are the shapes measured best on C10H22 / C54H18 by hand
-    // (2048 persistent workgroups beat one workgroup per tile: C10H22 7.6 vs
-    // 7.9 ms, C54H18 404 vs 433 ms).
+    // defaults are the shapes that no class loses much with from water to
+    // C54H18 (the tuning tables hold those of a workload); grid only bounds
+    // the launch, which tile_launch sizes by the tiles and the occupancy.
     struct TileShape {
         int units = GTF_TILE_UNITS;
         int unit_pq = GTF_UNIT_PQ;
@@ -171,9 +171,11 @@ struct GtfSystem {
     };
     TileShape shape[GTF_NCLASSES];
     // classes run by the bra/ket-exchanged tile kernel (bit = class index;
-    // only classes that have one).  Default: the classes where it is faster on
-    // MI355X, because it needs fewer threads per quartet and so forms R less
-    // often.
+    // only classes that have one).  Default: the classes where it is faster,
+    // because it needs fewer units per quartet and so forms R less often; on
+    // C10H22 alone, standard / exchanged, (dd|ps) 297 / 104 us, (dd|ds) 201 /
+    // 79, (dd|dp) 267 / 136, (dp|ds) 289 / 184.  The others are within 10 % or
+    // change sides between C10H22 and C54H18.
     unsigned exchanged_mask = (1u << 4) | (1u << 12) | (1u << 13) | (1u << 16) | (1u << 17) |
                               (1u << 18) | (1u << 19);
     bool exchanged(int cls) const;

@@ -42,15 +42,15 @@ void GTF_NAME(GTF_CLASS, GTF_PART)(EriClassInfo& e)
     e.jk = eri_kernel<LA, LB, LC, LD, NC, EPI_JK>;
     e.store = eri_kernel<LA, LB, LC, LD, NC, EPI_STORE>;
     if constexpr (A == B) e.diag = eri_kernel<LA, LB, LC, LD, NC, EPI_DIAG>;
-#else
-    using Real = std::conditional<GTF_PART == 1, double, float>::type;
-    eri_kernel_t(&tile)[2] = GTF_PART == 1 ? e.jk_tile : e.jk_tile_lo;
-    tile[0] = eri_jk_tile_kernel<LA, LB, LC, LD, NT, Real, false>;
-    tile[1] = eri_jk_tile_kernel<LA, LB, LC, LD, NT, Real, true>;
+#elif GTF_PART == 1
+    e.jk_tile[0] = eri_jk_tile_kernel<LA, LB, LC, LD, NT, double, false>;
+    e.jk_tile[1] = eri_jk_tile_kernel<LA, LB, LC, LD, NT, double, true>;
     if constexpr (EXCHANGED) {
-        eri_kernel_t(&tile_t)[2] = GTF_PART == 1 ? e.jk_tile_t : e.jk_tile_t_lo;
-        tile_t[0] = eri_jk_tile_t_kernel<LA, LB, LC, LD, NCT, Real, false>;
-        tile_t[1] = eri_jk_tile_t_kernel<LA, LB, LC, LD, NCT, Real, true>;
+        e.jk_tile_t[0] = eri_jk_tile_t_kernel<LA, LB, LC, LD, NCT, double, false>;
+        e.jk_tile_t[1] = eri_jk_tile_t_kernel<LA, LB, LC, LD, NCT, double, true>;
     }
+#else
+    e.jk_tile_lo = eri_jk_tile_kernel<LA, LB, LC, LD, NT, float, false>;
+    if constexpr (EXCHANGED) e.jk_tile_t_lo = eri_jk_tile_t_kernel<LA, LB, LC, LD, NCT, float, false>;
 #endif
 }

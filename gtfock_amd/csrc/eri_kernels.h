@@ -857,12 +857,12 @@ struct EriClassInfo {
     bool full_E;       // the standard tile kernel reads the full coefficients
     int nints;      // integrals per quartet
     eri_kernel_t jk, diag, store;
-    // tile kernels, [0] Boys slab read from HBM, [1] staged in LDS
-    eri_kernel_t jk_tile[2];     // FP64 quartets (v_bra v_ket >= tau2)
-    eri_kernel_t jk_tile_lo[2];  // FP32 quartets (v_bra v_ket < tau2)
+    // tile kernels: FP64 quartets (v_bra v_ket >= tau2), [0] Boys slab read
+    // from HBM, [1] staged in LDS; FP32 quartets (v_bra v_ket < tau2)
+    eri_kernel_t jk_tile[2], jk_tile_lo;
     // classes that have a tile kernel with the contractions exchanged
     // (nsplit_t > 0): threads per quartet, ket components per thread
     int nsplit_t, nc_t;
-    eri_kernel_t jk_tile_t[2], jk_tile_t_lo[2];
+    eri_kernel_t jk_tile_t[2], jk_tile_t_lo;
 };
 const EriClassInfo* gtf_eri_class(int cls);

@@ -301,15 +301,14 @@ __device__ __forceinline__ void prim_quartet_R(const_as<double>* B, const double
     hermite_R<L, Real>(R, F, Real(on ? GTF_TWO_PI_2_5 * rd : 0.0), Real(-2.0 * alphad), Real(Xd), Real(Yd), Real(Zd));
 }
 
-#ifndef PAIR_MAX_L
 #define PAIR_MAX_L 1
-#endif
 // Runs body(i, R) over the bra primitives of one ket primitive.  With
 // primitive screening the wavefront goes on while any lane's bound passes (the
 // bounds fall with i) and a lane that has ended adds zeros.  The classes of L
-// <= 2 form R of two bra primitives at a time: a primitive quartet is a chain
-// of about 70 dependent operations, and their 3-4 wavefronts per SIMD do not
-// fill its gaps.
+// <= PAIR_MAX_L form R of two bra primitives at a time: a primitive quartet is
+// a chain of about 70 dependent operations, and their 3-4 wavefronts per SIMD
+// do not fill its gaps (with L = 2 too, (ps|ps) took 197 registers and gained
+// nothing).
 template <int L, bool PSCREEN, typename Real, bool BLDS, typename Coef, typename Body>
 __device__ __forceinline__ void bra_loop(const BraRef<Coef>& b, const double2& k0, const double2& k1, double qj, bool on,
                                          const double* __restrict__ boys_slab, Body&& body)
