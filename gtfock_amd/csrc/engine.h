@@ -23,6 +23,10 @@
 // chip holds of it
 #define GTF_TILES_PER_WG 3
 #define GTF_MIN_TILE_UNITS 4
+// Most primitive quartets of a tile per double of its exchange rows: the batch of
+// 40 molecules 28.1 ms (29.0 without the bound), C54H18 184 ms either way; at
+// half of it C54H18 takes 187.5 ms.
+#define GTF_FLUSH_PQ 150.0
 // default primitive screening threshold of the J/K builds
 #define GTF_PRIM_TOL_DEFAULT 1e-15
 
