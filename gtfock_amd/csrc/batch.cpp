@@ -656,7 +656,8 @@ int GtfBatch::purify(const std::vector<int>& active)
                    gtf_bgemm(stream, L, skip, d_iters, p_D, p_D2, p_D3, 0, d_low) ||
                    (purif_mode == GTF_LOW_SPLIT && gtf_oz_square_cube(stream, o, oz, p_D, p_D2, p_D3)) ||
                    gtf_bpurif_stats(stream, L, skip, p_D, p_D2, p_D3, d_iters, d_stats, it, 1e-11, d_low, purif_until) ||
-                   gtf_bpurif_update(stream, L, skip, d_iters, d_stats, p_D, p_D2, p_D3, it)) {
+                   gtf_bpurif_update(stream, L, skip, d_iters, d_stats, p_D, p_D2, p_D3, it,
+                                     purif_mode == GTF_LOW_SPLIT && purif_resid > 0.0)) {
             return -1;
         }
         if (it % 2 == 1) {

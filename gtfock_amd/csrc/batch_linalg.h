@@ -36,8 +36,9 @@ int gtf_bpurif_init(hipStream_t st, const BatchLayout& L, const int* nocc, const
 int gtf_bpurif_stats(hipStream_t st, const BatchLayout& L, const int* skip, const double* D, const double* D2,
                      const double* D3, int* iters, double* stats, int it, double tol, int* fp32 = nullptr,
                      double fp32_until = 0.0, int* low_iters = nullptr);
+// sym: with the means of D2, D3 and their transposes (D stays symmetric)
 int gtf_bpurif_update(hipStream_t st, const BatchLayout& L, const int* skip, const int* iters, const double* stats,
-                      double* D, const double* D2, const double* D3, int it);
+                      double* D, const double* D2, const double* D3, int it, bool sym);
 // One FP64 purification iteration: D2 = D D, D3 = D D2 and the update of D
 // (which must be symmetric); iters[m] = it for a molecule whose ||D - D2||_F is
 // below tol, after its update, also in host_iters (pinned host memory, may be

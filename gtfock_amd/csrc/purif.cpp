@@ -261,13 +261,16 @@ static int purify(purif_t* p, double* F_block, double* D_block, int* iters)
             }
         }
     } else {
+        // the split products of an SCF that hands over to FP64; without the
+        // hand-over (split_resid 0) and in the FP32 form they are used as they come
+        const bool sym = mode == GTF_LOW_SPLIT && d->split_resid > 0.0;
         for (it = 0; it < 200; it++) {
             if (gtf_bgemm(d->stream, L, nullptr, d->d_iters, d->D, d->D, d->D2, 0, d->d_low) ||
                 gtf_bgemm(d->stream, L, nullptr, d->d_iters, d->D, d->D2, d->D3, 0, d->d_low) ||
                 (mode == GTF_LOW_SPLIT && gtf_oz_square_cube(d->stream, o, d->oz, d->D, d->D2, d->D3)) ||
                 gtf_bpurif_stats(d->stream, L, nullptr, d->D, d->D2, d->D3, d->d_iters, d->d_stats, it, 1e-11, d->d_low,
                                  d->low_until, d->d_lowit) ||
-                gtf_bpurif_update(d->stream, L, nullptr, d->d_iters, d->d_stats, d->D, d->D2, d->D3, it))
+                gtf_bpurif_update(d->stream, L, nullptr, d->d_iters, d->d_stats, d->D, d->D2, d->D3, it, sym))
                 return -1;
             if (it % PURIF_CHECK == PURIF_CHECK - 1) {
                 PD_CHECK(hipMemcpyAsync(&it_done, d->d_iters, sizeof(int), hipMemcpyDeviceToHost, d->stream));

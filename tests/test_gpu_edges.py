@@ -128,3 +128,23 @@ def test_dgemm_edges(g, n):
     A, B = rng.normal(size=(2, n, n))
     bound = 2.0 * (n + 1) * np.finfo(float).eps * (np.abs(A) @ np.abs(B.T)) + 1e-300
     assert (np.abs(g.dgemm(A, B, transB=True) - A @ B.T) <= bound).all()
+
+
+# the symmetric update of the split products: one tile, remainders, several
+# tiles; the last iterations are FP64, so the projector is as exact as theirs
+@gpu
+@pytest.mark.parametrize("n", [2, 34, 64, 130])
+def test_split_purification_edges(g, sto3g, tmp_path, n):
+    xyz = _hydrogens(tmp_path / "m.xyz", n)
+    b, ob = g.BasisSet(sto3g, xyz), oracle.Basis(sto3g, xyz)
+    S = ob.overlap()
+    X = oracle.inv_sqrt(S)
+    pu = g.Purif(b)
+    pu.set_xs(X, S)
+    pu.set_precision("split")
+    D, _ = pu.purify(X @ ob.core_hamiltonian() @ X)
+    pu.close()
+    print("split n = %d: %.2e %.2e" % (n, np.abs(D - D.T).max(), np.abs(D @ S @ D - D).max()))
+    assert np.abs(D - D.T).max() < 1e-12
+    assert np.abs(D @ S @ D - D).max() < 1e-10
+    assert abs(np.trace(D @ S) - ob.nocc) < 1e-9
