@@ -949,8 +949,8 @@ void GtfSystem::cut_class_tiles(int cls, TileList& hv, TileList& lv)
         }
         // a class with little work is cut finer, so that it spreads over the
         // chip, down to a unit for each wavefront
-        const double even = std::min<double>(
-            sh.tile_pq, std::max(total / (GTF_TILES_PER_WG * resident), GTF_MIN_TILE_UNITS * total / units));
+        const double least = GTF_MIN_TILE_UNITS * total / units;
+        const double even = std::min<double>(sh.tile_pq, std::max(total / (GTF_TILES_PER_WG * resident), least));
         struct Tile {
             double cost;
             int row, run0, nrun;
@@ -969,7 +969,8 @@ void GtfSystem::cut_class_tiles(int cls, TileList& hv, TileList& lv)
             // a tile flushes the exchange rows of its bra shells once; past
             // GTF_FLUSH_PQ primitive quartets per double of them a larger tile
             // saves little and balances worse
-            const double target = std::min(even, GTF_FLUSH_PQ * 2.0 * (ci->la + ci->lb + 1) * mol_nbf[h_sigmol[A][p.r]]);
+            const double flush = GTF_FLUSH_PQ * 2.0 * (ci->la + ci->lb + 1) * mol_nbf[h_sigmol[A][p.r]];
+            const double target = std::min(even, std::max(least, flush));
             // a wavefront takes all chunks of 64 kets: at most an eighth of a tile
             const double most = target / 8;
             for (long j = p.b; j < p.e;) {
