@@ -5,6 +5,7 @@
 #include <sys/time.h>
 
 #include <algorithm>
+#include <array>
 #include <cmath>
 #include <cstring>
 #include <atomic>
@@ -253,6 +254,26 @@ static int launch(eri_kernel_t fn, EriArgs& a, int blocks, hipStream_t st, size_
     return 0;
 }
 
+// VGPRs of the tile kernels, FP64 standard and exchanged, FP32 the same, by
+// class: asked for once in a process (84 runtime calls)
+static const std::array<int, 4 * GTF_NCLASSES>& tile_registers()
+{
+    static const std::array<int, 4 * GTF_NCLASSES> regs = [] {
+        std::array<int, 4 * GTF_NCLASSES> r;
+        for (int c = 0; c < GTF_NCLASSES; c++) {
+            const EriClassInfo* ci = gtf_eri_class(c);
+            const eri_kernel_t fn[4] = {ci->jk_tile[1], ci->jk_tile_t[1], ci->jk_tile_lo, ci->jk_tile_t_lo};
+            for (int k = 0; k < 4; k++) {
+                hipFuncAttributes fa{};
+                const bool known = fn[k] && hipFuncGetAttributes(&fa, (const void*)fn[k]) == hipSuccess && fa.numRegs > 0;
+                r[4 * c + k] = known ? (fa.numRegs + 7) / 8 * 8 : 256;
+            }
+        }
+        return r;
+    }();
+    return regs;
+}
+
 int GtfSystem::screen(double tolscr)
 {
     if (const char* s = getenv("GTF_JK_TILES")) use_tiles = atoi(s) != 0;
@@ -266,19 +287,6 @@ int GtfSystem::screen(double tolscr)
             hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && lds > 0)
             max_lds = (size_t)lds - 64;  // the kernels' static LDS
         if (hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || ncu < 1) ncu = 256;
-        for (int c = 0; c < GTF_NCLASSES; c++) {
-            const EriClassInfo* ci = gtf_eri_class(c);
-            for (int ex = 0; ex < 2; ex++) {
-                hipFuncAttributes fa{};
-                const eri_kernel_t fn[2] = {ex ? ci->jk_tile_t[1] : ci->jk_tile[1],
-                                            ex ? ci->jk_tile_t_lo : ci->jk_tile_lo};
-                for (int lo = 0; lo < 2; lo++) {
-                    tile_regs[4 * c + 2 * lo + ex] = 256;
-                    if (fn[lo] && hipFuncGetAttributes(&fa, (const void*)fn[lo]) == hipSuccess && fa.numRegs > 0)
-                        tile_regs[4 * c + 2 * lo + ex] = (fa.numRegs + 7) / 8 * 8;
-                }
-            }
-        }
     }
     tol = tolscr;
     tol2 = tolscr * tolscr;
@@ -1032,7 +1040,7 @@ GtfSystem::TileLaunch GtfSystem::tile_launch(int cls, int n, int nd, bool low) c
     TileLaunch t{};
     const EriClassInfo* ci = gtf_eri_class(cls);
     const int NA = 2 * ci->la + 1, NB = 2 * ci->lb + 1, NCD = (2 * ci->lc + 1) * (2 * ci->ld + 1);
-    const int simd_waves = std::max(1, 512 / std::max(1, tile_regs[4 * cls + 2 * low + exchanged(cls)]));
+    const int simd_waves = std::max(1, 512 / std::max(1, tile_registers()[4 * cls + 2 * low + exchanged(cls)]));
     const size_t rows = (size_t)(NA + NB) * nbf;
     int best = 0;
     for (int threads = 256; threads <= ci->tile_threads; threads *= 2) {

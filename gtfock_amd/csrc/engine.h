@@ -149,7 +149,6 @@ struct GtfSystem {
     };
     TileLaunch tile_launch(int cls, int n, int nd, bool low = false) const;
     int ncu = 256;                            // CUs of the device
-    int tile_regs[4 * GTF_NCLASSES] = {0};    // VGPRs of the tile kernels: FP64 standard, exchanged, FP32 the same
     size_t max_lds = 65536;
     bool use_tiles = true;
     // Tile shape of each class (the autotuner's search space): at most
