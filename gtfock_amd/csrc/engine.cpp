@@ -1043,21 +1043,26 @@ GtfSystem::TileLaunch GtfSystem::tile_launch(int cls, int n, int nd, bool low) c
     const int simd_waves = std::max(1, 512 / std::max(1, tile_registers()[4 * cls + 2 * low + exchanged(cls)]));
     const size_t rows = (size_t)(NA + NB) * nbf;
     int best = 0;
-    for (int threads = 256; threads <= ci->tile_threads; threads *= 2) {
-        const int w = threads / 64;
-        const size_t plain = sizeof(double) * (size_t)nd * tile_work(NA + NB, nbf, NA * NB, NCD, nd == 1 ? w : 0);
-        const size_t with = plain + sizeof(double) * (rows + GTF_BOYS_LDS);
-        const bool staged = shape[cls].boys_lds && !low && nd == 1 && with <= max_lds;
-        const size_t lds = staged ? with : plain;
-        const int wgs = (int)std::min<size_t>(max_lds / lds, std::max(1, 4 * simd_waves / w));
-        if (wgs * w > best) {
-            best = wgs * w;
-            t.staged = staged;
-            t.lds = lds;
-            t.threads = threads;
-            t.grid = std::min({n, shape[cls].grid, wgs * ncu});
+    // the J_PQ buffers of a single density come before the wavefronts that the
+    // LDS would hold without them
+    for (int buffered = nd == 1; buffered >= 0 && best == 0; buffered--)
+        for (int threads = 256; threads <= ci->tile_threads; threads *= 2) {
+            const int w = threads / 64;
+            const size_t plain =
+                sizeof(double) * (size_t)nd * tile_work(NA + NB, nbf, NA * NB, NCD, buffered ? w : 0);
+            const size_t with = plain + sizeof(double) * (rows + GTF_BOYS_LDS);
+            const bool staged = shape[cls].boys_lds && !low && nd == 1 && with <= max_lds;
+            const size_t lds = staged ? with : plain;
+            const int wgs = (int)std::min<size_t>(max_lds / lds, std::max(1, 4 * simd_waves / w));
+            if (wgs * w > best) {
+                best = wgs * w;
+                t.staged = staged;
+                t.buffered = buffered;
+                t.lds = lds;
+                t.threads = threads;
+                t.grid = std::min({n, shape[cls].grid, wgs * ncu});
+            }
         }
-    }
     return t;
 }
 
@@ -1185,6 +1190,7 @@ int GtfSystem::launch_class(int cls, hipStream_t cs, const double* D, double* J,
             if (a.ntiles == 0) continue;
             const TileLaunch t = tile_launch(cls, a.ntiles, nd, low);
             const int bl = t.staged ? 1 : 0;
+            a.jpq_lds = t.buffered;
             a.tiles = low ? d_tiles_lo[cls] : d_tiles[cls];
             a.runs = low ? d_runs_lo[cls] : d_runs[cls];
             a.pv.peps = low ? prim_tol_fp32() : prim_tol;

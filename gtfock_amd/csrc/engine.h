@@ -141,9 +141,9 @@ struct GtfSystem {
     };
     // launch of a class's n tiles digesting nd densities; staged: with the Boys
     // slab and the density rows in LDS (asked for by the shape and within
-    // max_lds)
+    // max_lds); buffered: with the wavefronts' J_PQ buffers in LDS
     struct TileLaunch {
-        bool staged;
+        bool staged, buffered;
         size_t lds;
         int threads, grid;  // grid 0: does not fit
     };

@@ -61,6 +61,7 @@ struct EriArgs {
     KetView kv;  // the ket list, for the tile kernels
     int ntiles;
     int nbf;  // LDS strip capacity (largest molecule)
+    int jpq_lds;  // the wavefronts have J_PQ buffers in LDS (TileLaunch::buffered)
     // exact screening of the block-padded rows
     const double* vbra;
     const double* vket;
@@ -552,12 +553,17 @@ __host__ __device__ constexpr int tile_min_waves()
     return L <= 1 ? 4 : L == 2 ? 3 : L <= 4 ? 2 : 1;
 }
 
-// LDS doubles of one density's work area: the strips, the J_MN copies and, for
-// a single density, the wavefronts' J_PQ buffers (several densities add J_PQ
-// straight to the accumulators: the buffers would not fit for the d classes)
-__host__ __device__ constexpr int tile_work(int rows, int nbf, int nab, int ncd, int waves)
+// LDS doubles of one density's work area: the strips, the J_MN copies and the
+// J_PQ buffers of `bufs` wavefronts.  Without buffers (0) the wavefronts add
+// J_PQ straight to the accumulators: for several densities, where the buffers
+// would not fit for the d classes, and for one density of a molecule whose
+// strips leave no room for them -- (dd|dd) from 1368 functions on.  There the
+// class takes 23.4 ms of C96H24's build (1464 functions) without the buffers,
+// 46.8 ms with global atomics for all of J and K (eri_kernel); buffers for
+// three of its four wavefronts, which would fit, gave 23.0 ms.
+__host__ __device__ constexpr int tile_work(int rows, int nbf, int nab, int ncd, int bufs)
 {
-    return rows * nbf + GTF_JMN_COPIES * nab + waves * ncd * 64;
+    return rows * nbf + GTF_JMN_COPIES * nab + bufs * ncd * 64;
 }
 
 // One class's tile kernel.  EX = false: a thread owns NC bra components and
@@ -583,7 +589,7 @@ __device__ __forceinline__ void tile_kernel_body(const EriArgs& a)
     const double* boys = tile_boys<L, BLDS>(a, smem, work);
     // the bra shells' density rows beside the work areas (BLDS): the digestion
     // gathers from them at the kets' columns
-    const bool buffered = a.nd == 1;
+    const bool buffered = a.jpq_lds;
     const int wsz = tile_work(NA + NB, a.nbf, NAB, NCD, buffered ? NT / 64 : 0);
     double* drow = work + (long)a.nd * wsz;
     const long long t_begin = (long long)wall_clock64();

@@ -100,6 +100,40 @@ def test_fock_edges(g, sto3g, tmp_path, nprim, natoms):
     assert max(err, err2) < FOCK_TOL
 
 
+# 1380 functions: the strips of (dd|dd) leave no room for the wavefronts' J_PQ
+# buffers in LDS (above 1367), and the class keeps its tiles without them; its
+# Schwarz values are 0.67 and 0.15, so a threshold of 0.2 sends a part to FP32
+@gpu
+@pytest.mark.parametrize("tau", [0.0, 0.2])
+def test_fock_without_jpq_buffers(g, tmp_path, tau):
+    gbs, xyz = str(tmp_path / "b.gbs"), str(tmp_path / "m.xyz")
+    with open(gbs, "w") as fh:
+        fh.write("spherical\n\n****\nH     0\nS   1   1.00\n  0.75  1.0\nD   1   1.00\n  0.75  1.0\n****\n")
+    with open(xyz, "w") as fh:
+        fh.write("230\n\n")
+        for k in range(230):
+            i = k // 2
+            fh.write("H %.6f %.6f %.6f\n" % (9.0 * (i % 5) + 0.75 * (k % 2), 9.0 * (i // 5 % 5) + 0.1 * (i % 3), 9.0 * (i // 25)))
+    b, ob = g.BasisSet(gbs, xyz), oracle.Basis(gbs, xyz)
+    assert b.nbf == 1380
+    a = np.random.default_rng(78).normal(size=(b.nbf, b.nbf))
+    D = 0.1 * (a + a.T)
+    pf = g.PFock(b)
+    pf.set_precision(tau)
+    kernel = pf.class_kernel(20)
+    err = np.abs(pf.fock(D) - sum(ob.fock(D)[:2])).max()
+    low = pf.mixed_counts()[0][20]
+    pf.close()
+    print("fock 1380, tau %g: %s, %d quartets in FP32, %.2e" % (tau, kernel, low, err))
+    assert kernel.startswith("eri_jk_tile_kernel<2, 2, 2, 2,")
+    if tau == 0.0:
+        assert err < FOCK_TOL
+    else:
+        # an integral below tau is off by the FP32 rounding of about 16 sums;
+        # a Fock element adds up to n^2 of them, with errors of either sign
+        assert low > 0 and err < 16 * 2.0**-24 * tau * b.nbf * np.abs(D).max()
+
+
 # one tile, a remainder of two, exact tiles, several tiles
 @gpu
 @pytest.mark.parametrize("n", [2, 32, 34, 64, 66, 130])
