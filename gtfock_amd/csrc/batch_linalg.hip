@@ -18,17 +18,19 @@
 // (gemm_tile.h).  A molecule is skipped when skip[m] != 0 or, during
 // purification, when it has already converged (done[m] >= 0); fp32[m] ==
 // GTF_LOW_FP32 selects the FP32 MFMA tile for it, GTF_LOW_SPLIT leaves it to
-// the split-BF16 products.
+// the split-BF16 products.  above: molecules of a larger leading dimension
+// only (the others are bgemm_rows_kernel's).
 template <int TRANSB>
 __global__ __launch_bounds__(256) void bgemm_kernel(const long* __restrict__ poff, const int* __restrict__ pld,
                                                     const int* __restrict__ skip, const int* __restrict__ done,
-                                                    const int* __restrict__ fp32, const double* __restrict__ A0,
-                                                    const double* __restrict__ B0, double* __restrict__ C0)
+                                                    const int* __restrict__ fp32, int above,
+                                                    const double* __restrict__ A0, const double* __restrict__ B0,
+                                                    double* __restrict__ C0)
 {
     const int m = blockIdx.z;
     const int ld = pld[m];
     const int row0 = blockIdx.y * GEMM_GT, col0 = blockIdx.x * GEMM_GT;
-    if (row0 >= ld || col0 >= ld || (skip && skip[m]) || (done && done[m] >= 0)) return;
+    if (row0 >= ld || col0 >= ld || ld <= above || (skip && skip[m]) || (done && done[m] >= 0)) return;
     const long o = poff[m];
     if (fp32 && fp32[m] == GTF_LOW_SPLIT) return;  // the split-BF16 products (ozaki.hip) cover it
     if (fp32 && fp32[m] == GTF_LOW_FP32) gemm_tile<TRANSB, true>(ld, A0 + o, B0 + o, C0 + o, row0, col0);
@@ -50,7 +52,7 @@ __device__ __forceinline__ double block_reduce(double v, double* sh, Op op)
     return r;
 }
 
-// C_m = A_m * B_m^T, every tile
+// C_m = A_m * B_m^T, every tile, of the molecules up to ROWS_MAX_LD
 __global__ __launch_bounds__(ROWS_THREADS) void bgemm_rows_kernel(const long* __restrict__ poff, const int* __restrict__ pld,
                                                          const int* __restrict__ skip, const int* __restrict__ done,
                                                          const double* __restrict__ A0, const double* __restrict__ B0,
@@ -58,7 +60,7 @@ __global__ __launch_bounds__(ROWS_THREADS) void bgemm_rows_kernel(const long* __
 {
     __shared__ double red[ROWS_W][ROWS_T * ROWS_T];
     const int m = blockIdx.z, ld = pld[m], row0 = blockIdx.y * ROWS_T, col0 = blockIdx.x * ROWS_T;
-    if (row0 >= ld || col0 >= ld || (skip && skip[m]) || (done && done[m] >= 0)) return;
+    if (row0 >= ld || col0 >= ld || ld > ROWS_MAX_LD || (skip && skip[m]) || (done && done[m] >= 0)) return;
     const long o = poff[m];
     rows_tile(ld, A0 + o, B0 + o, row0, col0, red);
     for (int k = threadIdx.x; k < ROWS_T * ROWS_T; k += ROWS_THREADS) C0[o + (long)(row0 + k / ROWS_T) * ld + col0 + k % ROWS_T] = red[0][k];
@@ -516,15 +518,19 @@ int gtf_bgemm(hipStream_t st, const BatchLayout& L, const int* skip, const int* 
               const double* B, double* C, int transB, const int* fp32)
 {
     if (L.nmol <= 0) return 0;
-    if (transB && !fp32 && L.maxpld <= ROWS_MAX_LD) {
-        dim3 tiles(L.maxpld / ROWS_T, L.maxpld / ROWS_T, L.nmol);
-        bgemm_rows_kernel<<<tiles, ROWS_THREADS, 0, st>>>(L.poff, L.pld, skip, done, A, B, C);
+    // the two A B^T kernels add in different orders, so each molecule takes the
+    // one of its own size, whatever shares the batch
+    int above = 0;
+    if (transB && !fp32) {
+        above = ROWS_MAX_LD;
+        const int t = std::min(L.maxpld, ROWS_MAX_LD) / ROWS_T;
+        bgemm_rows_kernel<<<dim3(t, t, L.nmol), ROWS_THREADS, 0, st>>>(L.poff, L.pld, skip, done, A, B, C);
         GTF_CHECK(hipGetLastError());
-        return 0;
+        if (L.maxpld <= ROWS_MAX_LD) return 0;
     }
     dim3 grid(L.maxpld / GEMM_GT, L.maxpld / GEMM_GT, L.nmol);
-    if (transB) bgemm_kernel<1><<<grid, 256, 0, st>>>(L.poff, L.pld, skip, done, fp32, A, B, C);
-    else bgemm_kernel<0><<<grid, 256, 0, st>>>(L.poff, L.pld, skip, done, fp32, A, B, C);
+    if (transB) bgemm_kernel<1><<<grid, 256, 0, st>>>(L.poff, L.pld, skip, done, fp32, above, A, B, C);
+    else bgemm_kernel<0><<<grid, 256, 0, st>>>(L.poff, L.pld, skip, done, fp32, above, A, B, C);
     GTF_CHECK(hipGetLastError());
     return 0;
 }

@@ -164,6 +164,34 @@ def test_dgemm_edges(g, n):
     assert (np.abs(g.dgemm(A, B, transB=True) - A @ B.T) <= bound).all()
 
 
+# a molecule's products are those of its own size, whatever shares the batch:
+# 36 functions alone and beside 258 and 516 (the matrices are padded to a
+# multiple of 64; the row products end at 512).  The regrouped batch carries S,
+# H and X over, and the first build is of a zero density, so its results are exact.
+@gpu
+@pytest.mark.parametrize("large", [43, 86])
+def test_batch_products_do_not_depend_on_the_batch(g, tmp_path, large):
+    gbs = _basis(tmp_path / "b.gbs", (2, 2, 2))
+    with open(gbs) as fh:
+        text = fh.read()
+    with open(gbs, "w") as fh:  # s and d: six functions an atom
+        fh.write(text[:text.index("P   2")] + text[text.index("D   2"):])
+    small = g.BasisSet(gbs, _hydrogens(tmp_path / "s.xyz", 6))
+    big = g.BasisSet(gbs, _hydrogens(tmp_path / "l.xyz", large))
+    assert (small.nbf, big.nbf) == (36, 6 * large)
+    alone = g.Batch([small])
+    alone.scf_begin(max_iters=3)
+    beside, origin = alone.regroup([big])
+    assert list(origin) == [0, -1]
+    alone.scf_step()
+    beside.scf_step()
+    D, E = alone.get_density()[0], beside.get_density()[0]
+    alone.close()
+    beside.close()
+    assert np.abs(D).max() > 0.1
+    assert np.array_equal(D, E)
+
+
 # the symmetric update of the split products: one tile, remainders, several
 # tiles; the last iterations are FP64, so the projector is as exact as theirs
 @gpu
