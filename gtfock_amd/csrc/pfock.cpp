@@ -602,7 +602,7 @@ int gtf_pfock_class_info(PFock_t pf, int cls, int* info)
     const bool ex = pf->sys.exchanged(cls);
     info[8] = ex ? 1 : 0;
     info[9] = ex ? ci->nc_t : 0;
-    info[10] = pf->sys.shape[cls].boys_lds;
+    info[10] = pf->sys.ntiles[cls] > 0 && pf->sys.tile_launch(cls, 1, 1).staged ? 1 : 0;
     return 0;
 }
 

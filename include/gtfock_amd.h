@@ -94,8 +94,10 @@ int gtf_pfock_class_times(PFock_t pfock, double *ms, long *launches);
 
 /* Kernel shape of quartet class cls: info[11] = {La, Lb, Lc, Ld, bra
  * components per thread NC, threads per quartet, FP64 bra-row tiles, FP32
- * bra-row tiles, exchanged, ket components per thread NCT, boys_lds}; with
- * no tiles the class runs eri_kernel<..., EPI_JK>, else
+ * bra-row tiles, exchanged, ket components per thread NCT, 1 if the launch
+ * of one density stages the Boys table and density rows in LDS (asked for by
+ * the shape's boys_lds and they fit)}; NC and the threads are those of the
+ * kernel that runs: with no tiles eri_kernel<..., EPI_JK>, else
  * eri_jk_tile_kernel<La, Lb, Lc, Ld, NC, double / float, boys_lds>, or
  * eri_jk_tile_t_kernel<La, Lb, Lc, Ld, NCT, double / float, boys_lds> when
  * exchanged = 1. */

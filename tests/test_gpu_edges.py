@@ -134,6 +134,22 @@ def test_fock_without_jpq_buffers(g, tmp_path, tau):
         assert low > 0 and err < 16 * 2.0**-24 * tau * b.nbf * np.abs(D).max()
 
 
+# the kernel named is the one launched: (dd|dd) stages the Boys table and ten
+# density rows in LDS (160 KB) beside its ten exchange rows up to 521 functions
+@gpu
+@pytest.mark.parametrize("natoms,staged", [(86, "true"), (88, "false")])
+def test_class_kernel_names_the_staging(g, tmp_path, natoms, staged):
+    gbs = str(tmp_path / "b.gbs")
+    with open(gbs, "w") as fh:
+        fh.write("spherical\n\n****\nH     0\nS   1   1.00\n  0.75  1.0\nD   1   1.00\n  0.75  1.0\n****\n")
+    b = g.BasisSet(gbs, _hydrogens(tmp_path / "m.xyz", natoms))
+    assert b.nbf == 6 * natoms
+    pf = g.PFock(b)
+    assert pf.tile_shape(20)["boys_lds"] == 1
+    assert pf.class_kernel(20) == "eri_jk_tile_kernel<2, 2, 2, 2, 1, double, %s>" % staged
+    pf.close()
+
+
 # one tile, a remainder of two, exact tiles, several tiles
 @gpu
 @pytest.mark.parametrize("n", [2, 32, 34, 64, 66, 130])
