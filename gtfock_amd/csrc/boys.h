@@ -31,44 +31,18 @@
 // 2e-15, 3e-13, 6e-12 and 8e-9 at most for m = 1, 3, 4 and 8.
 //   M <= BOYS_FAST_M: 2^n times the hardware's 2^f in FP32, good to 1e-7, which
 //     is 1e-18 of F_m, a hundredth of its last bit (largest error over 36..45
-//     the same as with libm's exp).  The table for these orders too: C54H18
-//     189 ms against 186.
-//   above: the same table, for T - BOYS_TMAX, in FP64; from 2 BOYS_TMAX on
-//     exp(-T) is below 1e-19 of F_m.  (FP32: 3.0e-15 of F_8, FP64 2.8e-15.)
+//     the same as with libm's exp).
+//   above: 2^n times the series of exp(r), |r| <= ln 2 / 2, to r^9 in FP64, good
+//     to 1e-11.  (FP32: 3.0e-15 of F_8, FP64 2.8e-15.)  The table for T -
+//     BOYS_TMAX instead cost (dd|dd) 11 %: its one wavefront per SIMD waits for
+//     the load.
 #define BOYS_FAST_M 4
-#define BOYS_EXP_TMAX 2.3195228302435696e-16  // exp(-BOYS_TMAX)
-
-// exp(-u) for 0 <= u <= BOYS_TMAX, at grid point i with dt = T0 - u
-template <int M, bool COLS>
-__device__ __forceinline__ double boys_exp(const double* __restrict__ slab, int i, double dt)
-{
-    const double e0 = slab[(COLS ? 1 : BOYS8_NM - M) * BOYS8_SLAB + i];
-    double x = fma(dt, 1.0 / 40320.0, 1.0 / 5040.0);
-    x = fma(x, dt, 1.0 / 720.0);
-    x = fma(x, dt, 1.0 / 120.0);
-    x = fma(x, dt, 1.0 / 24.0);
-    x = fma(x, dt, 1.0 / 6.0);
-    x = fma(x, dt, 0.5);
-    x = fma(x, dt, 1.0);
-    return fma(e0 * x, dt, e0);
-}
-
 template <int M, bool COLS = false>
 __device__ __forceinline__ void boys_eval8(double T, double* F, const double* __restrict__ slab)
 {
-    // above BOYS_FAST_M one table exponential serves both sides of the branch,
-    // which the lanes of a wavefront mostly disagree on
-    constexpr bool SHARED = M > BOYS_FAST_M;
-    const bool near = T < BOYS_TMAX;
-    int i = 0;
-    double dt = 0.0, e = 0.0;
-    if (SHARED || near) {
-        const double u = near ? T : fmin(T - BOYS_TMAX, BOYS_TMAX);
-        i = (int)(u * BOYS8_INV_DELTA + 0.5);
-        dt = fma((double)i, BOYS8_DELTA, -u);
-        if constexpr (M > 0) e = boys_exp<M, COLS>(slab, i, dt);
-    }
-    if (near) {
+    if (T < BOYS_TMAX) {
+        const int i = (int)(T * BOYS8_INV_DELTA + 0.5);
+        const double dt = fma((double)i, BOYS8_DELTA, -T);
         const double2* r = reinterpret_cast<const double2*>(slab) + i * (COLS ? 1 : BOYS8_NTERM / 2);
         constexpr int S = COLS ? BOYS8_NGRID : 1;
         const double2 c01 = r[0], c23 = r[S], c45 = r[2 * S], c67 = r[3 * S];
@@ -81,6 +55,15 @@ __device__ __forceinline__ void boys_eval8(double T, double* F, const double* __
         f = fma(f, dt, c01.x);
         F[M] = f;
         if constexpr (M > 0) {
+            const double e0 = slab[(COLS ? 1 : BOYS8_NM - M) * BOYS8_SLAB + i];
+            double x = fma(dt, 1.0 / 40320.0, 1.0 / 5040.0);
+            x = fma(x, dt, 1.0 / 720.0);
+            x = fma(x, dt, 1.0 / 120.0);
+            x = fma(x, dt, 1.0 / 24.0);
+            x = fma(x, dt, 1.0 / 6.0);
+            x = fma(x, dt, 0.5);
+            x = fma(x, dt, 1.0);
+            const double e = fma(e0 * x, dt, e0);
             const double t2 = T + T;
             static_for<0, M>([&](auto k) {
                 constexpr int m = M - 1 - decltype(k)::value;
@@ -91,13 +74,24 @@ __device__ __forceinline__ void boys_eval8(double T, double* F, const double* __
         const double rt = rsqrt_nr(T);
         F[0] = 0.88622692545275801365 * rt;  // sqrt(pi)/2
         if constexpr (M > 0) {
-            if constexpr (SHARED) {
-                e *= T < 2.0 * BOYS_TMAX ? BOYS_EXP_TMAX : 0.0;
+            const double y = T * -1.4426950408889634074;  // -log2(e)
+            const double n = rint(y);
+            double x;
+            if constexpr (M <= BOYS_FAST_M) {
+                x = (double)__builtin_amdgcn_exp2f((float)(y - n));
             } else {
-                const double y = T * -1.4426950408889634074;  // -log2(e)
-                const double n = rint(y);
-                e = ldexp((double)__builtin_amdgcn_exp2f((float)(y - n)), (int)n);
+                const double r = fma(n, -0.69314718055994530942, -T);  // -ln(2)
+                x = fma(r, 1.0 / 362880.0, 1.0 / 40320.0);
+                x = fma(x, r, 1.0 / 5040.0);
+                x = fma(x, r, 1.0 / 720.0);
+                x = fma(x, r, 1.0 / 120.0);
+                x = fma(x, r, 1.0 / 24.0);
+                x = fma(x, r, 1.0 / 6.0);
+                x = fma(x, r, 0.5);
+                x = fma(x, r, 1.0);
+                x = fma(x, r, 1.0);
             }
+            const double e = ldexp(x, (int)n);
             const double h = 0.5 * rt * rt;
             static_for<1, M + 1>([&](auto k) {
                 constexpr int m = decltype(k)::value;
