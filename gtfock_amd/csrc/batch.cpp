@@ -1092,9 +1092,9 @@ double gtf_batch_job_bytes(BasisSet_t basis)
             most[type] = std::max(most[type], np);
             // ket record of a primitive pair (KetView)
             record[type] = 16.0 * KetView::rec(nnz) + 8.0 * ((KetView::full(type) ? full : 0) + 1);
-            // per primitive pair: (p, P), its Schwarz bound, full and compact E
-            // in both precisions, the ket record with the padding of its block
-            pairs += np * (40.0 + 12.0 * (full + nnz) + 1.25 * record[type]) + 128.0;
+            // per primitive pair: (p, P), its Schwarz bound, full E, compact E in
+            // both precisions, the ket record with the padding of its block
+            pairs += np * (40.0 + 8.0 * full + 12.0 * nnz + 1.25 * record[type]) + 128.0;
         }
     // a type's kets are padded to 64 in every primitive-count bucket
     for (int t = 0; t < GTF_NPAIRTYPES; t++)

@@ -244,7 +244,7 @@ void GtfSystem::dfree(void* p)
 
 PairView GtfSystem::pair_view() const
 {
-    return PairView{d_s1, d_s2, d_pnprim, d_ppoff, d_peoff, d_prim, d_E, d_pzoff, d_Ez, d_pq, d_Ef, d_Ezf, 0.0};
+    return PairView{d_s1, d_s2, d_pnprim, d_ppoff, d_peoff, d_prim, d_E, d_pzoff, d_Ez, d_pq, d_Ezf, 0.0};
 }
 
 static int launch(eri_kernel_t fn, EriArgs& a, int blocks, hipStream_t st, size_t lds = 0, int threads = 256)
@@ -751,9 +751,13 @@ int GtfSystem::build_tiles()
     SYS_CHECK(hipStreamSynchronize(stream));
     if (tau > 0.0 && !d_Ezf) {
         // the FP32 tiles read the bra coefficients as scalars, already rounded
-        d_Ef = dalloc<float>(nE);
-        d_Ezf = dalloc<float>(nEz);
-        if (!d_Ef || !d_Ezf || gtf_round_f32(stream, d_E, nE, d_Ef) || gtf_round_f32(stream, d_Ez, nEz, d_Ezf)) return -1;
+        float* f = dalloc<float>(nEz);
+        if (!f) return -1;
+        if (gtf_round_f32(stream, d_Ez, nEz, f)) {
+            dfree(f);
+            return -1;
+        }
+        d_Ezf = f;
     }
     // fill the shared prefix and segment-maximum caches first: the classes
     // are then cut on host threads that only read shared state

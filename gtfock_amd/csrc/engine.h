@@ -65,7 +65,7 @@ struct GtfSystem {
     double* d_E = nullptr;
     long* d_pzoff = nullptr;
     double* d_Ez = nullptr;
-    float *d_Ef = nullptr, *d_Ezf = nullptr;  // rounded copies, made with the first FP32 tiles
+    float* d_Ezf = nullptr;  // rounded copy, made with the first FP32 tiles
     long nprimpairs = 0, nE = 0, nEz = 0, nprimpairs_kept = 0;
     // primitive-pair screening threshold on max |E| of a pair block
     double prim_eps = 1e-20;

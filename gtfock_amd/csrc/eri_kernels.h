@@ -599,7 +599,9 @@ __device__ __forceinline__ void tile_kernel_body(const EriArgs& a)
     int run0, nrun, bra, oM, oN, f1, nbf, rb;
     long mat;
     double vb;
-    BraRef<Real> br;
+    // the full coefficients are in FP64 only
+    using Coef = std::conditional_t<LOW && (STATIC || EX), float, double>;
+    BraRef<Coef> br;
     br.peps = a.pv.peps;
     // reads tile `task` (and its density rows); false when there is none
     auto open_tile = [&](int task) GTF_INLINE {
@@ -621,7 +623,7 @@ __device__ __forceinline__ void tile_kernel_body(const EriArgs& a)
         br.n = h.nprim;
         br.prim = as_const((const double*)(a.pv.prim + h.prim));
         br.q = as_const(a.pv.q + h.prim);
-        if constexpr (LOW) br.E = as_const(STATIC || EX ? a.pv.Ezf : a.pv.Ef) + h.E;
+        if constexpr (std::is_same_v<Coef, float>) br.E = as_const(a.pv.Ezf) + h.E;
         else br.E = as_const(STATIC || EX ? a.pv.Ez : a.pv.E) + h.E;
         if constexpr (BLDS)
             for (int d = 0; d < a.nd; d++) {
@@ -764,7 +766,7 @@ __device__ __forceinline__ void tile_kernel_body(const EriArgs& a)
                         finish(std::integral_constant<int, 0>{}, std::integral_constant<int, NAB>{},
                                std::integral_constant<int, -1>{}, std::integral_constant<int, 1>{}, acc, sp);
                     } else if constexpr (!STATIC) {
-                        BraRef<Real> b1 = br;
+                        BraRef<Coef> b1 = br;
                         b1.E += sp * S::HAB;
                         Real acc[1][NCD];
                         eri_lane<LA, LB, LC, LD, -1, 1, Real, BLDS>(b1, kr, j0, js, boys, acc);

@@ -264,7 +264,9 @@ __device__ __forceinline__ const_as<T>* as_const(const T* p)
 }
 
 // the bra pair of a tile (wave-uniform); Coef: the type its coefficients are
-// read in (float copies for the FP32 form)
+// read in (the FP32 form has a rounded copy of the compact ones; the full ones,
+// which only a run-time component of a d-p or d-d bra reads, it rounds as it
+// reads them)
 template <typename Coef>
 struct BraRef {
     const_as<double>* prim;  // (p, Px, Py, Pz) per primitive pair
@@ -374,8 +376,8 @@ __device__ __forceinline__ void ket_loop(const KetRef& k, int j0, int js, Body&&
 // points at in the full layout.  The bra contraction is summed over the bra
 // primitives before the ket coefficients are applied, except for a d-d bra
 // (one primitive pair in practice), where it would only hold registers.
-template <int LA, int LB, int LC, int LD, int A0, int NC, typename Real, bool BLDS>
-__device__ __forceinline__ void eri_lane(const BraRef<Real>& b, const KetRef& k, int j0, int js,
+template <int LA, int LB, int LC, int LD, int A0, int NC, typename Real, bool BLDS, typename Coef>
+__device__ __forceinline__ void eri_lane(const BraRef<Coef>& b, const KetRef& k, int j0, int js,
                                          const double* __restrict__ boys_slab,
                                          Real (&acc)[NC][EriShape<LA, LB, LC, LD>::NCD])
 {
@@ -426,13 +428,13 @@ __device__ __forceinline__ void eri_lane(const BraRef<Real>& b, const KetRef& k,
             }
             static_for<0, NC>([&](auto c_) GTF_INLINE {
                 constexpr int c = decltype(c_)::value;
-                const_as<Real>* E = b.E + (long)i * ESTRIDE;
+                const_as<Coef>* E = b.E + (long)i * ESTRIDE;
                 static_for<0, HCD>([&](auto h2_) GTF_INLINE {
                     constexpr int h2 = decltype(h2_)::value;
                     Real v = SUM_BRA ? W[c][h2] : Real(0);
                     static_for<0, HAB>([&](auto h1_) GTF_INLINE {
                         constexpr int h1 = decltype(h1_)::value;
-                        if constexpr (A0 < 0) v += E[h1] * R[hsum<h1, h2>()];
+                        if constexpr (A0 < 0) v += Real(E[h1]) * R[hsum<h1, h2>()];
                         else if constexpr (TA::data.nz[A0 < 0 ? 0 : A0 + c][h1])
                             v += E[TA::data.pos[A0 < 0 ? 0 : A0 + c][h1]] * R[hsum<h1, h2>()];
                     });

@@ -163,7 +163,7 @@ struct PairView {
     const long* zoff;    // offset into Ez[]
     const double* Ez;    // the same, structural nonzeros only (herm_nz_pos order)
     const double* q;     // Schwarz bound per primitive pair (a pair's primitives in descending order)
-    const float *Ef, *Ezf;  // E and Ez rounded to FP32 (systems with FP32 tiles)
+    const float* Ezf;    // Ez rounded to FP32 (systems with FP32 tiles)
     double peps;         // primitive quartets with q_bra q_ket < peps are skipped (0: none)
 };
 

@@ -134,6 +134,37 @@ def test_fock_without_jpq_buffers(g, tmp_path, tau):
         assert low > 0 and err < 16 * 2.0**-24 * tau * b.nbf * np.abs(D).max()
 
 
+# Hermite coefficients of a primitive pair, all and structural nonzeros
+FULL = {"ss": 1, "ps": 12, "pp": 90, "ds": 50, "dp": 300, "dd": 875}
+NONZERO = {"ss": 1, "ps": 6, "pp": 33, "ds": 24, "dp": 122, "dd": 391}
+
+
+def _prim_pairs(nprim, natoms):
+    """{pair type: primitive pairs} of natoms atoms that each have an s, a p and a
+    d shell of nprim primitives."""
+    out = {}
+    for t in FULL:
+        a, b = ("spd".index(c) for c in t)
+        out[t] = (natoms * (natoms + 1) // 2 if a == b else natoms * natoms) * nprim[a] * nprim[b]
+    return out
+
+
+# the FP32 tiles add a rounded copy of the nonzero coefficients, and lists of a
+# quarter of it at most (a run of 64 kets has 20 bytes)
+@gpu
+def test_mixed_precision_memory(g, tmp_path):
+    nprim, natoms = (4, 4, 4), 20
+    b = g.BasisSet(_basis(tmp_path / "b.gbs", nprim), _hydrogens(tmp_path / "m.xyz", natoms))
+    pf = g.PFock(b)
+    before = pf.stats()["device_bytes"]
+    pf.set_precision(1e-4)
+    added = pf.stats()["device_bytes"] - before
+    pf.close()
+    copy = sum(4 * NONZERO[t] * n for t, n in _prim_pairs(nprim, natoms).items())
+    print("FP64 %.1f MB, mixed adds %.1f MB, coefficients %.1f MB" % (before / 1e6, added / 1e6, copy / 1e6))
+    assert added < 1.25 * copy
+
+
 # the kernel named is the one launched: (dd|dd) stages the Boys table and ten
 # density rows in LDS (160 KB) beside its ten exchange rows up to 521 functions
 @gpu
