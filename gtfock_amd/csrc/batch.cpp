@@ -1081,33 +1081,48 @@ double gtf_batch_job_bytes(BasisSet_t basis)
     if (!basis) return -1.0;
     const BasisSet* b = basis;
     double pairs = 0.0, blocks = 0.0;
-    int most[GTF_NPAIRTYPES] = {0};  // primitive pairs of a shell pair, by type
-    double record[GTF_NPAIRTYPES] = {0.0};
+    constexpr int NB = GtfSystem::NBUCKET;
+    static const int top[NB] = {1, 4, 12, 32, INT32_MAX};  // the primitive-count buckets
+    // per type and bucket: kets, the most primitive pairs of one; per type:
+    // primitive pairs, ket record of one (KetView)
+    long kets[GTF_NPAIRTYPES][NB] = {};
+    int most[GTF_NPAIRTYPES][NB] = {};
+    double prims[GTF_NPAIRTYPES] = {}, record[GTF_NPAIRTYPES] = {};
     for (int s = 0; s < b->nshells; s++)
         for (int t = 0; t <= s; t++) {
             int la = b->L[s], lb = b->L[t];
             if (lb > la) std::swap(la, lb);
             const int np = b->nprim[s] * b->nprim[t], type = pair_type(la, lb);
             const int full = nsph(la) * nsph(lb) * nherm(la + lb), nnz = herm_nnz_lookup(la, lb);
-            most[type] = std::max(most[type], np);
-            // ket record of a primitive pair (KetView)
+            int k = 0;
+            while (np > top[k]) k++;
+            kets[type][k]++;
+            most[type][k] = std::max(most[type][k], np);
+            prims[type] += np;
             record[type] = 16.0 * KetView::rec(nnz) + 8.0 * ((KetView::full(type) ? full : 0) + 1);
             // per primitive pair: (p, P), its Schwarz bound, full E, compact E in
-            // both precisions, the ket record with the padding of its block
-            pairs += np * (40.0 + 8.0 * full + 12.0 * nnz + 1.25 * record[type]) + 128.0;
+            // both precisions
+            pairs += np * (40.0 + 8.0 * full + 12.0 * nnz) + 128.0;
         }
-    // a type's kets are padded to 64 in every primitive-count bucket
-    for (int t = 0; t < GTF_NPAIRTYPES; t++)
-        for (int k = 0; k < GtfSystem::NBUCKET; k++) {
-            static const int top[GtfSystem::NBUCKET] = {1, 4, 12, 32, INT32_MAX};
-            if (most[t] > (k > 0 ? top[k - 1] : 0)) blocks += 64.0 * std::min(top[k], most[t]) * record[t];
+    // the ket records of the molecule alone, its 64-ket blocks as long as their
+    // bucket's most primitives; beside others it shares blocks (pack_kets)
+    for (int t = 0; t < GTF_NPAIRTYPES; t++) {
+        double slots = 0.0;
+        long left = 0;  // of the open block
+        for (int k = NB - 1; k >= 0; k--) {
+            if (kets[t][k] >= GTF_KET_OWN) left = 0;
+            const long open = std::max(0L, kets[t][k] - left + GTF_KET_BLOCK - 1) / GTF_KET_BLOCK;
+            slots += (double)open * GTF_KET_BLOCK * most[t][k];
+            left += open * GTF_KET_BLOCK - kets[t][k];
         }
+        blocks += std::max(slots, 1.25 * prims[t]) * record[t];
+    }
     const double n = b->nbf, pl = ((b->nbf + 63) / 64) * 64;
     // + the split purification's BF16 slices of both operands at the most
     // slices (and their exponents and row maxima)
     const double split = 2.0 * 2.0 * OZ_SLICES_MAX * pl * pl + 4.0 * 8.0 * pl * pl / 64.0;
     // + the list-ordered density and J_PQ copies (an n x n matrix)
-    return pairs * 1.6 + blocks + 8.0 * (10.5 * n * n + (8.0 + 2.0 * B_MAX_DIIS) * pl * pl) + split + (1 << 20);
+    return (pairs + blocks) * 1.6 + 8.0 * (10.5 * n * n + (8.0 + 2.0 * B_MAX_DIIS) * pl * pl) + split + (1 << 20);
 }
 
 int gtf_batch_get_density(gtf_batch_t b, int m, double* D)

@@ -19,6 +19,8 @@
 #define GTF_NCLASSES 21
 // ket-list block re-sorted by primitive count (one wavefront)
 #define GTF_KET_BLOCK 64
+// kets of a segment whose records start a block of their own (KetView)
+#define GTF_KET_OWN 256
 
 // A tile of the J/K kernels is one bra pair and several runs of its kets:
 // TileHead.  A run is int4 (first ket, span word, chunk word, 0).
@@ -168,7 +170,7 @@ struct PairView {
 };
 
 // Ket side of one pair type's significant-pair list, in list order, for the
-// tile kernels: 64 kets of a segment form a block whose primitive pairs are
+// tile kernels: 64 kets form a block whose primitive pairs are
 // stored primitive by primitive, each as rec(nnz) rows of 64 double2 -- (p,
 // Px), (Py, Pz) and the compact Hermite coefficients two by two -- so that the
 // lanes of a wavefront, which hold consecutive kets, read whole lines.

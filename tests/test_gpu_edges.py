@@ -149,6 +149,28 @@ def _prim_pairs(nprim, natoms):
     return out
 
 
+# the molecules of a batch share the 64-ket blocks of the records: one molecule's
+# lists of 1 to 3 kets pad 64, sixty-four of them a few in a hundred
+@gpu
+def test_batch_memory_shares_ket_blocks(g, tmp_path):
+    nprim, natoms, nmol = (6, 3, 1), 2, 64
+    gbs, xyz = _basis(tmp_path / "b.gbs", nprim), _hydrogens(tmp_path / "m.xyz", natoms)
+    bases = [g.BasisSet(gbs, xyz) for _ in range(nmol)]
+    one, many = g.Batch(bases[:1]), g.Batch(bases)
+    used1, used = one.stats()["device_bytes"], many.stats()["device_bytes"]
+    one.close()
+    many.close()
+    # p, P, bound and both coefficient forms; the record with, for pp, ds and
+    # dp, the full form; a quarter more where a block mixes primitive counts
+    pairs = sum(n * (40 + 8 * (FULL[t] + NONZERO[t])
+                     + 1.25 * (8 + 16 * (2 + (NONZERO[t] + 1) // 2) + (8 * FULL[t] if t in ("pp", "ds", "dp") else 0)))
+                for t, n in _prim_pairs(nprim, natoms).items())
+    print("one %.2f MB, %d %.2f MB, a molecule's primitive pairs %.3f MB" % (used1 / 1e6, nmol, used / 1e6, pairs / 1e6))
+    # beside them what one holds at most, and 32 KB a molecule for lists, tiles
+    # and matrices
+    assert used < used1 + nmol * (pairs + 32768)
+
+
 # the FP32 tiles add a rounded copy of the nonzero coefficients, and lists of a
 # quarter of it at most (a run of 64 kets has 20 bytes)
 @gpu
