@@ -1080,7 +1080,7 @@ double gtf_batch_job_bytes(BasisSet_t basis)
 {
     if (!basis) return -1.0;
     const BasisSet* b = basis;
-    double pairs = 0.0, blocks = 0.0;
+    double pairs = 0.0, low = 0.0, blocks = 0.0;
     constexpr int NB = GtfSystem::NBUCKET;
     static const int top[NB] = {1, 4, 12, 32, INT32_MAX};  // the primitive-count buckets
     // per type and bucket: kets, the most primitive pairs of one; per type:
@@ -1094,15 +1094,29 @@ double gtf_batch_job_bytes(BasisSet_t basis)
             if (lb > la) std::swap(la, lb);
             const int np = b->nprim[s] * b->nprim[t], type = pair_type(la, lb);
             const int full = nsph(la) * nsph(lb) * nherm(la + lb), nnz = herm_nnz_lookup(la, lb);
-            int k = 0;
-            while (np > top[k]) k++;
-            kets[type][k]++;
-            most[type][k] = std::max(most[type][k], np);
-            prims[type] += np;
+            // records are kept of the primitive pairs that the set-up keeps: those
+            // of exp(-mu R^2) below 1e-26 are far under its threshold
+            double r2 = 0.0;
+            for (int d = 0; d < 3; d++) {
+                const double x = b->xyz[3 * b->atom[s] + d] - b->xyz[3 * b->atom[t] + d];
+                r2 += x * x;
+            }
+            int kept = 0, k = 0;
+            for (int i = 0; i < b->nprim[s]; i++)
+                for (int j = 0; j < b->nprim[t]; j++) {
+                    const double x = b->alpha[b->poff[s] + i], y = b->alpha[b->poff[t] + j];
+                    kept += x * y * r2 <= 60.0 * (x + y);
+                }
+            if (kept > 0) {
+                while (kept > top[k]) k++;
+                kets[type][k]++;
+                most[type][k] = std::max(most[type][k], kept);
+                prims[type] += kept;
+            }
             record[type] = 16.0 * KetView::rec(nnz) + 8.0 * ((KetView::full(type) ? full : 0) + 1);
-            // per primitive pair: (p, P), its Schwarz bound, full E, compact E in
-            // both precisions
-            pairs += np * (40.0 + 8.0 * full + 12.0 * nnz) + 128.0;
+            // per primitive pair: (p, P), its Schwarz bound, full and compact E
+            pairs += np * (40.0 + 8.0 * (full + nnz)) + 96.0;
+            low += 4.0 * np * nnz;  // the FP32 tiles' coefficients
         }
     // the ket records of the molecule alone, its 64-ket blocks as long as their
     // bucket's most primitives; beside others it shares blocks (pack_kets)
@@ -1115,14 +1129,15 @@ double gtf_batch_job_bytes(BasisSet_t basis)
             slots += (double)open * GTF_KET_BLOCK * most[t][k];
             left += open * GTF_KET_BLOCK - kets[t][k];
         }
-        blocks += std::max(slots, 1.25 * prims[t]) * record[t];
+        blocks += 1.1 * std::max(slots, 1.25 * prims[t]) * record[t];
     }
     const double n = b->nbf, pl = ((b->nbf + 63) / 64) * 64;
     // + the split purification's BF16 slices of both operands at the most
     // slices (and their exponents and row maxima)
     const double split = 2.0 * 2.0 * OZ_SLICES_MAX * pl * pl + 4.0 * 8.0 * pl * pl / 64.0;
-    // + the list-ordered density and J_PQ copies (an n x n matrix)
-    return (pairs + blocks) * 1.6 + 8.0 * (10.5 * n * n + (8.0 + 2.0 * B_MAX_DIIS) * pl * pl) + split + (1 << 20);
+    // the pairs' 0.6 covers the lists and tiles; + the list-ordered density and
+    // J_PQ copies (an n x n matrix)
+    return pairs * 1.6 + low + blocks + 8.0 * (10.5 * n * n + (8.0 + 2.0 * B_MAX_DIIS) * pl * pl) + split + (1 << 20);
 }
 
 int gtf_batch_get_density(gtf_batch_t b, int m, double* D)

@@ -187,6 +187,24 @@ def test_mixed_precision_memory(g, tmp_path):
     assert added < 1.25 * copy
 
 
+# the server admits jobs by this estimate: it covers what a batch of the molecule
+# allocates, and not 40 % more, or a budget holds fewer jobs than it could
+@gpu
+@pytest.mark.parametrize("mol", ["c10h22", "c54h18"])
+def test_job_estimate_is_close(g, gbs, mol_dir, mol):
+    b = g.BasisSet(gbs, str(mol_dir / (mol + ".xyz")))
+    est = g.lib().gtf_batch_job_bytes(b.h)
+    bt = g.Batch([b], tau=1e-4)
+    bt.set_purif_precision("split")
+    bt.scf_begin(max_iters=3)
+    bt.scf_step()
+    bt.scf_step()
+    used = bt.stats()["device_bytes"]
+    bt.close()
+    print("%s: estimate %.1f MB, allocated %.1f MB" % (mol, est / 1e6, used / 1e6))
+    assert used <= est <= 1.4 * used
+
+
 # the kernel named is the one launched: (dd|dd) stages the Boys table and ten
 # density rows in LDS (160 KB) beside its ten exchange rows up to 521 functions
 @gpu
