@@ -130,14 +130,12 @@ struct GtfSystem {
     int ntiles[GTF_NCLASSES] = {0}, ntiles_lo[GTF_NCLASSES] = {0};
     TileHead* d_tiles[GTF_NCLASSES] = {nullptr};     // FP64 tiles
     TileHead* d_tiles_lo[GTF_NCLASSES] = {nullptr};  // FP32 tiles
-    // their runs of kets, and the bra row of each run
+    // their runs of kets
     int4 *d_runs[GTF_NCLASSES] = {nullptr}, *d_runs_lo[GTF_NCLASSES] = {nullptr};
-    int *d_run_row[GTF_NCLASSES] = {nullptr}, *d_run_row_lo[GTF_NCLASSES] = {nullptr};
     int nruns[GTF_NCLASSES] = {0}, nruns_lo[GTF_NCLASSES] = {0};
     struct TileList {
         std::vector<TileHead> tiles;
         std::vector<int4> runs;
-        std::vector<int> run_row;
     };
     // launch of a class's n tiles digesting nd densities; staged: with the Boys
     // slab and the density rows in LDS (asked for by the shape and within

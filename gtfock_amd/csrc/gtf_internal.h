@@ -23,7 +23,7 @@
 #define GTF_KET_OWN 256
 
 // A tile of the J/K kernels is one bra pair and several runs of its kets:
-// TileHead.  A run is int4 (first ket, span word, chunk word, 0).
+// TileHead.  A run is int4 (first ket, span word, chunk word, bra row).
 // span word: kets, first component chunk and number of them
 #define GTF_RUN_SPAN(kets, sp0, spn) ((kets) | (sp0) << 15 | (spn) << 20)
 #define GTF_RUN_KETS(y) ((y) & 32767)

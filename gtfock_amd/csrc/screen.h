@@ -35,7 +35,6 @@ int gtf_pack_kets(hipStream_t st, const PairView& pv, const int* fstart, const K
 // runs over the same kets only the one holding chunk 0 of both kinds counts
 struct CensusArgs {
     const int4* runs;
-    const int* run_row;  // bra row of each run
     int nruns;
     const int* bra_list;
     const int* ket_list;

@@ -318,9 +318,8 @@ __global__ void fill_qlist_diag_kernel(int n, const int* __restrict__ ids, int2*
     if (k < n) q[k] = make_int2(ids[k], ids[k]);
 }
 
-// Primitive quartets the J/K kernels evaluate over the runs of a tile list
-// (run, bra row): for each quartet of a run that passes the
-// kernels' tests (Schwarz, one orientation in a diagonal class, the
+// Primitive quartets the J/K kernels evaluate over the runs of a tile list: for
+// each quartet of a run that passes the kernels' tests (Schwarz, one orientation in a diagonal class, the
 // precision split), the pairs (i, j) of bra and ket primitives with
 // q_i q_j >= peps when the class screens primitives, else all of them.
 // With both lists in descending order of q that is what the kernels' loops
@@ -330,7 +329,7 @@ __global__ __launch_bounds__(256) void prim_census_kernel(CensusArgs c)
 {
     const int4 t = c.runs[blockIdx.x];
     if (GTF_RUN_IC0(t.z) != 0 || GTF_RUN_SP0(t.y) != 0) return;
-    const int row = c.run_row[blockIdx.x];
+    const int row = t.w;
     const int bra = c.bra_list[row];
     const int nbp = c.pv.nprim[bra];
     const double* __restrict__ qb = c.pv.q + c.pv.poff[bra];
