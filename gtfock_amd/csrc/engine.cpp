@@ -754,9 +754,9 @@ int GtfSystem::build_tiles()
     if (tau > 0.0 && !d_Ezf) {
         // the FP32 tiles read the bra coefficients as scalars, already rounded
         float* f = dalloc<float>(nEz);
-        if (!f) return -1;
-        if (gtf_round_f32(stream, d_Ez, nEz, f)) {
+        if (!f || gtf_round_f32(stream, d_Ez, nEz, f)) {
             dfree(f);
+            drop_tiles(0, GTF_NCLASSES);  // cut for another tau
             return -1;
         }
         d_Ezf = f;
@@ -796,17 +796,35 @@ int GtfSystem::build_class_tiles(int cls)
     return upload_tiles(hv, lv, cls, cls + 1);
 }
 
-// Replaces the device tiles of the classes [c0, c1) by hv (FP64) and lv
-// (FP32), in one allocation and one copy; the stream must have no launch in
-// flight that reads the old ones.  An allocation that several classes share is
-// freed with the last of them.
-int GtfSystem::upload_tiles(const TileList* hv, const TileList* lv, int c0, int c1)
+// An allocation that several classes share is freed with the last of them; the
+// stream must have no launch in flight that reads it.
+void GtfSystem::free_tiles(int c0, int c1)
 {
     for (int c = c0; c < c1; c++) {
         void* old = tile_mem[c];
         tile_mem[c] = nullptr;
         if (old && std::find(tile_mem, tile_mem + GTF_NCLASSES, old) == tile_mem + GTF_NCLASSES) dfree(old);
     }
+}
+
+void GtfSystem::drop_tiles(int c0, int c1)
+{
+    free_tiles(c0, c1);
+    for (int c = c0; c < c1; c++) {
+        d_tiles[c] = d_tiles_lo[c] = nullptr;
+        d_runs[c] = d_runs_lo[c] = nullptr;
+        ntiles[c] = ntiles_lo[c] = nruns[c] = nruns_lo[c] = 0;
+        nq_lo[c] = 0;
+        nprimq_lo[c] = 0.0;
+    }
+}
+
+// Replaces the device tiles of the classes [c0, c1) by hv (FP64) and lv
+// (FP32), in one allocation and one copy.  Where that fails the classes are
+// left without tiles.
+int GtfSystem::upload_tiles(const TileList* hv, const TileList* lv, int c0, int c1)
+{
+    free_tiles(c0, c1);
     // every list's place; 64-byte aligned
     struct Part {
         const void* p;
@@ -822,7 +840,11 @@ int GtfSystem::upload_tiles(const TileList* hv, const TileList* lv, int c0, int 
                 size += (q.bytes + 63) / 64 * 64;
             }
     char* mem = dalloc<char>(size);
-    if (!mem) return -1;
+    if (!mem) {
+        drop_tiles(c0, c1);
+        return -1;
+    }
+    std::fill(tile_mem + c0, tile_mem + c1, (void*)mem);
     // gathered in one buffer for one copy, large ones by several threads in
     // pieces: the first touch of the pages takes longer than the copy to the
     // device (480 MB of the batch of 256 molecules: 106 ms in one thread)
@@ -841,10 +863,14 @@ int GtfSystem::upload_tiles(const TileList* hv, const TileList* lv, int c0, int 
     for (int t = 1; t < nth; t++) pool.emplace_back(work);
     work();
     for (std::thread& t : pool) t.join();
-    if (size) SYS_CHECK(hipMemcpyAsync(mem, host.get(), size, hipMemcpyHostToDevice, stream));
+    // the copy reads host
+    if ((size && hipMemcpyAsync(mem, host.get(), size, hipMemcpyHostToDevice, stream) != hipSuccess) ||
+        hipStreamSynchronize(stream) != hipSuccess) {
+        drop_tiles(c0, c1);
+        return -1;
+    }
     for (int c = c0; c < c1; c++) {
         const Part* q = part.data() + 4 * (c - c0);
-        tile_mem[c] = mem;
         d_tiles[c] = (TileHead*)(mem + q[0].at);
         d_runs[c] = (int4*)(mem + q[1].at);
         nruns[c] = (int)hv[c].runs.size();
@@ -852,8 +878,6 @@ int GtfSystem::upload_tiles(const TileList* hv, const TileList* lv, int c0, int 
         d_runs_lo[c] = (int4*)(mem + q[3].at);
         nruns_lo[c] = (int)lv[c].runs.size();
     }
-    // the upload reads host
-    SYS_CHECK(hipStreamSynchronize(stream));
     return 0;
 }
 

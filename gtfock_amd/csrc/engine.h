@@ -237,6 +237,9 @@ struct GtfSystem {
     int build_class_tiles(int cls);
     void cut_class_tiles(int cls, TileList& hv, TileList& lv);
     int upload_tiles(const TileList* hv, const TileList* lv, int c0, int c1);
+    void free_tiles(int c0, int c1);
+    // leaves the classes [c0, c1) without tiles: they run in FP64, by eri_kernel
+    void drop_tiles(int c0, int c1);
     void* tile_mem[GTF_NCLASSES] = {nullptr};  // the allocation that holds a class's tiles
     // CSR of molecule 0 in the reference layout (host)
     void csr(std::vector<int>& shellptr, std::vector<int>& shellid, std::vector<int>& shellrid,
