@@ -324,8 +324,11 @@ __global__ void bpurif_update_kernel(const long* __restrict__ poff, const int* _
 // The same with the means of the products and their transposes: the split
 // products are not symmetric, and the iterations amplify an antisymmetric part
 // of D (with it C54H18's SCF with split products took 24 builds, FP64's 21;
-// without it 21).  A workgroup takes a 32 x 32 tile of the lower triangle and
-// its mirror, transposed through LDS.
+// without it 21).  A workgroup takes a 32 x 32 tile and reads the mirrored ones
+// of D2 and D3 through LDS.  A mirrored element comes out the same bit for bit,
+// D being symmetric.  Bound by latency: with a tile and its mirror in one
+// workgroup, half as many of them and three barriers, a split purification of
+// n = 106 took 3.30 ms, now 3.15 (3.28 with the unsymmetric update).
 __global__ __launch_bounds__(256) void bpurif_update_sym_kernel(const long* __restrict__ poff, const int* __restrict__ pld,
                                                             const int* __restrict__ skip, const int* __restrict__ iters,
                                                             const double* __restrict__ stats, double* __restrict__ D0,
@@ -333,37 +336,30 @@ __global__ __launch_bounds__(256) void bpurif_update_sym_kernel(const long* __re
                                                             const double* __restrict__ D30, int it)
 {
     __shared__ double s2[ROWS_T][ROWS_T + 1], s3[ROWS_T][ROWS_T + 1];
-    const int m = blockIdx.y;
-    if ((skip && skip[m]) || (iters[m] >= 0 && iters[m] != it)) return;
-    const int ld = pld[m], t = blockIdx.x;
-    if (t >= tri_tiles(ld)) return;
-    int ti = (int)((sqrtf(8.0f * t + 1.0f) - 1.0f) * 0.5f);
-    while (ti * (ti + 1) / 2 > t) ti--;
-    while ((ti + 1) * (ti + 2) / 2 <= t) ti++;
-    const int tj = t - ti * (ti + 1) / 2;
+    const int m = blockIdx.z, ld = pld[m], row0 = blockIdx.y * ROWS_T, col0 = blockIdx.x * ROWS_T;
+    if (row0 >= ld || col0 >= ld || (skip && skip[m]) || (iters[m] >= 0 && iters[m] != it)) return;
+    constexpr int N = ROWS_T * ROWS_T / 256, STEP = 256 / ROWS_T;
     const double c = stats[3 * m + 1] / stats[3 * m + 2];
     double* D = D0 + poff[m];
     const double* D2 = D20 + poff[m];
     const double* D3 = D30 + poff[m];
     const int tx = threadIdx.x % ROWS_T, ty = threadIdx.x / ROWS_T;
-    const long lower = (long)ti * ROWS_T * ld + tj * ROWS_T, upper = (long)tj * ROWS_T * ld + ti * ROWS_T;
-    for (int r = ty; r < ROWS_T; r += 256 / ROWS_T) {
-        s2[r][tx] = D2[upper + (long)r * ld + tx];
-        s3[r][tx] = D3[upper + (long)r * ld + tx];
+    const long own = (long)(row0 + ty) * ld + col0 + tx, mirror = (long)(col0 + ty) * ld + row0 + tx;
+    double d[N], d2[N], d3[N];
+    for (int k = 0; k < N; k++) {
+        const long o = (long)k * STEP * ld;
+        d[k] = D[own + o];
+        d2[k] = D2[own + o];
+        d3[k] = D3[own + o];
+        s2[ty + k * STEP][tx] = D2[mirror + o];
+        s3[ty + k * STEP][tx] = D3[mirror + o];
     }
     __syncthreads();
-    double v[ROWS_T * ROWS_T / 256];
-    for (int r = ty, k = 0; r < ROWS_T; r += 256 / ROWS_T, k++) {
-        const long e = lower + (long)r * ld + tx;
-        const double d2 = 0.5 * (D2[e] + s2[tx][r]), d3 = 0.5 * (D3[e] + s3[tx][r]);
-        v[k] = c < 0.5 ? ((1.0 - 2.0 * c) * D[e] + (1.0 + c) * d2 - d3) / (1.0 - c) : ((1.0 + c) * d2 - d3) / c;
-        D[e] = v[k];
+    for (int k = 0; k < N; k++) {
+        const int r = ty + k * STEP;
+        const double x = 0.5 * (d2[k] + s2[tx][r]), y = 0.5 * (d3[k] + s3[tx][r]);
+        D[own + (long)k * STEP * ld] = c < 0.5 ? ((1.0 - 2.0 * c) * d[k] + (1.0 + c) * x - y) / (1.0 - c) : ((1.0 + c) * x - y) / c;
     }
-    if (ti == tj) return;
-    __syncthreads();
-    for (int r = ty, k = 0; r < ROWS_T; r += 256 / ROWS_T, k++) s2[r][tx] = v[k];
-    __syncthreads();
-    for (int r = ty; r < ROWS_T; r += 256 / ROWS_T) D[upper + (long)r * ld + tx] = s2[tx][r];
 }
 
 // The same after bpurif_product_kernel: every workgroup adds up the molecule's
@@ -579,8 +575,8 @@ int gtf_bpurif_update(hipStream_t st, const BatchLayout& L, const int* skip, con
                       double* D, const double* D2, const double* D3, int it, bool sym)
 {
     if (sym)
-        bpurif_update_sym_kernel<<<dim3(tri_tiles(L.maxpld), L.nmol), 256, 0, st>>>(L.poff, L.pld, skip, iters, stats,
-                                                                                  D, D2, D3, it);
+        bpurif_update_sym_kernel<<<dim3(L.maxpld / ROWS_T, L.maxpld / ROWS_T, L.nmol), 256, 0, st>>>(
+            L.poff, L.pld, skip, iters, stats, D, D2, D3, it);
     else
         bpurif_update_kernel<<<per_mol_grid(L.maxpld * L.maxpld, L.nmol), 256, 0, st>>>(L.poff, L.pld, skip, iters,
                                                                                       stats, D, D2, D3, it);
