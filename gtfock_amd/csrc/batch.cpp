@@ -1088,6 +1088,7 @@ double gtf_batch_job_bytes(BasisSet_t basis)
     long kets[GTF_NPAIRTYPES][NB] = {};
     int most[GTF_NPAIRTYPES][NB] = {};
     double prims[GTF_NPAIRTYPES] = {}, record[GTF_NPAIRTYPES] = {};
+    const bool has_d = std::find(b->L.begin(), b->L.end(), 2) != b->L.end();
     for (int s = 0; s < b->nshells; s++)
         for (int t = 0; t <= s; t++) {
             int la = b->L[s], lb = b->L[t];
@@ -1113,7 +1114,7 @@ double gtf_batch_job_bytes(BasisSet_t basis)
                 most[type][k] = std::max(most[type][k], kept);
                 prims[type] += kept;
             }
-            record[type] = 16.0 * KetView::rec(nnz) + 8.0 * ((KetView::full(type) ? full : 0) + 1);
+            record[type] = 16.0 * KetView::rec(nnz) + 8.0 * ((KetView::full(type) && has_d ? full : 0) + 1);
             // per primitive pair: (p, P), its Schwarz bound, full and compact E
             pairs += np * (40.0 + 8.0 * (full + nnz)) + 96.0;
             low += 4.0 * np * nnz;  // the FP32 tiles' coefficients

@@ -541,7 +541,7 @@ int GtfSystem::pack_kets()
         k[t].n = nsig[t];
         k[t].sig = d_sig[t];
         k[t].nnz = herm_nnz_lookup(la[t], lb[t]);
-        k[t].nfull = KetView::full(t) ? nsph(la[t]) * nsph(lb[t]) * nherm(la[t] + lb[t]) : 0;
+        k[t].nfull = KetView::full(t) && nsig[5] > 0 ? nsph(la[t]) * nsph(lb[t]) * nherm(la[t] + lb[t]) : 0;
     }
     // records, bounds, full coefficients, then info and the int arrays; every
     // part is a multiple of 16 bytes or comes last

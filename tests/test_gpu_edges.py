@@ -171,6 +171,26 @@ def test_batch_memory_shares_ket_blocks(g, tmp_path):
     assert used < used1 + nmol * (pairs + 32768)
 
 
+# without d functions nothing reads the full coefficients of the kets: the
+# primitive pairs, a record each, and a tenth for padded blocks (300 kets in 320
+# places), lists, tiles
+@gpu
+def test_memory_without_d_functions(g, tmp_path):
+    nprim, natoms = (4, 4, 1), 24
+    gbs = _basis(tmp_path / "b.gbs", nprim)
+    with open(gbs) as fh:
+        text = fh.read()
+    with open(gbs, "w") as fh:
+        fh.write(text[:text.index("D   1")] + "****\n")
+    pf = g.PFock(g.BasisSet(gbs, _hydrogens(tmp_path / "m.xyz", natoms)))
+    used = pf.stats()["device_bytes"]
+    pf.close()
+    pairs = sum(n * (40 + 8 * (FULL[t] + NONZERO[t]) + 8 + 16 * (2 + (NONZERO[t] + 1) // 2))
+                for t, n in _prim_pairs(nprim, natoms).items() if "d" not in t)
+    print("device memory %.1f MB, primitive pairs %.1f MB" % (used / 1e6, pairs / 1e6))
+    assert used < 1.1 * pairs + 0.3e6  # Boys tables
+
+
 # the FP32 tiles add a rounded copy of the nonzero coefficients, and lists of a
 # quarter of it at most (a run of 64 kets has 20 bytes)
 @gpu
