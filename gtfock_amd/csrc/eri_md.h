@@ -374,8 +374,11 @@ __device__ __forceinline__ void ket_loop(const KetRef& k, int j0, int js, Body&&
 // primitive.  A0 >= 0: the compact E of the whole pair, its structural zeros
 // skipped at compile time; A0 < 0: one component (NC = 1) whose rows b.E
 // points at in the full layout.  The bra contraction is summed over the bra
-// primitives before the ket coefficients are applied, except for a d-d bra
-// (one primitive pair in practice), where it would only hold registers.
+// primitives before the ket coefficients are applied: of (dd|dd) they are 200 KB
+// a wavefront, from L2, and applied within the loop over the bra primitives they
+// took C54H18's class 7.6 ms, now 4.1, and 24 d shells of four primitives 67 ms,
+// now 14.  Not for (dd|ss), where one coefficient a component is applied and the
+// sum only holds registers (2.9 ms instead of 2.2).
 template <int LA, int LB, int LC, int LD, int A0, int NC, typename Real, bool BLDS, typename Coef>
 __device__ __forceinline__ void eri_lane(const BraRef<Coef>& b, const KetRef& k, int j0, int js,
                                          const double* __restrict__ boys_slab,
@@ -386,7 +389,7 @@ __device__ __forceinline__ void eri_lane(const BraRef<Coef>& b, const KetRef& k,
     using TC = NzTab<LC, LD>;
     constexpr int L = S::L, HAB = S::HAB, HCD = S::HCD, NCD = S::NCD, NZC = TC::data.nnz;
     constexpr int ESTRIDE = A0 >= 0 ? TA::data.nnz : S::ESZ_AB;
-    constexpr bool SUM_BRA = LA + LB < 4;
+    constexpr bool SUM_BRA = LA + LB < 4 || LC + LD > 0;
     constexpr bool PSCREEN = prim_screened<LA, LB, LC, LD>();
     // small ket blocks are loaded ahead of the bra loop
     constexpr bool EARLY = NZC <= 6;
@@ -421,11 +424,6 @@ __device__ __forceinline__ void eri_lane(const BraRef<Coef>& b, const KetRef& k,
         bra_loop<L, PSCREEN, Real, BLDS>(b, k0, k1, qj, on, boys_slab, [&](int i, const Real (&R)[S::HL]) GTF_INLINE {
             // component by component: a row of E is in SGPRs once and used for
             // every h2
-            if constexpr (!SUM_BRA && !EARLY) {
-                // opaque, or the ket's coefficients (350 for d-d) would all be
-                // loaded ahead of the bra loop
-                asm volatile("" : "+v"(rec));
-            }
             static_for<0, NC>([&](auto c_) GTF_INLINE {
                 constexpr int c = decltype(c_)::value;
                 const_as<Coef>* E = b.E + (long)i * ESTRIDE;
