@@ -903,6 +903,7 @@ void GtfSystem::cut_class_tiles(int cls, TileList& hv, TileList& lv)
     // component chunks of the kernel that runs the class, and the most kets of
     // a run
     const int ns = exchanged(cls) ? ci->nsplit_t : ci->nsplit_tile;
+    const int cl = exchanged(cls) ? 0 : ci->comp_lanes;
     const int kmax = std::min(GTF_RUN_MAX_KETS, std::max(1, sh.units / ns));
     ntiles[cls] = ntiles_lo[cls] = 0;
     nq_lo[cls] = 0;
@@ -929,14 +930,15 @@ void GtfSystem::cut_class_tiles(int cls, TileList& hv, TileList& lv)
     const double unit_fixed = 12.0;
     auto chunking = [&](int nb, int nkmax, long kets) {
         Chunking c{0, 0, 0.0};
-        if (kets <= GTF_KET_BLOCK / 2) c.ljc = std::min(log2_floor(GTF_KET_BLOCK / kets), log2_floor(nkmax));
+        if (kets << cl <= GTF_KET_BLOCK / 2)
+            c.ljc = std::min(log2_floor(GTF_KET_BLOCK / (kets << cl)), log2_floor(nkmax));
         const long upq = std::max(1L, (long)nb * nkmax >> c.ljc);
         c.lic = std::min({log2_floor(std::max(1, nkmax >> c.ljc)), log2_floor((upq + sh.unit_pq - 1) / sh.unit_pq),
                           GTF_MAX_LIC});
         c.unit = GTF_KET_BLOCK * ((double)upq / (1L << c.lic) + unit_fixed);
         return c;
     };
-    auto blocks = [](long kets, int ljc) { return ((kets << ljc) + GTF_KET_BLOCK - 1) / GTF_KET_BLOCK; };
+    auto blocks = [&](long kets, int ljc) { return ((kets << (ljc + cl)) + GTF_KET_BLOCK - 1) / GTF_KET_BLOCK; };
     // the part of each row in FP64 and in FP32 runs
     struct Part {
         int r, nb, nkmax;

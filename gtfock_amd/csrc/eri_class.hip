@@ -35,7 +35,8 @@ void GTF_NAME(GTF_CLASS, GTF_PART)(EriClassInfo& e)
     e.nints = S::NAB * S::NCD;
     e.tile_threads = tile_threads<LA, LB, LC, LD>();
     e.nc_tile = NT;
-    e.nsplit_tile = (S::NAB + NT - 1) / NT;
+    e.comp_lanes = tile_static(S::NAB, NT) ? 0 : comp_lanes<LA, LB, LC, LD>();
+    e.nsplit_tile = (S::NAB + (NT << e.comp_lanes) - 1) / (NT << e.comp_lanes);
     e.full_E = !tile_static(S::NAB, NT);
     e.nc_t = EXCHANGED ? NCT : 0;
     e.nsplit_t = EXCHANGED ? (S::NCD + NCT - 1) / NCT : 0;

@@ -330,7 +330,7 @@ __global__ __launch_bounds__(256) void eri_kernel(EriArgs a)
 // The tile's work is cut into wavefront units: 64 lanes over (ket, ket
 // primitive class), one chunk of the ket primitives, one chunk of the split
 // side's components.  The bra pair and the component chunk are the same for
-// all lanes of a unit; the kets are consecutive in their list.  2^lic chunks
+// all lanes of a unit (but see comp_lanes); the kets are consecutive in their list.  2^lic chunks
 // of the ket primitives (primitives ic, ic + 2^lic, ...: the primitives are
 // ordered by their bound, so an interleaved chunk holds its share of the ones
 // that screening drops) keep a unit near unit_pq primitive quartets per lane;
@@ -415,6 +415,8 @@ struct DigestCtx {
     long nk;
     double* jpq;            // LDS: the ket's J_PQ, a component every 64; null: in jk
     double* jk;             // the list's J_PQ, a component every nk
+    int clane;              // comp_lanes: distance of a ket's lanes
+    bool lead;              // and the first of them
 };
 
 // update_F digestion (pfock/fock_task.c:29-117) of bra components A0 .. A0 +
@@ -424,7 +426,7 @@ struct DigestCtx {
 // same element of the strip are summed over the thread's components first.
 // crt: the run-time component of a kernel that has one bra component (A0 < 0)
 // or one ket component (C0 < 0) per thread.
-template <int LA, int LB, int LC, int LD, int A0, int NAr, int C0, int NCr, bool JREG, typename Get>
+template <int LA, int LB, int LC, int LD, int A0, int NAr, int C0, int NCr, bool JREG, int CL, typename Get>
 __device__ __forceinline__ void digest_unit(const DigestCtx& x, int crt, Get&& get, double* jreg)
 {
     using S = EriShape<LA, LB, LC, LD>;
@@ -464,8 +466,14 @@ __device__ __forceinline__ void digest_unit(const DigestCtx& x, int crt, Get&& g
             double s = 0.0;
             static_for<0, NAr>([&](auto c_) GTF_INLINE { s += dmn[decltype(c_)::value] * get(c_, d_); });
             const int cd = (KRT ? crt : CD0) + decltype(d_)::value;
-            if (x.jpq) x.jpq[cd * 64] += cJ2 * s;
-            else GTF_ATOMIC_ADD(&x.jk[cd * x.nk], cJ2 * s);
+            if (x.jpq) {
+                x.jpq[cd * 64] += cJ2 * s;
+                return;
+            }
+            // the lanes of a ket are all here (those without a component with zeros)
+            for (int m = 0; m < CL; m++) s += __shfl_xor(s, x.clane << m, 64);
+            if (CL > 0 && !x.lead) return;
+            GTF_ATOMIC_ADD(&x.jk[cd * x.nk], cJ2 * s);
         });
     }
     // K_MP -= cMP sum_nq D_nq I,  K_MQ -= cMQ sum_np D_np I  for each m, and
@@ -557,10 +565,7 @@ __host__ __device__ constexpr int tile_min_waves()
 // J_PQ buffers of `bufs` wavefronts.  Without buffers (0) the wavefronts add
 // J_PQ straight to the accumulators: for several densities, where the buffers
 // would not fit for the d classes, and for one density of a molecule whose
-// strips leave no room for them -- (dd|dd) from 1368 functions on.  There the
-// class takes 23.4 ms of C96H24's build (1464 functions) without the buffers,
-// 46.8 ms with global atomics for all of J and K (eri_kernel); buffers for
-// three of its four wavefronts, which would fit, gave 23.0 ms.
+// strips leave no room for them -- (dd|dd) from 1368 functions on.
 __host__ __device__ constexpr int tile_work(int rows, int nbf, int nab, int ncd, int bufs)
 {
     return rows * nbf + GTF_JMN_COPIES * nab + bufs * ncd * 64;
@@ -582,6 +587,7 @@ __device__ __forceinline__ void tile_kernel_body(const EriArgs& a)
     // compile-time component chunks, or (one component of very many) run-time
     constexpr bool STATIC = tile_static(SIDE, NC);
     constexpr bool JREG_ABLE = NSPLIT == 1 && NAB <= 3;
+    constexpr int CL = !STATIC && !EX ? comp_lanes<LA, LB, LC, LD>() : 0;
     extern __shared__ __attribute__((aligned(16))) double smem[];
     __shared__ int s_task, s_unit;
     const int NT = blockDim.x;
@@ -603,6 +609,7 @@ __device__ __forceinline__ void tile_kernel_body(const EriArgs& a)
     using Coef = std::conditional_t<LOW && (STATIC || EX), float, double>;
     BraRef<Coef> br;
     br.peps = a.pv.peps;
+    const Coef* lane_E = nullptr;
     // reads tile `task` (and its density rows); false when there is none
     auto open_tile = [&](int task) GTF_INLINE {
         if (task >= a.ntiles) return false;
@@ -625,6 +632,7 @@ __device__ __forceinline__ void tile_kernel_body(const EriArgs& a)
         br.q = as_const(a.pv.q + h.prim);
         if constexpr (std::is_same_v<Coef, float>) br.E = as_const(a.pv.Ezf) + h.E;
         else br.E = as_const(STATIC || EX ? a.pv.Ez : a.pv.E) + h.E;
+        if constexpr (CL > 0) lane_E = a.pv.E + h.E;
         if constexpr (BLDS)
             for (int d = 0; d < a.nd; d++) {
                 const double* D = a.D + d * a.dstride + mat;
@@ -676,7 +684,7 @@ __device__ __forceinline__ void tile_kernel_body(const EriArgs& a)
                 nkt = GTF_RUN_KETS(span), sp0 = GTF_RUN_SP0(span), spn = GTF_RUN_SPN(span);
                 lic = GTF_RUN_LIC(chunks), ljc = GTF_RUN_LJC(chunks);
                 ic0 = GTF_RUN_IC0(chunks), icn = GTF_RUN_ICN(chunks);
-                left = (((nkt << ljc) + 63) >> 6) - 1;
+                left = (((nkt << (ljc + CL)) + 63) >> 6) - 1;
                 blk = 0;
             }
             left -= d;
@@ -686,7 +694,7 @@ __device__ __forceinline__ void tile_kernel_body(const EriArgs& a)
         for (int unit = take(); seek(unit);) {
             unit = take();
             const int u = blk * 64 + lane;
-            const int q = u >> ljc, jc = u & ((1 << ljc) - 1);
+            const int q = u >> (ljc + CL), cl = (u >> ljc) & ((1 << CL) - 1), jc = u & ((1 << ljc) - 1);
             const int j = kbeg + q;
             bool on = q < nkt;
             if (on) {
@@ -745,15 +753,17 @@ __device__ __forceinline__ void tile_kernel_body(const EriArgs& a)
                     x.dk = a.dk + d * NCD * a.nket + oj;
                     x.nk = a.nket;
                     x.jpq = buffered ? jpq + lane : nullptr;
+                    x.clane = CL > 0 ? 1 << ljc : 0;
+                    x.lead = cl == 0;
                     x.jk = a.jk + d * NCD * a.nket + oj;
                     auto get = [&](auto c_, auto d_) GTF_INLINE { return (double)cell(c_, d_); };
                     if constexpr (JREG_ABLE) {
                         if (jreg_on) {
-                            digest_unit<LA, LB, LC, LD, A0, NAr, C0, NCr, true>(x, crt, get, jreg);
+                            digest_unit<LA, LB, LC, LD, A0, NAr, C0, NCr, true, CL>(x, crt, get, jreg);
                             continue;
                         }
                     }
-                    digest_unit<LA, LB, LC, LD, A0, NAr, C0, NCr, false>(x, crt, get, nullptr);
+                    digest_unit<LA, LB, LC, LD, A0, NAr, C0, NCr, false, CL>(x, crt, get, nullptr);
                 }
             };
             for (int sp = sp0; sp < sp0 + spn; sp++)
@@ -765,6 +775,16 @@ __device__ __forceinline__ void tile_kernel_body(const EriArgs& a)
                         eri_lane_t<LA, LB, LC, LD, -1, 1, Real, BLDS>(br, kr, j0, js, kf, boys, acc);
                         finish(std::integral_constant<int, 0>{}, std::integral_constant<int, NAB>{},
                                std::integral_constant<int, -1>{}, std::integral_constant<int, 1>{}, acc, sp);
+                    } else if constexpr (CL > 0) {
+                        const int comp = (sp << CL) + cl;
+                        BraRef<Coef> b1 = br;
+                        b1.lane_E = lane_E + min(comp, NAB - 1) * S::HAB;
+                        KetRef k1 = kr;
+                        if (comp >= NAB) k1.n = 0;  // a lane without a component: zeros
+                        Real acc[1][NCD];
+                        eri_lane<LA, LB, LC, LD, -1, 1, Real, BLDS, true>(b1, k1, j0, js, boys, acc);
+                        finish(std::integral_constant<int, -1>{}, std::integral_constant<int, 1>{},
+                               std::integral_constant<int, 0>{}, std::integral_constant<int, NCD>{}, acc, min(comp, NAB - 1));
                     } else if constexpr (!STATIC) {
                         BraRef<Coef> b1 = br;
                         b1.E += sp * S::HAB;
@@ -791,7 +811,17 @@ __device__ __forceinline__ void tile_kernel_body(const EriArgs& a)
                     }
                 }
             // the block's J_PQ
-            if (buffered && on && jc == 0)
+            if constexpr (CL > 0) {
+                // summed over the lanes of a ket
+                if (buffered)
+                    for (int cd = 0; cd < NCD; cd++) {
+                        double* p = jpq + cd * 64 + lane;
+                        double v = *p;
+                        if (v != 0.0) *p = 0.0;
+                        for (int s = 0; s < CL; s++) v += __shfl_xor(v, 1 << (ljc + s), 64);
+                        if (on && (jc | cl) == 0 && v != 0.0) GTF_ATOMIC_ADD(&a.jk[cd * a.nket + j], v);
+                    }
+            } else if (buffered && on && jc == 0)
                 for (int cd = 0; cd < NCD; cd++) {
                     double* p = jpq + cd * 64 + lane;
                     const double v = *p;
@@ -861,7 +891,8 @@ struct EriClassInfo {
     int nsplit;     // and threads per quartet
     int tile_threads;  // largest workgroup of the tile kernels
     int nc_tile;       // bra components per thread of the tile kernels
-    int nsplit_tile;
+    int nsplit_tile;   // chunks of the bra components
+    int comp_lanes;    // log2 of the lanes that share a ket, a component each, in the standard tile kernels
     bool full_E;       // the standard tile kernel reads the full coefficients
     int nints;      // integrals per quartet
     eri_kernel_t jk, diag, store;

@@ -119,6 +119,20 @@ __host__ __device__ constexpr int tile_nct()
 // a chunk known at compile time (see tile_chunk)
 __host__ __device__ constexpr bool tile_static(int total, int nc) { return (total + nc - 1) / nc <= TILE_STATIC_SPLITS; }
 
+// log2 of the lanes of a wavefront that hold one ket, each with another bra
+// component, in the standard tile kernels of run-time components.  (dd|dd) is
+// bound by the ket coefficients, 200 KB from L2 for every component of 64 kets;
+// with four components of 16 kets a load serves four lanes.  The bra's
+// coefficients are then the lane's own, vector loads of four lines, and the
+// seventh group of 25 components has three lanes without one.  C54H18's class
+// 4.1 -> 3.2 ms, 60 d shells 2.8 -> 2.35 ms; C96H24's, which has no J_PQ buffers,
+// 13.7 -> 14.4 ms.
+template <int LA, int LB, int LC, int LD>
+__host__ __device__ constexpr int comp_lanes()
+{
+    return LA + LB + LC + LD >= 8 ? 2 : 0;
+}
+
 // classes whose kernels apply the primitive screening of eri_block (by
 // total angular momentum L)
 __host__ __device__ constexpr bool prim_screened_l(int L) { return L <= 3; }
@@ -274,6 +288,7 @@ struct BraRef {
     const_as<Coef>* E;       // compact, or full from component c0 (the chunk's rows)
     int n;                   // primitive pairs
     double peps;
+    const Coef* lane_E;      // full, from this lane's component (comp_lanes)
 };
 
 // the ket of a lane: its first record (see KetView), its primitive pairs
@@ -379,7 +394,7 @@ __device__ __forceinline__ void ket_loop(const KetRef& k, int j0, int js, Body&&
 // took C54H18's class 7.6 ms, now 4.1, and 24 d shells of four primitives 67 ms,
 // now 14.  Not for (dd|ss), where one coefficient a component is applied and the
 // sum only holds registers (2.9 ms instead of 2.2).
-template <int LA, int LB, int LC, int LD, int A0, int NC, typename Real, bool BLDS, typename Coef>
+template <int LA, int LB, int LC, int LD, int A0, int NC, typename Real, bool BLDS, bool LANE_E = false, typename Coef>
 __device__ __forceinline__ void eri_lane(const BraRef<Coef>& b, const KetRef& k, int j0, int js,
                                          const double* __restrict__ boys_slab,
                                          Real (&acc)[NC][EriShape<LA, LB, LC, LD>::NCD])
@@ -422,6 +437,18 @@ __device__ __forceinline__ void eri_lane(const BraRef<Coef>& b, const KetRef& k,
             });
         };
         bra_loop<L, PSCREEN, Real, BLDS>(b, k0, k1, qj, on, boys_slab, [&](int i, const Real (&R)[S::HL]) GTF_INLINE {
+            if constexpr (LANE_E) {
+                const Coef* E = b.lane_E + (long)i * ESTRIDE;
+                static_for<0, HAB>([&](auto h1_) GTF_INLINE {
+                    constexpr int h1 = decltype(h1_)::value;
+                    const Real e = Real(E[h1]);
+                    static_for<0, HCD>([&](auto h2_) GTF_INLINE {
+                        constexpr int h2 = decltype(h2_)::value;
+                        W[0][h2] += e * R[hsum<h1, h2>()];
+                    });
+                });
+                return;
+            }
             // component by component: a row of E is in SGPRs once and used for
             // every h2
             static_for<0, NC>([&](auto c_) GTF_INLINE {

@@ -595,7 +595,7 @@ int gtf_pfock_class_info(PFock_t pf, int cls, int* info)
     info[2] = ci->lc;
     info[3] = ci->ld;
     info[4] = pf->sys.ntiles[cls] > 0 ? ci->nc_tile : ci->nc;
-    info[5] = pf->sys.ntiles[cls] > 0 ? ci->nsplit_tile : ci->nsplit;
+    info[5] = pf->sys.ntiles[cls] > 0 ? ci->nsplit_tile << ci->comp_lanes : ci->nsplit;
     info[6] = pf->sys.ntiles[cls];
     info[7] = pf->sys.ntiles_lo[cls];
     // the exchanged tile kernel runs the class: ket components per thread

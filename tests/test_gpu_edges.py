@@ -100,6 +100,29 @@ def test_fock_edges(g, sto3g, tmp_path, nprim, natoms):
     assert max(err, err2) < FOCK_TOL
 
 
+# (dd|dd) holds four components of 16 kets in a wavefront: 1 ket with its 16
+# primitive pairs over the lanes, 15, 21 and 36 kets; one density and two
+@gpu
+@pytest.mark.parametrize("nprim,natoms", [((1, 1, 4), 1), ((1, 1, 2), 5), ((1, 1, 1), 6), ((1, 1, 2), 8)])
+def test_fock_dd_lanes(g, tmp_path, nprim, natoms):
+    gbs, xyz = _basis(tmp_path / "b.gbs", nprim), _hydrogens(tmp_path / "m.xyz", natoms)
+    b, ob = g.BasisSet(gbs, xyz), oracle.Basis(gbs, xyz)
+    rng = np.random.default_rng(79)
+    Ds = [0.1 * (a + a.T) for a in rng.normal(size=(2, b.nbf, b.nbf))]
+    refs = [sum(ob.fock(D)[:2]) for D in Ds]
+    pf = g.PFock(b, max_numdmat=2)
+    err = np.abs(pf.fock(Ds[0]) - refs[0]).max()
+    pf.set_num_den_mat(2)
+    for k, D in enumerate(Ds):
+        pf.put_den_mat(D, index=k)
+    pf.commit()
+    pf.compute_fock()
+    err2 = max(np.abs(pf.get_mat(g.MAT_F, index=k) - refs[k]).max() for k in range(2))
+    pf.close()
+    print("fock dd %s %d: %.2e, two densities %.2e" % (nprim, natoms, err, err2))
+    assert max(err, err2) < FOCK_TOL
+
+
 # 1380 functions: the strips of (dd|dd) leave no room for the wavefronts' J_PQ
 # buffers in LDS (above 1367), and the class keeps its tiles without them; its
 # Schwarz values are 0.67 and 0.15, so a threshold of 0.2 sends a part to FP32
