@@ -892,7 +892,7 @@ int GtfSystem::upload_tiles(const TileList* hv, const TileList* lv, int c0, int 
 // A row holds the kets of one primitive-count bucket, often fewer than a
 // hundred, so a tile takes the runs of all of its bra's rows until it has
 // about tile_pq primitive quartets; a row beyond that is cut at multiples of
-// 64 kets, then by bra-primitive chunks, then by component chunks.
+// 64 kets, then by ket-primitive chunks, then by component chunks.
 void GtfSystem::cut_class_tiles(int cls, TileList& hv, TileList& lv)
 {
     const double tau2 = class_tau2(cls);

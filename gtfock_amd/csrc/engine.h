@@ -150,10 +150,11 @@ struct GtfSystem {
     size_t max_lds = 65536;
     bool use_tiles = true;
     // Tile shape of each class (the autotuner's search space): at most
-    // `units` work units and about `tile_pq` primitive quartets per tile,
-    // about `unit_pq` primitive quartets per unit (how finely a quartet's bra
-    // primitives are chunked), `grid` persistent workgroups per launch, each
-    // taking tiles from the class counter until none are left,
+    // `units` work units in a run of kets and about `tile_pq` primitive
+    // quartets per tile, about `unit_pq` primitive quartets per lane of a unit
+    // (how finely a quartet's ket primitives are chunked), at most `grid`
+    // persistent workgroups per launch, each taking tiles from the class
+    // counter until none are left,
     // `boys_lds` whether the workgroups of FP64 tiles and one density stage
     // the Boys slab and the bra shells' density rows in LDS (where they fit), and
     // `fp32` whether the class evaluates its quartets below the Schwarz

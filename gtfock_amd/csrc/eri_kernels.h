@@ -543,7 +543,7 @@ __device__ __forceinline__ void digest_unit(const DigestCtx& x, int crt, Get&& g
 }
 
 // Largest workgroup of a class's tile kernel (the host takes it or 256, see
-// GtfSystem::tile_threads).  A kernel compiled for 512 threads has at most 256
+// GtfSystem::tile_launch).  A kernel compiled for 512 threads has at most 256
 // VGPRs; the classes of L >= 5 need more, run one wavefront per SIMD and take
 // 256 threads.
 template <int LA, int LB, int LC, int LD>

